@@ -10,12 +10,12 @@
 // tile solve with GEMM updates by -1, folding alpha into the first step.  The
 // same sweep is kept, but each diagonal solve is a GEMM with the explicit
 // inverse of the diagonal block (all inverses computed up front by a
-// recursive TRTRI whose leaves are 64 x 64 single-wave kernels), so every
+// recursive TRTRI with leaves of order 128), so every
 // step runs on MFMA instead of a latency-bound substitution.
 //
 // POTRF (reference blas/zpotrf.c:89-187, unbuilt there): right-looking
 // blocked Cholesky with block order nb.  Step k factors the diagonal block
-// (recursive: leaves of order 64, inverse built alongside), forms the panel
+// (recursive: leaves of order 128, inverse built alongside), forms the panel
 // as a GEMM with the inverse, and applies the rank-nb update to the trailing
 // triangle in one launch.  With lookahead the next diagonal block is updated
 // first and factored on a side stream while the bulk update runs.
@@ -64,6 +64,9 @@ static inline int half64(int n)
   return h >= n ? n - 64 : h;
 }
 
+// Order of the factorization and inverse leaves.
+constexpr int LEAF = 128;
+
 template <typename T>
 static void fill_zero(hipStream_t s, int m, int n, T* Y, long ldy)
 {
@@ -71,79 +74,110 @@ static void fill_zero(hipStream_t s, int m, int n, T* Y, long ldy)
   gemm<T>(s, NoTrans, NoTrans, m, n, 0, T(0), Y, ldy, Y, ldy, T(0), Y, ldy);
 }
 
+// Inverses of `cnt` triangular blocks of order n (block b at A + b sA,
+// leading dimension lda) into Tinv + b sInv: leaves of order LEAF, then pairs
+// of neighbouring blocks joined level by level, I21 = -I22 A21 I11 (Upper: I12
+// = -I11 A12 I22), each level's pairs one batched launch per product and the
+// products limited to where the inverses are not zero.  The other triangle of
+// the inverses must be zero.  leaves: the leaves' inverses are still to be
+// formed.
+template <typename T>
+static void inverse_levels(hipStream_t s, int uplo, int diag, int n, const T* A, long lda, long sA, T* Tinv,
+                           long ldinv, long sInv, int cnt, int wslot, bool leaves)
+{
+  if (cnt <= 0 || n <= 0) return;
+  // op(offset, batch, stride): `full` places of stride `step` in every block,
+  // batched over the blocks or over the places, whichever is more
+  auto each = [&](int full, int step, auto&& op) {
+    if (full <= 0) return;
+    if (cnt >= full)
+      for (int p = 0; p < full; ++p) op((long)p * step * (1 + lda), (long)p * step * (1 + ldinv), cnt, sA, sInv);
+    else
+      for (int b = 0; b < cnt; ++b) op(b * sA, b * sInv, full, (long)step * (1 + lda), (long)step * (1 + ldinv));
+  };
+  if (leaves) {
+    const int full = n / LEAF, last = n % LEAF;
+    each(full, LEAF, [&](long oa, long oi, int batch, long da, long di) {
+      trtri_leaf<T>(s, uplo, diag, LEAF, A + oa, lda, da, Tinv + oi, ldinv, di, batch);
+    });
+    if (last)
+      trtri_leaf<T>(s, uplo, diag, last, A + (long)full * LEAF * (1 + lda), lda, sA,
+                    Tinv + (long)full * LEAF * (1 + ldinv), ldinv, sInv, cnt);
+  }
+  for (int h = LEAF; h < n; h *= 2) {
+    const int full = n / (2 * h), rem = n % (2 * h);
+    auto join = [&](int n2, long oa, long oi, int batch, long da, long di) {
+      const T* Ab = A + oa;
+      T* Ib = Tinv + oi;
+      T* I22 = Ib + (long)h * (1 + ldinv);
+      const long sW = (long)h * n2;
+      T* W = (T*)scratch(wslot, sizeof(T) * (size_t)sW * batch);
+      if (uplo == Lower) {
+        gemm<T>(s, NoTrans, NoTrans, n2, h, h, T(1), Ab + h, lda, Ib, ldinv, T(0), W, n2, TRI_FULL, batch, da, di, sW,
+                KRANGE_B_LOWER);
+        gemm<T>(s, NoTrans, NoTrans, n2, h, n2, T(-1), I22, ldinv, W, n2, T(0), Ib + h, ldinv, TRI_FULL, batch, di, sW,
+                di, KRANGE_A_LOWER);
+      } else {
+        gemm<T>(s, NoTrans, NoTrans, h, n2, n2, T(1), Ab + (long)h * lda, lda, I22, ldinv, T(0), W, h, TRI_FULL, batch,
+                da, di, sW, KRANGE_B_UPPER);
+        gemm<T>(s, NoTrans, NoTrans, h, n2, h, T(-1), Ib, ldinv, W, h, T(0), Ib + (long)h * ldinv, ldinv, TRI_FULL,
+                batch, di, sW, di, KRANGE_A_UPPER);
+      }
+    };
+    each(full, 2 * h, [&](long oa, long oi, int batch, long da, long di) { join(h, oa, oi, batch, da, di); });
+    if (rem > h) join(rem - h, (long)full * 2 * h * (1 + lda), (long)full * 2 * h * (1 + ldinv), cnt, sA, sInv);
+  }
+}
+
 template <typename T>
 void dev_trtri(const Exec& x, hipStream_t s, int uplo, int diag, int n, const T* A, long lda, T* Tinv, long ldinv,
                int wslot)
 {
-  if (n <= 64) {
-    trtri_leaf<T>(s, uplo, diag, n, A, lda, 0, Tinv, ldinv, 0, 1);
-    return;
-  }
-  const int n1 = half64(n), n2 = n - n1;
-  const T* A11 = A;
-  const T* A22 = A + n1 + (long)n1 * lda;
-  T* I11 = Tinv;
-  T* I22 = Tinv + n1 + (long)n1 * ldinv;
-  dev_trtri<T>(x, s, uplo, diag, n1, A11, lda, I11, ldinv, wslot);
-  dev_trtri<T>(x, s, uplo, diag, n2, A22, lda, I22, ldinv, wslot);
-  T* W = (T*)scratch(wslot, sizeof(T) * (size_t)n1 * n2);
-  if (uplo == Lower) {
-    // I21 = -I22 A21 I11
-    const T* A21 = A + n1;
-    T* I21 = Tinv + n1;
-    gemm<T>(s, NoTrans, NoTrans, n2, n1, n1, T(1), A21, lda, I11, ldinv, T(0), W, n2);
-    gemm<T>(s, NoTrans, NoTrans, n2, n1, n2, T(-1), I22, ldinv, W, n2, T(0), I21, ldinv);
-    fill_zero<T>(s, n1, n2, Tinv + (long)n1 * ldinv, ldinv);
-  } else {
-    // I12 = -I11 A12 I22
-    const T* A12 = A + (long)n1 * lda;
-    T* I12 = Tinv + (long)n1 * ldinv;
-    gemm<T>(s, NoTrans, NoTrans, n1, n2, n2, T(1), A12, lda, I22, ldinv, T(0), W, n1);
-    gemm<T>(s, NoTrans, NoTrans, n1, n2, n1, T(-1), I11, ldinv, W, n1, T(0), I12, ldinv);
-    fill_zero<T>(s, n2, n1, Tinv + n1, ldinv);
+  fill_zero<T>(s, n, n, Tinv, ldinv);
+  inverse_levels<T>(s, uplo, diag, n, A, lda, 0, Tinv, ldinv, 0, 1, wslot, true);
+}
+
+// Cholesky of the first nc columns of the trapezoid of nr rows at A (Lower;
+// Upper: the first nc rows of nr columns), right-looking in blocks of LEAF:
+// leaf (factor and inverse in one launch, the inverse of block j at Tinv + j
+// sInv), panel solve in place, one product on what is left of the nc columns.
+// Three launches per block, each over everything it touches: N = 8192, 512
+// columns 0.2-0.3 ms.  pair: see potrf_diag.
+template <typename T>
+static void potrf_columns(hipStream_t s, int uplo, int nr, int nc, T* A, long lda, T* Tinv, long ldinv, long sInv,
+                          int* info, int base, int pair)
+{
+  for (int j = 0; j < nc; j += LEAF) {
+    const int w = std::min(LEAF, nc - j), below = nr - j - w, right = nc - j - w;
+    T* D = A + (long)j * (1 + lda);
+    T* I = Tinv + (long)(j / LEAF) * sInv;
+    potrf_leaf<T>(s, uplo, w, D, lda, 0, I, ldinv, 0, 1, info, base + j, pair);
+    if (below <= 0) break;
+    if (uplo == Lower) {
+      trsm_panel<T>(s, uplo, below, w, D + w, lda, I, ldinv);
+      if (right > 0)
+        gemm<T>(s, NoTrans, Trans, below, right, w, T(-1), D + w, lda, D + w, lda, T(1), D + (long)w * (1 + lda), lda,
+                TRI_LOWER);
+    } else {
+      T* P = D + (long)w * lda;
+      trsm_panel<T>(s, uplo, below, w, P, lda, I, ldinv);
+      if (right > 0)
+        gemm<T>(s, Trans, NoTrans, right, below, w, T(-1), P, lda, P, lda, T(1), D + (long)w * (1 + lda), lda,
+                TRI_UPPER);
+    }
   }
 }
 
-// Recursive Cholesky of one diagonal block with its inverse (Tinv = inv(L)
-// for Lower, inv(U) for Upper).
+// Cholesky of one diagonal block with its inverse (Tinv = inv(L) for Lower,
+// inv(U) for Upper; its other triangle must be zero).
 // pair != 0: A is the real form of a complex block (orders 2i, 2i + 1 stand
 // for complex order i), and a failing pivot reports its complex order.
 template <typename T>
 static void potrf_diag(hipStream_t s, int uplo, int n, T* A, long lda, T* Tinv, long ldinv, int* info, int base,
-                       int wslot, bool zeroed = false, int pair = 0)
+                       int wslot, int pair = 0)
 {
-  if (n <= 64) {
-    potrf_leaf<T>(s, uplo, n, A, lda, 0, Tinv, ldinv, 0, 1, info, base, pair);
-    return;
-  }
-  const int n1 = half64(n), n2 = n - n1;
-  T* A11 = A;
-  T* A22 = A + n1 + (long)n1 * lda;
-  T* I11 = Tinv;
-  T* I22 = Tinv + n1 + (long)n1 * ldinv;
-  potrf_diag<T>(s, uplo, n1, A11, lda, I11, ldinv, info, base, wslot, zeroed, pair);
-  T* W = (T*)scratch(wslot, sizeof(T) * (size_t)n1 * n2);
-  if (uplo == Lower) {
-    T* A21 = A + n1;
-    T* I21 = Tinv + n1;
-    copy2d<T>(s, n2, n1, A21, lda, W, n2);
-    gemm<T>(s, NoTrans, Trans, n2, n1, n1, T(1), W, n2, I11, ldinv, T(0), A21, lda);   // L21 = A21 inv(L11)^T
-    gemm<T>(s, NoTrans, Trans, n2, n2, n1, T(-1), A21, lda, A21, lda, T(1), A22, lda, TRI_LOWER);
-    potrf_diag<T>(s, uplo, n2, A22, lda, I22, ldinv, info, base + n1, wslot, zeroed, pair);
-    gemm<T>(s, NoTrans, NoTrans, n2, n1, n1, T(1), A21, lda, I11, ldinv, T(0), W, n2);  // L21 inv(L11)
-    gemm<T>(s, NoTrans, NoTrans, n2, n1, n2, T(-1), I22, ldinv, W, n2, T(0), I21, ldinv);
-    if (!zeroed) fill_zero<T>(s, n1, n2, Tinv + (long)n1 * ldinv, ldinv);
-  } else {
-    T* A12 = A + (long)n1 * lda;
-    T* I12 = Tinv + (long)n1 * ldinv;
-    copy2d<T>(s, n1, n2, A12, lda, W, n1);
-    gemm<T>(s, Trans, NoTrans, n1, n2, n1, T(1), I11, ldinv, W, n1, T(0), A12, lda);     // U12 = inv(U11)^T A12
-    gemm<T>(s, Trans, NoTrans, n2, n2, n1, T(-1), A12, lda, A12, lda, T(1), A22, lda, TRI_UPPER);
-    potrf_diag<T>(s, uplo, n2, A22, lda, I22, ldinv, info, base + n1, wslot, zeroed, pair);
-    gemm<T>(s, NoTrans, NoTrans, n1, n2, n2, T(1), A12, lda, I22, ldinv, T(0), W, n1);   // U12 inv(U22)
-    gemm<T>(s, NoTrans, NoTrans, n1, n2, n1, T(-1), I11, ldinv, W, n1, T(0), I12, ldinv);
-    if (!zeroed) fill_zero<T>(s, n2, n1, Tinv + n1, ldinv);
-  }
+  potrf_columns<T>(s, uplo, n, n, A, lda, Tinv, ldinv, (long)LEAF * (1 + ldinv), info, base, pair);
+  inverse_levels<T>(s, uplo, NonUnit, n, A, lda, 0, Tinv, ldinv, 0, 1, wslot, false);
 }
 
 enum { WS_TRSM = 4, WS_TRSMW = 5, WS_SPLITK = 31 };
@@ -183,22 +217,66 @@ static bool gemm_splitk(hipStream_t s, int ta, int tb, int m, int n, int k, T al
   return true;
 }
 
-void potrf_scratch_caps(int n, int nb, size_t elt, size_t cap[4])
-{
-  nb = std::max(64, std::min(nb, std::max(n, 1)));
-  // the largest recursion node of a diagonal block of order <= nb is the top
-  // one: W holds its n1 x n2 block
-  const size_t h = nb > 64 ? (size_t)half64(nb) * (size_t)(nb - half64(nb)) : 0;
-  cap[WS_DIAG0] = cap[WS_DIAG1] = elt * std::max<size_t>(h, 1);
-  cap[WS_PANEL] = elt * std::max<size_t>((size_t)std::max(n - nb, 0) * nb, 1);
-  cap[WS_INV] = elt * 2 * (size_t)nb * nb;
-}
-
 // Trailing updates of POTRF: 1 (default) paired, 0 one per panel.
 // XKBLAS_POTRF_PAIR sets the initial value.
 static int g_potrf_pair = getenv("XKBLAS_POTRF_PAIR") ? (atoi(getenv("XKBLAS_POTRF_PAIR")) != 0) : 1;
 static int potrf_pairing() { return g_potrf_pair; }
 void potrf_set_pairing(int v) { g_potrf_pair = v < 0 ? 1 : (v ? 1 : 0); }
+
+// Width of the block columns of potrf_panels: one block column while the
+// trailing products are shorter than the chain anyway (order 517: 0.20 ms
+// against 0.27 with two streams, 1024: 0.38 against 0.45), then 512 (order
+// 2048 / 8192 / 16384: 0.94 / 7.04 / 35.2 ms; 256: 0.99 / 7.26 / 37.4;
+// 1024: 0.92 / 7.13 / 35.3; FP32 order 8192: 4.92, 5.05, 5.17 ms).
+static int panel_width(int n) { return n <= 1024 ? n : 512; }
+
+// Blocked Cholesky in the MFMA modes: block columns of panel_width(n) factored
+// over their whole height on the side stream (potrf_columns), beside the
+// trailing update of the block column before on the compute stream; the next
+// block column is updated first (lookahead).
+template <typename T>
+static void potrf_panels(const Exec& x, int uplo, int n, T* A, long lda, int* info, hipEvent_t ev_diag,
+                         hipEvent_t ev_look)
+{
+  const int nb = panel_width(n), nt = (n + nb - 1) / nb;
+  T* inv = (T*)scratch(WS_INV, sizeof(T) * (size_t)LEAF * LEAF);
+  const bool lookahead = x.s_diag != nullptr && nt > 1;
+  hipStream_t sd = lookahead ? x.s_diag : x.s;
+  auto blk = [&](int i, int j) { return A + (long)i * nb + (long)j * nb * lda; };
+  if (lookahead) {
+    XK_HIP(hipEventRecord(ev_look, x.s));
+    XK_HIP(hipStreamWaitEvent(sd, ev_look, 0));
+    gemm_set_priority_stream(sd);  // the chain's launches issue ahead of the trailing update's waves
+  }
+  potrf_columns<T>(sd, uplo, n, std::min(nb, n), A, lda, inv, LEAF, 0, info, 0, 0);
+  for (int k = 0; k < nt; ++k) {
+    if (lookahead) {
+      XK_HIP(hipEventRecord(ev_diag, sd));
+      XK_HIP(hipStreamWaitEvent(x.s, ev_diag, 0));
+    }
+    if (k == nt - 1) break;
+    const int rest = n - (k + 1) * nb, k1 = std::min(nb, rest), r2 = rest - k1;
+    if (uplo == Lower) {
+      const T* U = blk(k + 1, k);
+      gemm<T>(x.s, NoTrans, Trans, rest, k1, nb, T(-1), U, lda, U, lda, T(1), blk(k + 1, k + 1), lda, TRI_LOWER);
+      if (lookahead) XK_HIP(hipEventRecord(ev_look, x.s));
+      if (r2 > 0)
+        gemm<T>(x.s, NoTrans, Trans, r2, r2, nb, T(-1), U + k1, lda, U + k1, lda, T(1), blk(k + 2, k + 2), lda,
+                TRI_LOWER);
+    } else {
+      const T* U = blk(k, k + 1);
+      gemm<T>(x.s, Trans, NoTrans, k1, rest, nb, T(-1), U, lda, U, lda, T(1), blk(k + 1, k + 1), lda, TRI_UPPER);
+      if (lookahead) XK_HIP(hipEventRecord(ev_look, x.s));
+      if (r2 > 0) {
+        const T* U2 = U + (long)k1 * lda;
+        gemm<T>(x.s, Trans, NoTrans, r2, r2, nb, T(-1), U2, lda, U2, lda, T(1), blk(k + 2, k + 2), lda, TRI_UPPER);
+      }
+    }
+    if (lookahead) XK_HIP(hipStreamWaitEvent(sd, ev_look, 0));
+    potrf_columns<T>(sd, uplo, rest, k1, blk(k + 1, k + 1), lda, inv, LEAF, 0, info, (k + 1) * nb, 0);
+  }
+  if (lookahead) gemm_set_priority_stream(nullptr);
+}
 
 template <typename T>
 void dev_potrf(const Exec& x, int uplo, int n, T* A, long lda, int nb, int* info,
@@ -211,14 +289,22 @@ void dev_potrf(const Exec& x, int uplo, int n, T* A, long lda, int nb, int* info
   const int keep_nb = hooks ? hooks->keep_nb : 0;
   XK_CHECK(!keep_inv || (keep_nb > 0 && (nt == 1 || nb % keep_nb == 0)),
            "dev_potrf: kept inverses need a block order that divides nb");
-  // inverses of two consecutive diagonal blocks (ping-pong for lookahead)
-  T* inv = (T*)scratch(WS_INV, sizeof(T) * (size_t)2 * nb * nb);
   hipEvent_t ev_diag = x.ev0, ev_look = x.ev1;
   const bool own_events = !ev_diag || !ev_look;
   if (own_events) {
     XK_HIP(hipEventCreateWithFlags(&ev_diag, hipEventDisableTiming));
     XK_HIP(hipEventCreateWithFlags(&ev_look, hipEventDisableTiming));
   }
+  if (!split_enabled<T>(x) && !hooks) {
+    potrf_panels<T>(x, uplo, n, A, lda, info, ev_diag, ev_look);
+    if (own_events) {
+      XK_HIP(hipEventDestroy(ev_diag));
+      XK_HIP(hipEventDestroy(ev_look));
+    }
+    return;
+  }
+  // inverses of two consecutive diagonal blocks (ping-pong for lookahead)
+  T* inv = (T*)scratch(WS_INV, sizeof(T) * (size_t)2 * nb * nb);
   const bool lookahead = x.s_diag != nullptr && nt > 1;
   hipStream_t sd = lookahead ? x.s_diag : x.s;
   // trailing updates of two panels at once (inner dimension 2 nb): longer
@@ -266,7 +352,7 @@ void dev_potrf(const Exec& x, int uplo, int n, T* A, long lda, int nb, int* info
       copy2d<T>(sd, sz, sz, ik + (long)j * keep_nb * (1 + nb), nb, keep_inv + g * keep_nb * keep_nb, keep_nb);
     }
   };
-  potrf_diag<T>(sd, uplo, tsz(0), blk(0, 0), lda, inv, nb, info, 0, WS_DIAG0, true);
+  potrf_diag<T>(sd, uplo, tsz(0), blk(0, 0), lda, inv, nb, info, 0, WS_DIAG0);
   keep(0, inv);
   if (hooks && hooks->beside_first) hooks->beside_first();
   for (int k = 0; k < nt; ++k) {
@@ -364,11 +450,11 @@ void dev_potrf(const Exec& x, int uplo, int n, T* A, long lda, int nb, int* info
     if (lookahead) {
       XK_HIP(hipStreamWaitEvent(sd, ev_look, 0));
       potrf_diag<T>(sd, uplo, k1, blk(k + 1, k + 1), lda, inv + (size_t)((k + 1) & 1) * nb * nb, nb, info,
-                    (k + 1) * nb, ((k + 1) & 1) ? WS_DIAG1 : WS_DIAG0, true);
+                    (k + 1) * nb, ((k + 1) & 1) ? WS_DIAG1 : WS_DIAG0);
     }
     if (!lookahead)
       potrf_diag<T>(x.s, uplo, tsz(k + 1), blk(k + 1, k + 1), lda, inv + (size_t)((k + 1) & 1) * nb * nb, nb,
-                    info, (k + 1) * nb, WS_DIAG0, true);
+                    info, (k + 1) * nb, WS_DIAG0);
     keep(k + 1, inv + (size_t)((k + 1) & 1) * nb * nb);
   }
   if (hooks && hooks->after_panel) hooks->after_panel(nt - 1, inv + (size_t)((nt - 1) & 1) * nb * nb);
@@ -383,55 +469,18 @@ void dev_potrf(const Exec& x, int uplo, int n, T* A, long lda, int nb, int* info
 // Diagonal block order of the TRSM sweep for a triangle of order na.
 static inline int trsm_block(int nb, int na) { return std::max(64, std::min(nb, na)); }
 
-// dev_trtri over `cnt` triangular blocks of order n at once: block b is
-// A + b sA (leading dimension lda), its inverse Tinv + b sInv (ldinv).  Every
-// level of the recursion is one batched launch per step for all blocks.
-template <typename T>
-static void trtri_batched(hipStream_t s, int uplo, int diag, int n, const T* A, long lda, long sA, T* Tinv,
-                          long ldinv, long sInv, int cnt, int wslot)
-{
-  if (n <= 64) {
-    trtri_leaf<T>(s, uplo, diag, n, A, lda, sA, Tinv, ldinv, sInv, cnt);
-    return;
-  }
-  const int n1 = half64(n), n2 = n - n1;
-  trtri_batched<T>(s, uplo, diag, n1, A, lda, sA, Tinv, ldinv, sInv, cnt, wslot);
-  trtri_batched<T>(s, uplo, diag, n2, A + n1 + (long)n1 * lda, lda, sA, Tinv + n1 + (long)n1 * ldinv, ldinv, sInv,
-                   cnt, wslot);
-  const long sW = (long)n1 * n2;
-  T* W = (T*)scratch(wslot, sizeof(T) * (size_t)sW * cnt);
-  const T* I11 = Tinv;
-  const T* I22 = Tinv + n1 + (long)n1 * ldinv;
-  if (uplo == Lower) {
-    // I21 = -I22 A21 I11, strictly upper block zeroed
-    gemm<T>(s, NoTrans, NoTrans, n2, n1, n1, T(1), A + n1, lda, I11, ldinv, T(0), W, n2, TRI_FULL, cnt, sA, sInv, sW);
-    gemm<T>(s, NoTrans, NoTrans, n2, n1, n2, T(-1), I22, ldinv, W, n2, T(0), Tinv + n1, ldinv, TRI_FULL, cnt, sInv,
-            sW, sInv);
-    T* Z = Tinv + (long)n1 * ldinv;
-    gemm<T>(s, NoTrans, NoTrans, n1, n2, 0, T(0), Z, ldinv, Z, ldinv, T(0), Z, ldinv, TRI_FULL, cnt, 0, 0, sInv);
-  } else {
-    // I12 = -I11 A12 I22, strictly lower block zeroed
-    gemm<T>(s, NoTrans, NoTrans, n1, n2, n2, T(1), A + (long)n1 * lda, lda, I22, ldinv, T(0), W, n1, TRI_FULL, cnt,
-            sA, sInv, sW);
-    gemm<T>(s, NoTrans, NoTrans, n1, n2, n1, T(-1), I11, ldinv, W, n1, T(0), Tinv + (long)n1 * ldinv, ldinv,
-            TRI_FULL, cnt, sInv, sW, sInv);
-    T* Z = Tinv + n1;
-    gemm<T>(s, NoTrans, NoTrans, n2, n1, 0, T(0), Z, ldinv, Z, ldinv, T(0), Z, ldinv, TRI_FULL, cnt, 0, 0, sInv);
-  }
-}
-
 // Inverses of all nb x nb diagonal blocks of the triangular na x na matrix A,
-// stored one after another (nb x nb each) in inv: the full-order blocks in
-// one batched recursion, a shorter last block on its own.
+// stored one after another (nb x nb each) in inv: the full-order blocks
+// batched, a shorter last block on its own.
 template <typename T>
 static void trsm_inverses(const Exec& x, int uplo, int diag, int na, const T* A, long lda, int nb, T* inv)
 {
   const int full = na / nb, last = na - full * nb;
-  if (full > 0)
-    trtri_batched<T>(x.s, uplo, diag, nb, A, lda, (long)nb * (1 + lda), inv, nb, (long)nb * nb, full, WS_DIAG0);
+  fill_zero<T>(x.s, nb, (full + (last > 0)) * nb, inv, nb);
+  inverse_levels<T>(x.s, uplo, diag, nb, A, lda, (long)nb * (1 + lda), inv, nb, (long)nb * nb, full, WS_DIAG0, true);
   if (last > 0)
-    dev_trtri<T>(x, x.s, uplo, diag, last, A + (long)full * nb * (1 + lda), lda, inv + (size_t)full * nb * nb, nb,
-                 WS_DIAG0);
+    inverse_levels<T>(x.s, uplo, diag, last, A + (long)full * nb * (1 + lda), lda, 0, inv + (size_t)full * nb * nb, nb,
+                      0, 1, WS_DIAG0, true);
 }
 
 // The block sweep of dev_trsm with the diagonal-block inverses given.
@@ -924,7 +973,7 @@ static void cpotrf_diag(hipStream_t s, int uplo, int n, T* A, long lda, T* Tinv,
                         int* info, int base)
 {
   cplx_realform<T>(s, uplo, n, A, lda, R, ldr);
-  potrf_diag<T>(s, Lower, 2 * n, R, ldr, Rinv, ldr, info, 2 * base, WS_ZDW, true, 1);
+  potrf_diag<T>(s, Lower, 2 * n, R, ldr, Rinv, ldr, info, 2 * base, WS_ZDW, 1);
   cplx_fromreal<T>(s, uplo, n, R, ldr, A, lda, Rinv, Tinv, ldinv);
 }
 

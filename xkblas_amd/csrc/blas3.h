@@ -25,9 +25,8 @@ struct Exec {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;  // POTRF's stream-ordering events (created per call when null)
 };
 
-// Scratch slots of dev_potrf, and the bytes each needs for order n, block nb.
+// Scratch slots of dev_potrf.
 enum { WS_DIAG0 = 0, WS_DIAG1 = 1, WS_PANEL = 2, WS_INV = 3 };
-void potrf_scratch_caps(int n, int nb, size_t elt, size_t cap[4]);
 
 template <typename T>
 void dev_gemm(const Exec& x, int transA, int transB, int m, int n, int k, T alpha, const T* A, long lda,

@@ -1,32 +1,15 @@
 // factor.hip — latency-bound diagonal-block kernels for gfx950:
-// Cholesky + inverse of blocks of order <= 64, triangular inverse, and small
+// Cholesky + inverse of blocks of order <= 128, triangular inverse, and small
 // helpers (2-D copy, triangle zeroing, int fill).
 //
-// The padded rows/columns of a leaf beyond n are the identity, so every
-// block is handled as a 64 x 64 problem.  The Cholesky leaf (four waves)
-// writes the factor and its inverse in one launch; the triangular-inverse
-// leaf (one wave) holds the block in LDS (column stride 65) and solves one
-// column of inv(L) per lane.
+// The rows/columns of a leaf's last 16 x 16 tile beyond n are the identity.
+// The Cholesky leaf writes the factor and its inverse in one launch.
 #include "common.h"
 #include "kernels.h"
 #include <climits>
+#include <utility>
 
 namespace xk {
-
-constexpr int LEAF = 64;
-constexpr int LLD = LEAF + 1;  // padded LDS column stride
-
-__device__ __forceinline__ double bcast(double x, int src)
-{
-  int lo = __double2loint(x), hi = __double2hiint(x);
-  lo = __builtin_amdgcn_readlane(lo, src);
-  hi = __builtin_amdgcn_readlane(hi, src);
-  return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ float bcast(float x, int src)
-{
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), src));
-}
 
 // sq = sqrt(p) and rs = 1 / sq for a finite pivot p > 0, without a division
 // and without a branch: p = 2^(2h) p' with p' in [0.5, 2) (exact scaling by
@@ -57,44 +40,6 @@ __device__ __forceinline__ void sqrt_rcp(float p, float& sq, float& rs)
   rs = 1.0f / sq;
 }
 
-// Row `lane` of the lower-triangular view L of block A:
-//   uplo == Lower: L = tril(A); uplo == Upper: L = triu(A)^T.
-template <typename T>
-__device__ __forceinline__ T lower_view(const T* A, long lda, int uplo, int n, int i, int j)
-{
-  if (i >= n || j >= n) return (i == j) ? T(1) : T(0);
-  if (j > i) return T(0);
-  return uplo == Lower ? A[i + (long)j * lda] : A[j + (long)i * lda];
-}
-
-// inv(L) for the 64 x 64 lower-triangular L held in LDS (column-major,
-// stride LLD); lane j computes column j.  unit: diagonal taken as 1.
-template <typename T>
-__device__ __forceinline__ void lower_inverse_to(const T* Ls, int lane, bool unit, T* Tinv, long ldinv, int n,
-                                                 int uplo)
-{
-  T x[LEAF];
-#pragma unroll
-  for (int i = 0; i < LEAF; ++i) {
-    T s = (i == lane) ? T(1) : T(0);
-#pragma unroll
-    for (int k = 0; k < i; ++k) s -= Ls[i + k * LLD] * x[k];
-    x[i] = unit ? s : s / Ls[i + i * LLD];
-    if (i < lane) x[i] = T(0);
-  }
-  // column `lane` of inv(L): X[i][lane].  Lower: Tinv[i + lane*ld];
-  // Upper (inv(U) = inv(L)^T): Tinv[lane + i*ld].
-  if (lane < n) {
-#pragma unroll
-    for (int i = 0; i < LEAF; ++i) {
-      if (i < n) {
-        if (uplo == Lower) Tinv[i + (long)lane * ldinv] = x[i];
-        else Tinv[lane + (long)i * ldinv] = x[i];
-      }
-    }
-  }
-}
-
 // Workgroup barrier that orders LDS accesses only: global stores in flight
 // are not waited for (nothing in the kernel reads them back).
 __device__ __forceinline__ void lds_barrier()
@@ -104,244 +49,468 @@ __device__ __forceinline__ void lds_barrier()
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Cholesky factor and its inverse for one block of order <= 64, blocked by
-// 16 and spread over four waves.
-// LDS: the lower triangle packed by rows, P[i (i + 1) / 2 + k] = L(i, k),
-// and one 64 x 16 block column of the inverse: 24.4 KB in FP64.
-// A trailing-update GEMM that fills a CU (four 33 KB workgroups) leaves
-// 28 KB of LDS free, so a leaf launched beside it starts at once in that gap
-// instead of waiting for a CU to drain (a leaf holding the block and its
-// inverse unpacked, 72 KB, waited up to milliseconds).  About 125 VGPRs: it
-// also fits beside three update-GEMM waves (104-112 VGPRs each) on a SIMD.
-// For each 16-column block jb:
-//   wave 0 factors the 16 x 16 diagonal block in registers (lane i holds row
-//   i, cross-lane reads for the broadcasts), with the pivots' roots and
-//   reciprocals from one reciprocal-square-root iteration (no division on
-//   the chain), then inverts it (lane c solves column c), writes L to A and
-//   the inverse in its place in P;
-//   all threads solve the panel below, L21 = A21 inv(L11)^T, and update the
-//   trailing triangle, A22 -= L21 L21^T.
-// Then P holds L below the diagonal blocks and the diagonal blocks'
-// inverses, from which inv(L) follows by block columns.  The barriers order
-// LDS only (no wait for the global stores of L and inv(L)).  Rows/columns
-// beyond n are the identity.  info receives the first order whose pivot is
-// not positive.
-constexpr int LB = 16;  // inner block of the leaf
+// ---------------------------------------------------------------- tiles
+// The leaves keep a block of order 16 NT in LDS as 16 x 16 tiles (lower
+// triangle only, tile (i, k) at slot i (i + 1) / 2 + k), each 256 elements
+// ordered so that element 64 r + l is what lane l holds in register r of an
+// MFMA accumulator: row l % 16, column tile_col(l / 16, r).  The operands of
+// X Y^T (v_mfma_*_16x16x4, Y issued first) take the same registers, the inner
+// index running over the columns in the accumulator's order, so a product's
+// result is the next one's operand without moving, and every tile access is
+// 64 consecutive elements.
+constexpr int LEAF = 128;
+constexpr int TS = 256;  // elements of a tile
 
-__device__ __forceinline__ int pk(int i, int k) { return (i * (i + 1) >> 1) + k; }
+typedef double leaf_d4 __attribute__((ext_vector_type(4)));
+typedef float leaf_f4 __attribute__((ext_vector_type(4)));
+template <typename T> struct LeafV;
+template <> struct LeafV<double> { typedef leaf_d4 type; };
+template <> struct LeafV<float> { typedef leaf_f4 type; };
 
-template <typename T>
-__global__ __launch_bounds__(256) void potrf_leaf_kernel(int uplo, int n, T* A, long lda, long sA, T* Tinv,
-                                                         long ldinv, long sInv, int* info, int base, int pair)
+__device__ __forceinline__ leaf_d4 leaf_mfma(double a, double b, leaf_d4 c)
 {
-  __shared__ T P[LEAF * (LEAF + 1) / 2];
-  __shared__ T X[LEAF * LB];            // X[i * LB + c]: rows of one block column of inv(L)
-  __shared__ T Lr[LB];                  // reciprocals of the diagonal block's pivots
-  // the leaf is the latency-bound step of the diagonal chain and shares its
-  // CU with update GEMM waves: its waves issue first
-  __builtin_amdgcn_s_setprio(3);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  A += (long)blockIdx.x * sA;
-  Tinv += (long)blockIdx.x * sInv;
-  auto put = [&](int i, int k, T v) {  // factor entry (i, k), k <= i, to the stored triangle
-    if (i < n && k < n) {
-      if (uplo == Lower) A[i + (long)k * lda] = v;
-      else A[k + (long)i * lda] = v;
-    }
-  };
-  {
-    // all loads in flight before the first LDS store
-    T v[LEAF * LEAF / 256];
-#pragma unroll
-    for (int u = 0; u < LEAF * LEAF / 256; ++u) {
-      const int e = tid + 256 * u, i = e & 63, k = e >> 6;
-      v[u] = k <= i ? lower_view(A, lda, uplo, n, i, k) : T(0);
-    }
-#pragma unroll
-    for (int u = 0; u < LEAF * LEAF / 256; ++u) {
-      const int e = tid + 256 * u, i = e & 63, k = e >> 6;
-      if (k <= i) P[pk(i, k)] = v[u];
-    }
-  }
-  lds_barrier();
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ leaf_f4 leaf_mfma(float a, float b, leaf_f4 c)
+{
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
 
-  int fail = INT_MAX;  // first order with a non-positive pivot (wave 0)
-  for (int jb = 0; jb < LEAF / LB; ++jb) {
-    const int c0 = jb * LB;
-    if (wave == 0) {
-      const int i = lane & (LB - 1);
-      const bool own = lane < LB;
-      T d[LB];
-#pragma unroll
-      for (int k = 0; k < LB; ++k) d[k] = k <= i ? P[pk(c0 + i, c0 + k)] : T(0);
-      // right-looking: the pivot chain needs no cross-lane data beyond the
-      // pivot itself (lane j + 1 updates its own diagonal entry).  The chain
-      // has no branch (lane j keeps reciprocal j, stored after the loop), so
-      // the updates of one step are scheduled under the next pivot's root.
-      T myrs = T(0);
-#pragma unroll
-      for (int j = 0; j < LB; ++j) {
-        const T p = bcast(d[j], j);
-        fail = (!(p > T(0)) && fail == INT_MAX && c0 + j < n) ? c0 + j : fail;
-        T sq, rs;
-        sqrt_rcp(p, sq, rs);
-        myrs = lane == j ? rs : myrs;
-        d[j] = i > j ? d[j] * rs : (i == j ? sq : T(0));
-#pragma unroll
-        for (int k = j + 1; k < LB; ++k) d[k] = fma(-d[j], bcast(d[j], k), d[k]);
-      }
-      if (lane < LB) Lr[lane] = myrs;
-      if (own) {
-#pragma unroll
-        for (int k = 0; k < LB; ++k)
-          if (k <= i) put(c0 + i, c0 + k, d[k]);
-      }
-      // column i of inv(L11): y_r = (delta_ri - sum_{k<r} L(r, k) y_k) / L(r, r),
-      // L(r, k) read from lane r
-      T y[LB];
-#pragma unroll
-      for (int r = 0; r < LB; ++r) {
-        T acc = (r == i) ? T(1) : T(0);
-#pragma unroll
-        for (int k = 0; k < r; ++k) acc = fma(-bcast(d[k], r), y[k], acc);
-        y[r] = r < i ? T(0) : acc * Lr[r];
-      }
-#pragma unroll
-      for (int r = 0; r < LB; ++r) d[r] = y[r];
-      if (own) {
-#pragma unroll
-        for (int r = 0; r < LB; ++r)
-          if (r >= i) P[pk(c0 + r, c0 + i)] = d[r];
-      }
-    }
-    lds_barrier();
-    const int m = LEAF - c0 - LB;  // rows below the diagonal block
-    if (m > 0) {
-      // panel: L[c0+LB+r][c0+c] = sum_{t <= c} A[c0+LB+r][c0+t] inv(L11)[c][t]
-      T pv[3];
-#pragma unroll 1
-      for (int u = 0; u < 3; ++u) {
-        const int e = tid + 256 * u;
-        pv[u] = T(0);
-        if (e < m * LB) {
-          const int r = e % m, c = e / m;
-          const T* arow = P + pk(c0 + LB + r, c0);
-          const T* irow = P + pk(c0 + c, c0);
-          T a0 = T(0), a1 = T(0);
-#pragma unroll
-          for (int t = 0; t < LB; t += 2) {
-            a0 = fma(arow[t], t <= c ? irow[t] : T(0), a0);
-            a1 = fma(arow[t + 1], t + 1 <= c ? irow[t + 1] : T(0), a1);
-          }
-          pv[u] = a0 + a1;
-        }
-      }
-      lds_barrier();
-#pragma unroll
-      for (int u = 0; u < 3; ++u) {
-        const int e = tid + 256 * u;
-        if (e < m * LB) P[pk(c0 + LB + e % m, c0 + e / m)] = pv[u];
-      }
-      lds_barrier();
-      // trailing triangle: L[c0+LB+r][c0+LB+q] -= sum_t L21[r][t] L21[q][t],
-      // q <= r < m, element e = r (r + 1) / 2 + q of the triangle; each
-      // element is read and written by its own thread only
-      const int cnt = m * (m + 1) / 2;
-#pragma unroll 1
-      for (int u = 0; u < 5; ++u) {  // cnt <= 48 * 49 / 2 < 5 * 256
-        const int e = tid + 256 * u;
-        if (e < cnt) {
-          int r = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);
-          if ((r + 1) * (r + 2) / 2 <= e) ++r;
-          if (r * (r + 1) / 2 > e) --r;
-          const int q = e - r * (r + 1) / 2;
-          const T* rr = P + pk(c0 + LB + r, c0);
-          const T* rq = P + pk(c0 + LB + q, c0);
-          T a0 = P[pk(c0 + LB + r, c0 + LB + q)], a1 = T(0);
-#pragma unroll
-          for (int t = 0; t < LB; t += 2) {
-            a0 = fma(-rr[t], rq[t], a0);
-            a1 = fma(-rr[t + 1], rq[t + 1], a1);
-          }
-          P[pk(c0 + LB + r, c0 + LB + q)] = a0 + a1;
-        }
-      }
-      lds_barrier();
-    }
-  }
-  // pair: orders 2i, 2i + 1 stand for order i of a complex block
-  if (tid == 0 && fail != INT_MAX) atomicMin(info, pair ? (base + fail) / 2 + 1 : base + fail + 1);
-  // the factor below the diagonal blocks to the stored triangle
-  for (int e = tid; e < LEAF * LEAF; e += 256) {
-    const int i = e & 63, k = e >> 6;
-    if (k < (i & ~(LB - 1))) put(i, k, P[pk(i, k)]);
-  }
-  if (!Tinv) return;
-  auto out = [&](int i, int j, T v) {  // inv(L)(i, j) to Tinv (Upper: inv(U) = inv(L)^T)
-    if (i < n && j < n) {
-      if (uplo == Lower) Tinv[i + (long)j * ldinv] = v;
-      else Tinv[j + (long)i * ldinv] = v;
-    }
-  };
-  // inv(L) by block columns jb: X_jb = inv(L_jb,jb), X_ib = -inv(L_ib,ib)
-  // sum_{t=jb}^{ib-1} L[ib][t] X_t; thread (r, c) owns entry (r, c) of a
-  // 16 x 16 block
-  const int r = tid & (LB - 1), c = tid >> 4;
-  for (int jb = 0; jb < LEAF / LB; ++jb) {
-    const int j0 = jb * LB;
-    const T xd = c <= r ? P[pk(j0 + r, j0 + c)] : T(0);  // inv(L_jb,jb)
-    X[(j0 + r) * LB + c] = xd;
-    out(j0 + r, j0 + c, xd);
-    for (int ib = 0; ib < jb; ++ib) out(ib * LB + r, j0 + c, T(0));
-    lds_barrier();
-    for (int ib = jb + 1; ib < LEAF / LB; ++ib) {
-      const int i0 = ib * LB;
-      const T* lrow = P + pk(i0 + r, 0);
-      T a0 = T(0), a1 = T(0);
-      for (int t = j0; t < i0; t += 2) {  // i0 - j0 is a multiple of 16
-        a0 = fma(lrow[t], X[t * LB + c], a0);
-        a1 = fma(lrow[t + 1], X[(t + 1) * LB + c], a1);
-      }
-      X[(i0 + r) * LB + c] = a0 + a1;
-      lds_barrier();
-      const T* drow = P + pk(i0 + r, i0);
-      a0 = T(0);
-      a1 = T(0);
-#pragma unroll
-      for (int s2 = 0; s2 < LB; s2 += 2) {
-        a0 = fma(s2 <= r ? drow[s2] : T(0), X[(i0 + s2) * LB + c], a0);
-        a1 = fma(s2 + 1 <= r ? drow[s2 + 1] : T(0), X[(i0 + s2 + 1) * LB + c], a1);
-      }
-      lds_barrier();
-      X[(i0 + r) * LB + c] = -(a0 + a1);
-      out(i0 + r, j0 + c, -(a0 + a1));
-      lds_barrier();
-    }
-  }
+__device__ __forceinline__ int tile_slot(int i, int k) { return ((i * (i + 1) >> 1) + k) * TS; }
+template <typename T>
+__device__ __forceinline__ int tile_col(int g, int r)
+{
+  return sizeof(T) == 8 ? g + 4 * r : 4 * g + r;
+}
+// position of column c (times 16) inside a tile
+template <typename T>
+__device__ __forceinline__ constexpr int col_pos(int c)
+{
+  return sizeof(T) == 8 ? c : (c >> 2) + 4 * (c & 3);
 }
 
 template <typename T>
-__global__ __launch_bounds__(64) void trtri_leaf_kernel(int uplo, int diag, int n, const T* A, long lda, long sA,
-                                                        T* Tinv, long ldinv, long sInv)
+__device__ __forceinline__ typename LeafV<T>::type tile_load(const T* t, int lane)
 {
-  __shared__ T Ls[LEAF * LLD];
-  const int lane = threadIdx.x;
+  return typename LeafV<T>::type{t[lane], t[lane + 64], t[lane + 128], t[lane + 192]};
+}
+template <typename T, typename V>
+__device__ __forceinline__ void tile_store(T* t, int lane, const V& v)
+{
+#pragma unroll
+  for (int r = 0; r < 4; ++r) t[lane + 64 * r] = v[r];
+}
+// the transpose of the tile at t as an operand
+template <typename T>
+__device__ __forceinline__ typename LeafV<T>::type tile_load_t(const T* t, int lane)
+{
+  typename LeafV<T>::type v;
+  const int row = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = t[tile_col<T>(g, r) + 16 * col_pos<T>(row)];
+  return v;
+}
+// acc + X Y^T
+template <typename V>
+__device__ __forceinline__ V tile_xyt(V acc, const V& x, const V& y)
+{
+#pragma unroll
+  for (int s = 0; s < 4; ++s) acc = leaf_mfma(y[s], x[s], acc);
+  return acc;
+}
+
+// value of lane J of this lane's row of 16 lanes
+template <int J>
+__device__ __forceinline__ double row_bcast(double x)
+{
+  const long y = __builtin_amdgcn_update_dpp(0L, __builtin_bit_cast(long, x), 0x150 + J, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, y);
+}
+template <int J>
+__device__ __forceinline__ float row_bcast(float x)
+{
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x150 + J, 0xf, 0xf, true));
+}
+
+template <typename F, int... J>
+__device__ __forceinline__ void for_each_index(F&& f, std::integer_sequence<int, J...>)
+{
+  (f(std::integral_constant<int, J>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void for_each(F&& f)
+{
+  for_each_index(f, std::make_integer_sequence<int, N>{});
+}
+
+__device__ __forceinline__ double frexp_mant(double p) { return __builtin_amdgcn_frexp_mant(p); }
+__device__ __forceinline__ float frexp_mant(float p) { return __builtin_amdgcn_frexp_mantf(p); }
+__device__ __forceinline__ int frexp_exp(double p) { return __builtin_amdgcn_frexp_exp(p); }
+__device__ __forceinline__ int frexp_exp(float p) { return __builtin_amdgcn_frexp_expf(p); }
+__device__ __forceinline__ double rcp_approx(double p) { return __builtin_amdgcn_rcp(p); }
+__device__ __forceinline__ float rcp_approx(float p) { return __builtin_amdgcn_rcpf(p); }
+__device__ __forceinline__ double scale2(double x, int h) { return __builtin_ldexp(x, h); }
+__device__ __forceinline__ float scale2(float x, int h) { return __builtin_ldexpf(x, h); }
+
+// d += (d of lane J of this lane's row of 16) * m, one instruction.  The
+// hardware wants two wait states between a vector write and such a read of
+// the same register and the compiler does not look into the statement: the
+// callers keep other instructions between (volatile statements stay in order).
+template <int J>
+__device__ __forceinline__ void fmac_bcast(double& d, double m)
+{
+  asm volatile("v_fmac_f64_dpp %0, %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "+v"(d) : "v"(m), "n"(J));
+}
+template <int J>
+__device__ __forceinline__ void fmac_bcast(float& d, float m)
+{
+  asm volatile("v_fmac_f32_dpp %0, %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "+v"(d) : "v"(m), "n"(J));
+}
+
+// x is computed here, between the statements before and after
+template <typename T>
+__device__ __forceinline__ void pin(T& x)
+{
+  asm volatile("" : "+v"(x));
+}
+
+// Cholesky factor and inverse of one 16 x 16 tile by one wave.  In: d[c] =
+// A(i, c), the whole symmetric row i = lane % 16 (the four rows of 16 lanes
+// hold the same data).  Out: l[c] = L(i, c) and d[c] = inv(L)(i, c), zero
+// above the diagonal.  Returns this lane's pivot.
+// Elimination without roots: W A = U with W unit lower triangular, the
+// columns of W taking the place of the eliminated columns, so that each of
+// the 16 steps is one reciprocal and 15 row updates from row j; the pivots'
+// roots follow once, for all 16 pivots at a time: L(i, j) = A_j(i, j) /
+// sqrt(p_j), inv(L) = diag(1 / sqrt(p)) W.
+// A step's chain is pivot (broadcast) -> mantissa -> reciprocal -> two
+// corrections -> multiplier -> next pivot: 8 dependent instructions.  The
+// updates of the step before stand between them, in this order (one wave,
+// in-order issue; ordered by the compiler, a leaf of 128 took 39.6 us instead
+// of 33.4).
+template <typename T>
+__device__ __forceinline__ T factor16(T (&d)[16], T (&l)[16], int i)
+{
+  T m = T(0), piv = T(1);
+  for_each<17>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;  // this step's pivot; the updates are those of pivot j - 1
+    // updates UA .. UB - 1 of pivot j - 1, columns in order from j
+    auto update = [&](auto from, auto to) {
+      if constexpr (j > 0) {
+        for_each<decltype(to)::value - decltype(from)::value>([&](auto q) {
+          constexpr int c = (j + decltype(from)::value + decltype(q)::value) % 16;
+          fmac_bcast<j - 1>(d[c], m);
+        });
+      }
+    };
+#define XK_UPD(a, b) update(std::integral_constant<int, a>{}, std::integral_constant<int, b>{})
+    if constexpr (j == 16) {
+      XK_UPD(0, 15);
+      d[15] = m;
+    } else {
+      XK_UPD(0, 3);
+      T p = row_bcast<j>(d[j]);
+      pin(p);
+      XK_UPD(3, 4);
+      // -A(i, j) / p for the rows below, p = 2^h p' with p' in [0.5, 1) (no
+      // overflow for a denormal p): r = 1 / p' to its hardware accuracy
+      // (1 - e), the quotient corrected by 1 + e + e^2
+      T ps = frexp_mant(p);
+      pin(ps);
+      int row = i;  // compared anew in each step: 32 lane masks do not fit the scalar registers
+      pin(row);
+      int h = -frexp_exp(p);
+      T a = row > j ? -d[j] : T(0);
+      pin(a);
+      XK_UPD(4, 5);
+      T r = rcp_approx(ps);
+      pin(r);
+      T q = scale2(a, h);
+      pin(q);
+      piv = row == j ? p : piv;
+      XK_UPD(5, 8);
+      T e = fma(-ps, r, T(1));
+      pin(e);
+      q *= r;
+      pin(q);
+      XK_UPD(8, 11);
+      e = fma(e, e, e);
+      pin(e);
+      XK_UPD(11, 15);
+      l[j] = d[j];
+      if constexpr (j > 0) d[j - 1] = m;
+      m = fma(q, e, q);
+    }
+#undef XK_UPD
+  });
+  T sq, rs;
+  sqrt_rcp(piv, sq, rs);
+  for_each<16>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    const T rj = row_bcast<j>(rs);
+    l[j] = i > j ? l[j] * rj : (i == j ? sq : T(0));
+    d[j] = i > j ? d[j] * rs : (i == j ? rs : T(0));
+  });
+  return piv;
+}
+
+// Row i = lane % 16 of a lower triangular tile in l[]; y[c] = inv(L)(i, c).
+template <typename T>
+__device__ __forceinline__ void invert16(const T (&l)[16], T (&y)[16], int i, T rdiag)
+{
+#pragma unroll
+  for (int c = 0; c < 16; ++c) y[c] = i == c ? T(1) : T(0);
+  for_each<16>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    // row j is final once scaled; rows below subtract L(i, j) times it
+    const T m = i > j ? l[j] : T(0);
+    for_each<j + 1>([&](auto cc) {
+      constexpr int c = decltype(cc)::value;
+      y[c] = i == j ? y[c] * rdiag : y[c];
+      y[c] = fma(-m, row_bcast<j>(y[c]), y[c]);
+    });
+  });
+}
+
+// The registers of tile operand (row i, columns tile_col(g, .)) out of a full row.
+template <typename T>
+__device__ __forceinline__ typename LeafV<T>::type row_to_tile(const T (&d)[16], int g)
+{
+  typename LeafV<T>::type v;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const T a = d[tile_col<T>(0, r)], b = d[tile_col<T>(1, r)], c = d[tile_col<T>(2, r)], e = d[tile_col<T>(3, r)];
+    const T lo = g & 1 ? b : a, hi = g & 1 ? e : c;
+    v[r] = g & 2 ? hi : lo;
+  }
+  return v;
+}
+
+// The lower triangle (as tiles) of a block of order n <= 16 NT: diagonal
+// tiles whole when sym (mirrored), else zero above the diagonal; rows and
+// columns beyond n are the identity.
+template <typename T, int NT>
+__device__ __forceinline__ void leaf_load(T* S, int uplo, int n, int nt, const T* A, long lda, bool sym, bool unit)
+{
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ti = lane & 15, g = lane >> 4;
+  // tiles of tile row / column `wave` so that all loads of a wave are in
+  // flight together: tile (a, b) with a - b = q for q = 0 .. NT - 1, a = wave
+  typename LeafV<T>::type v[NT];
+#pragma unroll
+  for (int b = 0; b < NT; ++b) {
+    v[b] = typename LeafV<T>::type{0, 0, 0, 0};
+    if (b > wave || wave >= nt) continue;
+    const int row = wave * 16 + ti;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int col = b * 16 + tile_col<T>(g, r);
+      T x = row == col ? T(1) : T(0);
+      if (row < n && col < n) {
+        const int hi = max(row, col), lo = min(row, col);
+        if ((sym || col <= row) && !(unit && row == col)) x = uplo == Lower ? A[hi + (long)lo * lda] : A[lo + (long)hi * lda];
+      }
+      v[b][r] = x;
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < NT; ++b)
+    if (b <= wave && wave < nt) tile_store(S + tile_slot(wave, b), lane, v[b]);
+}
+
+// Cholesky factor and its inverse for one block of order <= 16 NT (NT = 4
+// or 8), one workgroup of NT waves, all products on MFMA tiles.
+// The chain of step k is wave 0's alone: factor and invert diagonal tile k in
+// registers (factor16), form panel tile (k + 1, k) = A inv(L_kk)^T and update
+// diagonal tile k + 1 with it, which is then ready for step k + 1.  Beside
+// the next factor16 the other waves update the remaining trailing tiles and
+// form row k of the inverse, inv(L)(k, j) = -inv(L_kk) sum_t L(k, t)
+// inv(L)(t, j), kept transposed (Z) in the places of row k of L, which
+// nothing reads any more.  Two barriers a step, ordering LDS only.
+// Bound by latency: 16 orders take 4 us, 2.1 of them the 16 dependent pivots;
+// order 128 33 us (FP64), where two leaves of order 64 with scalar panels and
+// the six launches that joined them took 130.
+// LDS: 20.5 KB (FP64, NT = 4), 73.7 KB (NT = 8).
+template <typename T, int NT>
+__global__ __launch_bounds__(64 * NT) void potrf_leaf_kernel(int uplo, int n, T* A, long lda, long sA, T* Tinv,
+                                                             long ldinv, long sInv, int* info, int base, int pair)
+{
+  typedef typename LeafV<T>::type V;
+  __shared__ T S[NT * (NT + 1) / 2 * TS];
+  // the latency-bound step of the diagonal chain may share its CU with
+  // update GEMM waves: its waves issue first
+  __builtin_amdgcn_s_setprio(2);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ti = lane & 15, g = lane >> 4;
+  const int nt = (n + 15) >> 4;
+  A += (long)blockIdx.x * sA;
+  if (Tinv) Tinv += (long)blockIdx.x * sInv;
+  // entry (i, k) of a lower triangle, to the stored triangle
+  auto put = [&](T* M, long ld, int i, int k, T v) {
+    if (i < n && k < n) {
+      if (uplo == Lower) M[i + (long)k * ld] = v;
+      else M[k + (long)i * ld] = v;
+    }
+  };
+  leaf_load<T, NT>(S, uplo, n, nt, A, lda, true, false);
+  lds_barrier();
+  int fail = INT_MAX;  // first order with a non-positive pivot (wave 0)
+  V z = {0, 0, 0, 0};  // this wave's tile of the inverse's current row
+  for (int k = 0; k < nt; ++k) {
+    const int c0 = k * 16;
+    T* Dk = S + tile_slot(k, k);
+    V dk;
+    if (wave == 0) {
+      __builtin_amdgcn_s_setprio(3);
+      T d[16], l[16];
+#pragma unroll
+      for (int c = 0; c < 16; ++c) d[c] = Dk[ti + 16 * col_pos<T>(c)];
+      const T piv = factor16(d, l, ti);
+      const unsigned long long bad = __ballot(!(piv > T(0)) && c0 + ti < n);
+      if (bad && fail == INT_MAX) fail = c0 + __ffsll(bad) - 1;
+      dk = row_to_tile(d, g);
+      tile_store(Dk, lane, dk);
+      const V lk = row_to_tile(l, g);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int col = tile_col<T>(g, r);
+        if (col <= ti) put(A, lda, c0 + ti, c0 + col, lk[r]);
+        if (Tinv) put(Tinv, ldinv, c0 + ti, c0 + col, dk[r]);
+      }
+    }
+    lds_barrier();
+    // row k - 1 of the inverse takes the place of row k - 1 of L
+    if (wave > 0 && wave < k) tile_store(S + tile_slot(k - 1, wave - 1), lane, z);
+    if (wave > 0) dk = tile_load(Dk, lane);
+    // panel: tile row k + 1 + wave
+    V lp = {0, 0, 0, 0};
+    const int pi = k + 1 + wave;
+    if (pi < nt) {
+      T* P = S + tile_slot(pi, k);
+      lp = tile_xyt(lp, tile_load(P, lane), dk);
+      tile_store(P, lane, lp);
+    }
+    lds_barrier();
+    if (wave == 0) {
+      if (k + 1 < nt) {
+        T* C = S + tile_slot(k + 1, k + 1);
+        V c = tile_load(C, lane);
+        c = tile_xyt(c, lp, -lp);
+        tile_store(C, lane, c);
+      }
+    } else {
+      // trailing tiles (i, j), k < j <= i, but the first, dealt to waves 1 ..
+      int t = wave;  // tile index in column order, (k + 1, k + 1) is 0
+      for (int j = k + 1; j < nt; ++j) {
+        const int h = nt - j;
+        for (; t < h; t += NT - 1) {
+          const int i = j + t;
+          T* C = S + tile_slot(i, j);
+          V c = tile_load(C, lane);
+          const V x = tile_load(S + tile_slot(i, k), lane), y = tile_load(S + tile_slot(j, k), lane);
+          c = tile_xyt(c, x, -y);
+          tile_store(C, lane, c);
+        }
+        t -= h;
+      }
+      // row k of the inverse, block column j = wave - 1
+      const int j = wave - 1;
+      if (j < k && Tinv) {
+        V s = {0, 0, 0, 0};
+        s = tile_xyt(s, tile_load_t(S + tile_slot(j, j), lane), tile_load(S + tile_slot(k, j), lane));
+        for (int u = j + 1; u < k; ++u)
+          s = tile_xyt(s, tile_load(S + tile_slot(u, j), lane), tile_load(S + tile_slot(k, u), lane));
+        z = V{0, 0, 0, 0};
+        z = tile_xyt(z, s, -dk);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) put(Tinv, ldinv, c0 + tile_col<T>(g, r), j * 16 + ti, z[r]);
+      }
+    }
+    // the panel's factor entries, and zeros across the diagonal of the inverse
+    if (pi < nt) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int col = c0 + tile_col<T>(g, r);
+        put(A, lda, pi * 16 + ti, col, lp[r]);
+        if (Tinv) put(Tinv, ldinv, col, pi * 16 + ti, T(0));
+      }
+    }
+  }
+  // pair: orders 2i, 2i + 1 stand for order i of a complex block
+  if (threadIdx.x == 0 && fail != INT_MAX) atomicMin(info, pair ? (base + fail) / 2 + 1 : base + fail + 1);
+}
+
+// Inverse of one triangular block of order <= 16 NT, one workgroup of NT
+// waves: wave j inverts diagonal tile j (invert16), then forms block column j
+// of the inverse downwards on MFMA tiles with its own tiles kept in
+// registers: one barrier in all.  The longest column is 35 tile products.
+template <typename T, int NT>
+__global__ __launch_bounds__(64 * NT) void trtri_leaf_kernel(int uplo, int diag, int n, const T* A, long lda, long sA,
+                                                             T* Tinv, long ldinv, long sInv)
+{
+  typedef typename LeafV<T>::type V;
+  __shared__ T S[NT * (NT + 1) / 2 * TS];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ti = lane & 15, g = lane >> 4;
+  const int nt = (n + 15) >> 4;
   A += (long)blockIdx.x * sA;
   Tinv += (long)blockIdx.x * sInv;
-#pragma unroll 4
-  for (int j = 0; j < LEAF; ++j) Ls[lane + j * LLD] = lower_view(A, lda, uplo, n, lane, j);
-  __syncthreads();
-  lower_inverse_to(Ls, lane, diag == Unit, Tinv, ldinv, n, uplo);
+  leaf_load<T, NT>(S, uplo, n, nt, A, lda, false, diag == Unit);
+  // inv(L)(i, k) to the stored triangle (inv(U) = inv(L)^T)
+  auto put = [&](int i, int k, T v) {
+    if (i < n && k < n) {
+      if (uplo == Lower) Tinv[i + (long)k * ldinv] = v;
+      else Tinv[k + (long)i * ldinv] = v;
+    }
+  };
+  if (wave < nt) {
+    T* D = S + tile_slot(wave, wave);  // loaded by this wave
+    T l[16], y[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) l[c] = D[ti + 16 * col_pos<T>(c)];
+    T own = T(1);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) own = ti == c ? l[c] : own;
+    invert16(l, y, ti, T(1) / own);
+    const V d = row_to_tile(y, g);
+    tile_store(D, lane, d);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) put(wave * 16 + ti, wave * 16 + tile_col<T>(g, r), d[r]);
+  }
+  lds_barrier();
+  if (wave >= nt) return;
+  V zt[NT];  // zt[u] = inv(L)(wave + u, wave) transposed
+  zt[0] = tile_load_t(S + tile_slot(wave, wave), lane);
+#pragma unroll
+  for (int v = 1; v < NT; ++v) {
+    const int k = wave + v;
+    if (k >= nt) break;
+    V s = {0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < v; ++u) s = tile_xyt(s, zt[u], tile_load(S + tile_slot(k, wave + u), lane));
+    const V z0 = {0, 0, 0, 0};
+    zt[v] = tile_xyt(z0, s, -tile_load(S + tile_slot(k, k), lane));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = k * 16 + tile_col<T>(g, r), col = wave * 16 + ti;
+      put(row, col, zt[v][r]);
+      put(col, row, T(0));
+    }
+  }
 }
 
 template <typename T>
 void potrf_leaf(hipStream_t s, int uplo, int n, T* A, long lda, long sA, T* Tinv, long ldinv, long sInv,
                 int batch, int* info, int base, int pair)
 {
-  XK_CHECK(n >= 1 && n <= LEAF, "potrf leaf order must be in [1,64]");
+  XK_CHECK(n >= 1 && n <= LEAF, "potrf leaf order must be in [1,128]");
   if (batch <= 0) return;
-  hipLaunchKernelGGL((potrf_leaf_kernel<T>), dim3(batch), dim3(256), 0, s, uplo, n, A, lda, sA, Tinv, ldinv, sInv,
-                     info, base, pair);
+  if (n <= 64)
+    hipLaunchKernelGGL((potrf_leaf_kernel<T, 4>), dim3(batch), dim3(256), 0, s, uplo, n, A, lda, sA, Tinv, ldinv,
+                       sInv, info, base, pair);
+  else
+    hipLaunchKernelGGL((potrf_leaf_kernel<T, 8>), dim3(batch), dim3(512), 0, s, uplo, n, A, lda, sA, Tinv, ldinv,
+                       sInv, info, base, pair);
   XK_HIP(hipGetLastError());
 }
 
@@ -349,10 +518,99 @@ template <typename T>
 void trtri_leaf(hipStream_t s, int uplo, int diag, int n, const T* A, long lda, long sA, T* Tinv, long ldinv,
                 long sInv, int batch)
 {
-  XK_CHECK(n >= 1 && n <= LEAF, "trtri leaf order must be in [1,64]");
+  XK_CHECK(n >= 1 && n <= LEAF, "trtri leaf order must be in [1,128]");
   if (batch <= 0) return;
-  hipLaunchKernelGGL((trtri_leaf_kernel<T>), dim3(batch), dim3(64), 0, s, uplo, diag, n, A, lda, sA, Tinv, ldinv,
-                     sInv);
+  if (n <= 64)
+    hipLaunchKernelGGL((trtri_leaf_kernel<T, 4>), dim3(batch), dim3(256), 0, s, uplo, diag, n, A, lda, sA, Tinv,
+                       ldinv, sInv);
+  else
+    hipLaunchKernelGGL((trtri_leaf_kernel<T, 8>), dim3(batch), dim3(512), 0, s, uplo, diag, n, A, lda, sA, Tinv,
+                       ldinv, sInv);
+  XK_HIP(hipGetLastError());
+}
+
+// P <- P inv(L)^T in place (Upper: P^T <- P^T inv(L)^T with inv(L) = inv(U)^T):
+// a workgroup of four waves takes 16 rows of P (columns, Upper), holds them in
+// LDS as the eight 16 x 16 tiles of their 128 columns, and wave w forms
+// column tiles w and 7 - w of the product (9 tile products each: inv(L) is
+// triangular) with inv(L) read straight from L2 into the operand registers.
+// Every workgroup has read its rows before it writes any, so P needs no copy.
+// Bound by latency (one load of each operand, 36 dependent MFMAs): about 4 us
+// at any m that fits the chip.
+template <typename T>
+__global__ __launch_bounds__(256) void trsm_panel_kernel(int uplo, int m, int n, T* __restrict__ P, long lda,
+                                                         const T* __restrict__ Linv, long ldinv, int prio)
+{
+  typedef typename LeafV<T>::type V;
+  constexpr int NT = LEAF / 16;
+  __shared__ T S[NT * TS];
+  if (prio) __builtin_amdgcn_s_setprio(3);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ti = lane & 15, g = lane >> 4;
+  const int r0 = blockIdx.x * 16;
+  // operand tiles (jn, kt) of inv(L): rows jn, inner index kt
+  auto load_y = [&](int jn, V(&y)[NT]) {
+    const int row = jn * 16 + ti;
+#pragma unroll
+    for (int kt = 0; kt < NT; ++kt) {
+      if (kt > jn) break;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int k = kt * 16 + tile_col<T>(g, r);
+        T v = T(0);
+        if (k <= row && row < n) v = uplo == Lower ? Linv[row + (long)k * ldinv] : Linv[k + (long)row * ldinv];
+        y[kt][r] = v;
+      }
+    }
+  };
+  V y[NT];
+  load_y(wave, y);
+  {
+    T v[NT];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+      const int i = uplo == Lower ? tid & 15 : tid >> 4, k = q * 16 + (uplo == Lower ? tid >> 4 : tid & 15);
+      v[q] = T(0);
+      if (r0 + i < m && k < n) v[q] = uplo == Lower ? P[r0 + i + (long)k * lda] : P[k + (long)(r0 + i) * lda];
+    }
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+      const int i = uplo == Lower ? tid & 15 : tid >> 4, k = uplo == Lower ? tid >> 4 : tid & 15;
+      S[q * TS + i + 16 * col_pos<T>(k)] = v[q];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int jn = h == 0 ? wave : NT - 1 - wave;
+    if (jn * 16 >= n) continue;
+    V acc = {0, 0, 0, 0};
+    if (h == 1) load_y(jn, y);
+#pragma unroll
+    for (int kt = 0; kt < NT; ++kt) {
+      if (kt > jn) break;
+      const V x = tile_load(S + kt * TS, lane);
+      // Upper: the transposed product, so that a lane's neighbours store neighbours
+      acc = uplo == Lower ? tile_xyt(acc, x, y[kt]) : tile_xyt(acc, y[kt], x);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = r0 + (uplo == Lower ? ti : tile_col<T>(g, r)), k = jn * 16 + (uplo == Lower ? tile_col<T>(g, r) : ti);
+      if (i < m && k < n) {
+        if (uplo == Lower) P[i + (long)k * lda] = acc[r];
+        else P[k + (long)i * lda] = acc[r];
+      }
+    }
+  }
+}
+
+template <typename T>
+void trsm_panel(hipStream_t s, int uplo, int m, int n, T* P, long lda, const T* Linv, long ldinv)
+{
+  XK_CHECK(n >= 1 && n <= LEAF, "panel solve: block order must be in [1,128]");
+  if (m <= 0) return;
+  hipLaunchKernelGGL((trsm_panel_kernel<T>), dim3((m + 15) / 16), dim3(256), 0, s, uplo, m, n, P, lda, Linv, ldinv,
+                     gemm_is_priority_stream(s));
   XK_HIP(hipGetLastError());
 }
 
@@ -437,6 +695,7 @@ void fill_int(hipStream_t s, int* p, int n, int v)
 }
 
 #define XK_INST(T)                                                                                           \
+  template void trsm_panel<T>(hipStream_t, int, int, int, T*, long, const T*, long);                           \
   template void potrf_leaf<T>(hipStream_t, int, int, T*, long, long, T*, long, long, int, int*, int, int);         \
   template void trtri_leaf<T>(hipStream_t, int, int, int, const T*, long, long, T*, long, long, int);         \
   template void copy2d<T>(hipStream_t, int, int, const T*, long, T*, long);                                    \

@@ -48,6 +48,7 @@ struct GemmParams {
   int m, n, k;
   int tiles_m, tiles_n;
   int tri;
+  int trap;        // triangle-masked output that is not square: full tile raster, tiles outside it leave at once
   int kmode;       // inner range per tile for a triangular operand (KRANGE_*)
   int vecA, vecB;  // 16-byte vector loads allowed (base and ld aligned)
   int prio;        // raise the waves' issue priority (latency-bound chain steps)
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams<T> p)
   {
     int pid = blockIdx.x;
     const int total = gridDim.x;
-    if (p.tri == TRI_FULL) {
+    if (p.tri == TRI_FULL || p.trap) {
       // a limited inner range makes the work per tile grow along the tile
       // rows or columns: no XCD blocking then (consecutive ids go to
       // different XCDs, which then share light and heavy tiles alike), and
@@ -128,6 +129,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams<T> p)
   }
   const int m0 = tm * BM, n0 = tn * BN;
   const int M = p.m, N = p.n, K = p.k;
+  if (p.trap && (p.tri == TRI_LOWER ? m0 + BM <= n0 : n0 + BN <= m0)) return;
 
   // ---- per-lane load coordinates
   // op(A) slice BM x BK.  !TA: runs along m.  TA: runs along k.
@@ -272,6 +274,7 @@ void gemm_set_tile(int bm) { g_force_tile = bm; }
 // (the latency-bound diagonal chain of POTRF, beside full-chip updates).
 static hipStream_t g_prio_stream = nullptr;
 void gemm_set_priority_stream(hipStream_t s) { g_prio_stream = s; }
+int gemm_is_priority_stream(hipStream_t s) { return s != nullptr && s == g_prio_stream; }
 int gemm_get_tile() { return g_force_tile; }
 
 template <typename T, int BM, int BK>
@@ -279,8 +282,8 @@ static void launch_shape(hipStream_t s, bool ta, bool tb, GemmParams<T>& p, int 
 {
   p.tiles_m = (p.m + BM - 1) / BM;
   p.tiles_n = (p.n + BM - 1) / BM;
-  long ntiles = (p.tri == TRI_FULL) ? (long)p.tiles_m * p.tiles_n
-                                    : (long)p.tiles_m * (p.tiles_m + 1) / 2;
+  long ntiles = (p.tri == TRI_FULL || p.trap) ? (long)p.tiles_m * p.tiles_n
+                                              : (long)p.tiles_m * (p.tiles_m + 1) / 2;
   XK_CHECK(ntiles < (1L << 31), "gemm grid too large");
   dim3 grid((unsigned)ntiles, 1, (unsigned)batch), block(256);
   if (!ta && !tb) hipLaunchKernelGGL((gemm_kernel<T, BM, BM, BK, false, false>), grid, block, 0, s, p);
@@ -295,9 +298,11 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, c
           const T* B, long ldb, T beta, T* C, long ldc, int tri, int batch, long sA, long sB, long sC, int kmode)
 {
   if (m <= 0 || n <= 0 || batch <= 0) return;
-  if (tri != TRI_FULL) XK_CHECK(m == n, "triangular gemm output must be square");
+  if (tri != TRI_FULL)
+    XK_CHECK(tri == TRI_LOWER ? m >= n : n >= m, "triangular gemm output must hold its whole diagonal");
   GemmParams<T> p;
   p.m = m; p.n = n; p.k = k; p.tri = tri; p.kmode = kmode;
+  p.trap = tri != TRI_FULL && m != n;
   p.alpha = alpha; p.beta = beta;
   p.A = A; p.lda = lda; p.sA = sA;
   p.B = B; p.ldb = ldb; p.sB = sB;
@@ -305,7 +310,7 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, c
   auto aligned = [](const void* q, long ld, long stride) {
     return ((uintptr_t)q % 16 == 0) && ((ld * (long)sizeof(T)) % 16 == 0) && ((stride * (long)sizeof(T)) % 16 == 0);
   };
-  p.prio = s == g_prio_stream && s != nullptr;
+  p.prio = gemm_is_priority_stream(s);
   p.vecA = aligned(A, lda, sA);
   p.vecB = aligned(B, ldb, sB);
   const bool ta = transA != NoTrans, tb = transB != NoTrans;
@@ -321,7 +326,7 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, c
     // tiles, four times the workgroups; the k order per element, hence the
     // result, is the same
     long t64 = (long)((m + 63) / 64) * ((n + 63) / 64);
-    if (p.tri != TRI_FULL) t64 = t64 / 2 + (m + 63) / 64;
+    if (p.tri != TRI_FULL && !p.trap) t64 = t64 / 2 + (m + 63) / 64;
     if (sizeof(T) == 8 && t64 * batch < 512) bm = 32;
   }
   if (bm == 128) launch_shape<T, 128, 16>(s, ta, tb, p, batch);

@@ -7,7 +7,9 @@
 namespace xk {
 
 // C <- alpha op(A) op(B) + beta C, op(A) m x k, op(B) k x n.  `tri` restricts
-// the written part of C to one triangle (C's (0,0) lies on the diagonal).
+// the written part of C to one triangle (C's (0,0) lies on the diagonal);
+// with TRI_LOWER m > n (TRI_UPPER: n > m) is the trapezoid below (right of)
+// the diagonal.
 // `batch` > 1 runs independent problems at element strides sA, sB, sC.
 // beta == 0 never reads C.  FP64 uses v_mfma_f64_16x16x4f64, FP32 uses
 // v_mfma_f32_16x16x4f32; tiles are staged through LDS, double-buffered.
@@ -23,7 +25,7 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha,
 void gemm_set_tile(int bm);
 int gemm_get_tile();
 
-// Cholesky of `batch` diagonal blocks of order n <= 64 (lower storage, or
+// Cholesky of `batch` diagonal blocks of order n <= 128 (lower storage, or
 // upper when uplo == Upper), in place, plus the inverse of each factor
 // written to Linv (lower: inv(L); upper: inv(U)).  info[0] receives
 // base_order + j + 1 for the first non-positive pivot (atomic min, starts at
@@ -34,11 +36,17 @@ template <typename T>
 void potrf_leaf(hipStream_t s, int uplo, int n, T* A, long lda, long strideA, T* Linv, long ldinv,
                 long strideInv, int batch, int* info, int base_order, int pair = 0);
 
-// Inverse of `batch` triangular blocks of order n <= 64 into Tinv (the other
+// Inverse of `batch` triangular blocks of order n <= 128 into Tinv (the other
 // triangle of Tinv is zeroed, like the full block).
 template <typename T>
 void trtri_leaf(hipStream_t s, int uplo, int diag, int n, const T* A, long lda, long strideA, T* Tinv,
                 long ldinv, long strideInv, int batch);
+
+// P <- P inv(L)^T in place for the m x n block P below (Lower) a factored
+// diagonal block of order n <= 128 with inverse Linv = inv(L); Upper: P (n x m)
+// <- inv(U)^T P right of it, Linv = inv(U).
+template <typename T>
+void trsm_panel(hipStream_t s, int uplo, int m, int n, T* P, long lda, const T* Linv, long ldinv);
 
 // Y <- X (m x n blocks), element-wise copy between column-major buffers.
 template <typename T>
@@ -60,6 +68,7 @@ void fill_int(hipStream_t s, int* p, int n, int v);
 // priority: the latency-bound diagonal chain of POTRF beside full-chip
 // trailing updates.
 void gemm_set_priority_stream(hipStream_t s);
+int gemm_is_priority_stream(hipStream_t s);
 // device address of the allocation-free batched run's fixed array, for the
 // current device (called once per device at initialisation)
 void batch_noalloc_init();
