@@ -74,6 +74,9 @@ static void fill_zero(hipStream_t s, int m, int n, T* Y, long ldy)
   gemm<T>(s, NoTrans, NoTrans, m, n, 0, T(0), Y, ldy, Y, ldy, T(0), Y, ldy);
 }
 
+// Leading dimension of a scratch operand of m rows: 16-byte aligned columns.
+static inline long even_ld(int m) { return (m + 3) / 4 * 4; }
+
 // Inverses of `cnt` triangular blocks of order n (block b at A + b sA,
 // leading dimension lda) into Tinv + b sInv: leaves of order LEAF, then pairs
 // of neighbouring blocks joined level by level, I21 = -I22 A21 I11 (Upper: I12
@@ -110,17 +113,17 @@ static void inverse_levels(hipStream_t s, int uplo, int diag, int n, const T* A,
       const T* Ab = A + oa;
       T* Ib = Tinv + oi;
       T* I22 = Ib + (long)h * (1 + ldinv);
-      const long sW = (long)h * n2;
+      const long ldw = even_ld(uplo == Lower ? n2 : h), sW = ldw * (uplo == Lower ? h : n2);
       T* W = (T*)scratch(wslot, sizeof(T) * (size_t)sW * batch);
       if (uplo == Lower) {
-        gemm<T>(s, NoTrans, NoTrans, n2, h, h, T(1), Ab + h, lda, Ib, ldinv, T(0), W, n2, TRI_FULL, batch, da, di, sW,
+        gemm<T>(s, NoTrans, NoTrans, n2, h, h, T(1), Ab + h, lda, Ib, ldinv, T(0), W, ldw, TRI_FULL, batch, da, di, sW,
                 KRANGE_B_LOWER);
-        gemm<T>(s, NoTrans, NoTrans, n2, h, n2, T(-1), I22, ldinv, W, n2, T(0), Ib + h, ldinv, TRI_FULL, batch, di, sW,
-                di, KRANGE_A_LOWER);
+        gemm<T>(s, NoTrans, NoTrans, n2, h, n2, T(-1), I22, ldinv, W, ldw, T(0), Ib + h, ldinv, TRI_FULL, batch, di,
+                sW, di, KRANGE_A_LOWER);
       } else {
-        gemm<T>(s, NoTrans, NoTrans, h, n2, n2, T(1), Ab + (long)h * lda, lda, I22, ldinv, T(0), W, h, TRI_FULL, batch,
-                da, di, sW, KRANGE_B_UPPER);
-        gemm<T>(s, NoTrans, NoTrans, h, n2, h, T(-1), Ib, ldinv, W, h, T(0), Ib + (long)h * ldinv, ldinv, TRI_FULL,
+        gemm<T>(s, NoTrans, NoTrans, h, n2, n2, T(1), Ab + (long)h * lda, lda, I22, ldinv, T(0), W, ldw, TRI_FULL,
+                batch, da, di, sW, KRANGE_B_UPPER);
+        gemm<T>(s, NoTrans, NoTrans, h, n2, h, T(-1), Ib, ldinv, W, ldw, T(0), Ib + (long)h * ldinv, ldinv, TRI_FULL,
                 batch, di, sW, di, KRANGE_A_UPPER);
       }
     };
@@ -378,22 +381,23 @@ void dev_potrf(const Exec& x, int uplo, int n, T* A, long lda, int nb, int* info
     const int r2 = rest - k1;
     const int c0 = pair ? k - 1 : k;
     const int kw = (k + 1 - c0) * nb;
-    T* W = (T*)scratch(WS_PANEL, sizeof(T) * (size_t)rest * kk);
+    const long ldw = even_ld(uplo == Lower ? rest : kk);
+    T* W = (T*)scratch(WS_PANEL, sizeof(T) * (size_t)ldw * (uplo == Lower ? kk : rest));
     if (uplo == Lower) {
       T* P = blk(k + 1, k);  // rest x kk panel
       // the panel's rows in block row k+1 first: the lookahead reads only
       // them, so the next diagonal factorization waits for k1 rows of the
       // panel product instead of all of them
-      copy2d<T>(x.s, k1, kk, P, lda, W, rest);
-      dev_gemm<T>(x, NoTrans, Trans, k1, kk, kk, T(1), W, rest, ik, nb, T(0), P, lda);
+      copy2d<T>(x.s, k1, kk, P, lda, W, ldw);
+      dev_gemm<T>(x, NoTrans, Trans, k1, kk, kk, T(1), W, ldw, ik, nb, T(0), P, lda);
       const T* U = A + (long)(k + 1) * nb + (long)c0 * nb * lda;  // rest x kw
       if (split) split_cache_register((const double*)U, lda, rest, kw, 1);
       // lookahead: update the next diagonal block and factor it on the side
       dev_syrk<T>(x, Lower, NoTrans, k1, kw, T(-1), U, lda, T(1), blk(k + 1, k + 1), lda);
       if (lookahead) XK_HIP(hipEventRecord(ev_look, x.s));
       if (r2 > 0) {
-        copy2d<T>(x.s, r2, kk, P + k1, lda, W + k1, rest);
-        dev_gemm<T>(x, NoTrans, Trans, r2, kk, kk, T(1), W + k1, rest, ik, nb, T(0), P + k1, lda);
+        copy2d<T>(x.s, r2, kk, P + k1, lda, W + k1, ldw);
+        dev_gemm<T>(x, NoTrans, Trans, r2, kk, kk, T(1), W + k1, ldw, ik, nb, T(0), P + k1, lda);
       }
       // the rest is enqueued before the diagonal factorization's many small
       // launches, so the compute stream has work while the host issues them:
@@ -416,15 +420,15 @@ void dev_potrf(const Exec& x, int uplo, int n, T* A, long lda, int nb, int* info
     } else {
       T* P = blk(k, k + 1);  // kk x rest panel
       // the panel's columns in block column k+1 first (as above)
-      copy2d<T>(x.s, kk, k1, P, lda, W, kk);
-      dev_gemm<T>(x, Trans, NoTrans, kk, k1, kk, T(1), ik, nb, W, kk, T(0), P, lda);
+      copy2d<T>(x.s, kk, k1, P, lda, W, ldw);
+      dev_gemm<T>(x, Trans, NoTrans, kk, k1, kk, T(1), ik, nb, W, ldw, T(0), P, lda);
       const T* U = A + (long)c0 * nb + (long)(k + 1) * nb * lda;  // kw x rest
       if (split) split_cache_register((const double*)U, lda, rest, kw, 0);
       dev_syrk<T>(x, Upper, Trans, k1, kw, T(-1), U, lda, T(1), blk(k + 1, k + 1), lda);
       if (lookahead) XK_HIP(hipEventRecord(ev_look, x.s));
       if (r2 > 0) {
-        copy2d<T>(x.s, kk, r2, P + (long)k1 * lda, lda, W + (long)k1 * kk, kk);
-        dev_gemm<T>(x, Trans, NoTrans, kk, r2, kk, T(1), ik, nb, W + (long)k1 * kk, kk, T(0), P + (long)k1 * lda,
+        copy2d<T>(x.s, kk, r2, P + (long)k1 * lda, lda, W + (long)k1 * ldw, ldw);
+        dev_gemm<T>(x, Trans, NoTrans, kk, r2, kk, T(1), ik, nb, W + (long)k1 * ldw, ldw, T(0), P + (long)k1 * lda,
                     lda);
       }
       if (r2 > 0) {
@@ -499,7 +503,8 @@ static void trsm_sweep(const Exec& x, int side, int uplo, int transA, int m, int
   };
   const int ta = tr ? Trans : NoTrans;
   if (side == Left) {
-    T* W = (T*)scratch(WS_TRSMW, sizeof(T) * (size_t)nb * n);
+    const long ldw = even_ld(nb);
+    T* W = (T*)scratch(WS_TRSMW, sizeof(T) * (size_t)ldw * n);
     for (int s = 0; s < nblk; ++s) {
       const int k = lower_eff ? s : nblk - 1 - s;
       const int kk = bsz(k);
@@ -508,8 +513,8 @@ static void trsm_sweep(const Exec& x, int side, int uplo, int transA, int m, int
       // the inverse product reads Bk and writes it: through W, or through
       // the split-k partials
       if (!gemm_splitk<T>(x.s, ta, NoTrans, kk, n, kk, la, inv + (size_t)k * nb * nb, nb, Bk, ldb, T(0), Bk, ldb)) {
-        copy2d<T>(x.s, kk, n, Bk, ldb, W, kk);
-        gemm<T>(x.s, ta, NoTrans, kk, n, kk, la, inv + (size_t)k * nb * nb, nb, W, kk, T(0), Bk, ldb);
+        copy2d<T>(x.s, kk, n, Bk, ldb, W, ldw);
+        gemm<T>(x.s, ta, NoTrans, kk, n, kk, la, inv + (size_t)k * nb * nb, nb, W, ldw, T(0), Bk, ldb);
       }
       if (s == nblk - 1) break;
       const bool plain = !split_enabled<T>(x);
@@ -525,7 +530,8 @@ static void trsm_sweep(const Exec& x, int side, int uplo, int transA, int m, int
       }
     }
   } else {
-    T* W = (T*)scratch(WS_TRSMW, sizeof(T) * (size_t)m * nb);
+    const long ldw = even_ld(m);
+    T* W = (T*)scratch(WS_TRSMW, sizeof(T) * (size_t)ldw * nb);
     const bool forward = !lower_eff;  // X T = B with T upper: first column block first
     for (int s = 0; s < nblk; ++s) {
       const int k = forward ? s : nblk - 1 - s;
@@ -533,8 +539,8 @@ static void trsm_sweep(const Exec& x, int side, int uplo, int transA, int m, int
       const T la = s == 0 ? alpha : T(1);
       T* Bk = B + (long)k * nb * ldb;
       if (!gemm_splitk<T>(x.s, NoTrans, ta, m, kk, kk, la, Bk, ldb, inv + (size_t)k * nb * nb, nb, T(0), Bk, ldb)) {
-        copy2d<T>(x.s, m, kk, Bk, ldb, W, m);
-        gemm<T>(x.s, NoTrans, ta, m, kk, kk, la, W, m, inv + (size_t)k * nb * nb, nb, T(0), Bk, ldb);
+        copy2d<T>(x.s, m, kk, Bk, ldb, W, ldw);
+        gemm<T>(x.s, NoTrans, ta, m, kk, kk, la, W, ldw, inv + (size_t)k * nb * nb, nb, T(0), Bk, ldb);
       }
       if (s == nblk - 1) break;
       const bool plain = !split_enabled<T>(x);
@@ -1184,9 +1190,10 @@ int dev_posv_ir(const Exec& x, const Exec& xl, const Exec& xf, int uplo, int n, 
       else to_f32(x.s, kk, n - r0, F + r0 + (long)r0 * ldf, ldf, nullptr, F32 + r0 + (long)r0 * ldf, ldf);
     }
     if (!gemm_splitk<double>(x.s, tA, NoTrans, kk, nrhs, kk, 1.0, ik, nbf, Xk, ldx, 0.0, Xk, ldx)) {
-      double* W = (double*)scratch(WS_TRSMW, sizeof(double) * (size_t)kk * nrhs);
-      copy2d<double>(x.s, kk, nrhs, Xk, ldx, W, kk);
-      gemm<double>(x.s, tA, NoTrans, kk, nrhs, kk, 1.0, ik, nbf, W, kk, 0.0, Xk, ldx);
+      const long ldw = even_ld(kk);
+      double* W = (double*)scratch(WS_TRSMW, sizeof(double) * (size_t)ldw * nrhs);
+      copy2d<double>(x.s, kk, nrhs, Xk, ldx, W, ldw);
+      gemm<double>(x.s, tA, NoTrans, kk, nrhs, kk, 1.0, ik, nbf, W, ldw, 0.0, Xk, ldx);
     }
     if (rest > 0) {
       // block column k of L below its diagonal block, or block row k of U

@@ -1,7 +1,8 @@
 // gemm.hip — FP64/FP32 MFMA GEMM for gfx950 (the tile body of every BLAS-3
-// call in the library).
+// call in the library): gemm_dma_kernel for aligned operands, gemm_kernel for
+// the rest.
 //
-// Work decomposition.  One workgroup (4 waves, 256 lanes) owns a BM x BN
+// Work decomposition of gemm_kernel.  One workgroup (4 waves, 256 lanes) owns a BM x BN
 // macro tile of C; each wave owns a (BM/2) x (BN/2) quarter as (BM/32) x
 // (BN/32) accumulators of 16x16 (v_mfma_*_16x16x4: 4 doubles / floats per
 // lane).  The k loop streams BK-deep slices of op(A) and op(B) through two
@@ -22,6 +23,8 @@
 // rastered in groups of 8 tile rows so that concurrently running tiles of one
 // XCD share op(A) panels in its L2.
 #include "common.h"
+#include <cmath>
+#include <type_traits>
 #include "tiles.h"
 #include "kernels.h"
 
@@ -61,6 +64,16 @@ struct GemmParams {
   long ldc, sC;
 };
 
+typedef __attribute__((address_space(3))) void lds_void;
+
+// at most CNT vector memory operations still in flight
+template <int CNT>
+__device__ __forceinline__ void wait_vmcnt()
+{
+  static_assert(CNT < 64, "vmcnt has six bits");
+  __builtin_amdgcn_s_waitcnt((CNT & 15) | ((CNT >> 4) << 14) | 0x0f70);
+}
+
 // Load V consecutive elements starting at p (16-byte aligned when vec).
 template <typename T, int V>
 __device__ __forceinline__ void load_run(const T* p, T (&r)[V])
@@ -72,6 +85,72 @@ __device__ __forceinline__ void load_run(const T* p, T (&r)[V])
   for (int i = 0; i < (int)(V * sizeof(T) / 16); ++i) {
     v16 x = q[i];
     __builtin_memcpy(reinterpret_cast<char*>(r) + 16 * i, &x, 16);
+  }
+}
+
+// First row and column of this workgroup's BM x BN tile; false when there is
+// nothing of it to write.
+template <int BM, int BN, typename T>
+__device__ __forceinline__ bool tile_origin(const GemmParams<T>& p, int& m0, int& n0)
+{
+  int pid = blockIdx.x, tm, tn;
+  const int total = gridDim.x;
+  if (p.tri == TRI_FULL || p.trap) {
+    // a limited inner range makes the work per tile grow along the tile
+    // rows or columns: no XCD blocking then (consecutive ids go to
+    // different XCDs, which then share light and heavy tiles alike), and
+    // the heaviest tiles are dispatched first
+    if (p.kmode == KRANGE_ALL) pid = xcd_range(pid, total);
+    constexpr int GM = 8;
+    const int group = GM * p.tiles_n;
+    const int g = pid / group;
+    const int first = g * GM;
+    const int gm = min(p.tiles_m - first, GM);
+    const int r = pid - g * group;
+    tm = first + r % gm;
+    tn = r / gm;
+    if (p.kmode == KRANGE_A_LOWER) tm = p.tiles_m - 1 - tm;
+    else if (p.kmode == KRANGE_B_UPPER) tn = p.tiles_n - 1 - tn;
+  } else {
+    int i, j;
+    tri_tile<8>(pid, total, p.tiles_m, i, j);
+    if (p.tri == TRI_LOWER) { tm = i; tn = j; }
+    else { tm = j; tn = i; }
+  }
+  m0 = tm * BM;
+  n0 = tn * BN;
+  return !(p.trap && (p.tri == TRI_LOWER ? m0 + BM <= n0 : n0 + BN <= m0));
+}
+
+// C = alpha acc + beta C on the selected triangle: the wave's TM x TN blocks
+// of 16 x 16 at rows gm0, columns gn0.
+template <typename T, int TM, int TN>
+__device__ __forceinline__ void store_tile(const GemmParams<T>& p, T* __restrict__ C, int gm0, int gn0, int lane,
+                                           const typename AccT<T>::type (&acc)[TM][TN])
+{
+  const T alpha = p.alpha, beta = p.beta;
+  const int lr = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int gm = gm0 + i * 16 + lr;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        // output row of the 16x16 MFMA block held by (lane, r): f64 uses
+        // lane/16 + 4r, f32 uses 4(lane/16) + r (measured on gfx950)
+        const int gn = gn0 + j * 16 + (sizeof(T) == 8 ? lk + 4 * r : lk * 4 + r);
+        bool ok = gm < p.m && gn < p.n;
+        if (p.tri == TRI_LOWER) ok = ok && gm >= gn;
+        else if (p.tri == TRI_UPPER) ok = ok && gm <= gn;
+        if (ok) {
+          T* c = C + (long)gm + (long)gn * p.ldc;
+          T v = alpha * acc[i][j][r];
+          if (beta != T(0)) v += beta * *c;
+          *c = v;
+        }
+      }
+    }
   }
 }
 
@@ -99,37 +178,9 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams<T> p)
   const T* __restrict__ B = p.B + (long)blockIdx.z * p.sB;
   T* __restrict__ C = p.C + (long)blockIdx.z * p.sC;
 
-  // ---- tile of this workgroup
-  int tm, tn;
-  {
-    int pid = blockIdx.x;
-    const int total = gridDim.x;
-    if (p.tri == TRI_FULL || p.trap) {
-      // a limited inner range makes the work per tile grow along the tile
-      // rows or columns: no XCD blocking then (consecutive ids go to
-      // different XCDs, which then share light and heavy tiles alike), and
-      // the heaviest tiles are dispatched first
-      if (p.kmode == KRANGE_ALL && (total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);
-      constexpr int GM = 8;
-      const int group = GM * p.tiles_n;
-      const int g = pid / group;
-      const int first = g * GM;
-      const int gm = min(p.tiles_m - first, GM);
-      const int r = pid - g * group;
-      tm = first + r % gm;
-      tn = r / gm;
-      if (p.kmode == KRANGE_A_LOWER) tm = p.tiles_m - 1 - tm;
-      else if (p.kmode == KRANGE_B_UPPER) tn = p.tiles_n - 1 - tn;
-    } else {
-      int i, j;
-      tri_tile<8>(pid, total, p.tiles_m, i, j);
-      if (p.tri == TRI_LOWER) { tm = i; tn = j; }
-      else { tm = j; tn = i; }
-    }
-  }
-  const int m0 = tm * BM, n0 = tn * BN;
   const int M = p.m, N = p.n, K = p.k;
-  if (p.trap && (p.tri == TRI_LOWER ? m0 + BM <= n0 : n0 + BN <= m0)) return;
+  int m0, n0;
+  if (!tile_origin<BM, BN>(p, m0, n0)) return;
 
   // ---- per-lane load coordinates
   // op(A) slice BM x BK.  !TA: runs along m.  TA: runs along k.
@@ -241,30 +292,190 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams<T> p)
     }
   }
 
-  // ---- epilogue: C = alpha acc + beta C on the selected triangle
-  const T alpha = p.alpha, beta = p.beta;
+  store_tile<T, TM, TN>(p, C, m0 + wm * WTM, n0 + wn * WTN, lane, acc);
+}
+
+// The kernel of aligned operands (16-byte base and leading dimension).  A
+// workgroup of four waves owns a BM x BM tile, each wave a quarter; slices of
+// 128 bytes of the inner dimension (16 doubles, 32 floats) go from memory
+// straight to LDS (1 KB per instruction, no registers between) through a ring
+// of NST stages: the loads of NST - 1 stages are in flight while one is
+// multiplied, one barrier per stage.
+// An operand whose rows (op(A): m, op(B): n) are contiguous in memory is kept
+// k-major, block b of 16 elements of row k at b ^ swizzle(k); one whose inner
+// index is contiguous is kept row-major (128 bytes a row), chunk c (16 bytes)
+// of row m at c ^ (m / 2 % 8): with these places every operand read (b64 or
+// b32 per lane) meets each bank once.  Rows beyond the matrix repeat its last
+// one (they only reach results that are not stored); a remainder of the inner
+// dimension is staged through registers with zeros.  A wave whose quarter
+// lies partly or wholly beyond the matrix multiplies only the 16 x 16 blocks
+// that hold results.
+// The inner order per element is gemm_kernel's: the same bits.
+template <typename T, int BM, int NST, bool TA, bool TB>
+__global__ __launch_bounds__(256, 2) void gemm_dma_kernel(GemmParams<T> p)
+{
+  constexpr int SZ = sizeof(T), E = 16 / SZ, BK = 128 / SZ;
+  constexpr int OP = BM * 128;      // bytes of one operand's stage
+  constexpr int CR = BM * SZ / 16;  // chunks of a k-major row
+  constexpr int Q = BM / 32;        // load instructions per wave, operand and stage
+  constexpr int TQ = BM / 32;       // 16 x 16 blocks of a wave's quarter, each way
+  typedef typename AccT<T>::type acc_t;
+  __shared__ __attribute__((aligned(1024))) char S[NST * 2 * OP];
+  if (p.prio) __builtin_amdgcn_s_setprio(3);
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave & 1, wn = wave >> 1;
+  const T* __restrict__ A = p.A + (long)blockIdx.z * p.sA;
+  const T* __restrict__ B = p.B + (long)blockIdx.z * p.sB;
+  T* __restrict__ C = p.C + (long)blockIdx.z * p.sC;
+  const int M = p.m, N = p.n, K = p.k;
+  int m0, n0;
+  if (!tile_origin<BM, BM>(p, m0, n0)) return;
+
+  // block permutation of k-major row k: rows that the lanes of one read take
+  // together (k .. k + 3) fall into different banks
+  auto swizzle = [](int k) { return SZ == 8 ? k & 1 : BM == 32 ? (k >> 1) & 1 : k & 3; };
+  // Place q of this lane in a stage of an operand: 16 bytes, elements
+  // (row, k ..) row-major or (row .., k) k-major of the tile.
+  auto place = [&](bool kmajor, int q, int& row, int& k) {
+    const int idx = (wave * Q + q) * 64 + lane;
+    if (kmajor) {
+      k = idx / CR;
+      row = ((idx % CR) ^ (swizzle(k) * (16 / E))) * E;
+    } else {
+      row = idx >> 3;
+      k = ((idx & 7) ^ ((row >> 1) & 7)) * E;
+    }
+  };
+  // byte offsets of those elements from the tile's first row at k = 0
+  unsigned offA[Q], offB[Q];
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int gm = m0 + wm * WTM + i * 16 + lr;
+  for (int q = 0; q < Q; ++q) {
+    int row, k;
+    place(!TA, q, row, k);
+    row = TA ? min(row, M - 1 - m0) : min(row, (M - 1) / E * E - m0);
+    offA[q] = (unsigned)(TA ? k + row * p.lda : row + k * p.lda) * SZ;
+    place(TB, q, row, k);
+    row = TB ? min(row, (N - 1) / E * E - n0) : min(row, N - 1 - n0);
+    offB[q] = (unsigned)(TB ? row + k * p.ldb : k + row * p.ldb) * SZ;
+  }
+  const char* A0 = reinterpret_cast<const char*>(TA ? A + m0 * p.lda : A + m0);
+  const char* B0 = reinterpret_cast<const char*>(TB ? B + n0 : B + n0 * p.ldb);
+  const long stepA = (TA ? 1 : p.lda) * SZ, stepB = (TB ? p.ldb : 1) * SZ;  // bytes per k
+  auto issue = [&](int buf, int k0) {
+    const char* a = A0 + k0 * stepA;
+    const char* b = B0 + k0 * stepB;
+    char* s = S + buf * 2 * OP + wave * (Q * 1024);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
+    for (int q = 0; q < Q; ++q)
+      __builtin_amdgcn_global_load_lds((const void*)(a + offA[q]), (lds_void*)(s + q * 1024), 16, 0, 0);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        // output row of the 16x16 MFMA block held by (lane, r): f64 uses
-        // lane/16 + 4r, f32 uses 4(lane/16) + r (measured on gfx950)
-        const int gn = n0 + wn * WTN + j * 16 + (sizeof(T) == 8 ? lk + 4 * r : lk * 4 + r);
-        bool ok = gm < M && gn < N;
-        if (p.tri == TRI_LOWER) ok = ok && gm >= gn;
-        else if (p.tri == TRI_UPPER) ok = ok && gm <= gn;
-        if (ok) {
-          T* c = C + (long)gm + (long)gn * p.ldc;
-          T v = alpha * acc[i][j][r];
-          if (beta != T(0)) v += beta * *c;
-          *c = v;
+    for (int q = 0; q < Q; ++q)
+      __builtin_amdgcn_global_load_lds((const void*)(b + offB[q]), (lds_void*)(s + OP + q * 1024), 16, 0, 0);
+  };
+  // the same through registers, zeros from k = kend on
+  auto issue_tail = [&](int buf, int k0, int kend) {
+#pragma unroll
+    for (int op = 0; op < 2; ++op) {
+      const bool kmajor = op == 0 ? !TA : TB;
+      const char* base = op == 0 ? A0 + k0 * stepA : B0 + k0 * stepB;
+      const int rows = op == 0 ? M - m0 : N - n0;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        int row, k;
+        place(kmajor, q, row, k);
+        T v[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const int rr = row + (kmajor ? e : 0), kk = k + (kmajor ? 0 : e);
+          v[e] = rr < rows && k0 + kk < kend
+                     ? *reinterpret_cast<const T*>(base + (op == 0 ? offA[q] : offB[q]) + e * SZ) : T(0);
+        }
+        __builtin_memcpy(S + buf * 2 * OP + op * OP + (wave * Q + q) * 1024 + lane * 16, v, 16);
+      }
+    }
+  };
+
+  acc_t acc[TQ][TQ];
+#pragma unroll
+  for (int i = 0; i < TQ; ++i)
+#pragma unroll
+    for (int j = 0; j < TQ; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+
+  const int lr = lane & 15, lk = lane >> 4;
+  // operand element of block i, inner index 4 s + lk, in a stage
+  auto operand = [&](const char* s, bool kmajor, int w, int i, int ks) -> T {
+    const int k = ks * 4 + lk;
+    int off;
+    if (kmajor) off = k * (BM * SZ) + (((w * TQ + i) ^ swizzle(k)) * 16 + lr) * SZ;
+    else off = (w * (BM / 2) + i * 16 + lr) * 128 + ((k / E) ^ ((lr >> 1) & 7)) * 16 + (k % E) * SZ;
+    return *reinterpret_cast<const T*>(s + off);
+  };
+
+  int kbeg = 0, kend = K;
+  if (p.kmode == KRANGE_A_LOWER) kend = min(K, m0 + BM);
+  else if (p.kmode == KRANGE_A_UPPER) kbeg = m0;
+  else if (p.kmode == KRANGE_B_UPPER) kend = min(K, n0 + BM);
+  else if (p.kmode == KRANGE_B_LOWER) kbeg = n0;
+  const int nk = (kend - kbeg + BK - 1) / BK;
+  auto stage = [&](int kt) {
+    const int k0 = kbeg + kt * BK;
+    if (k0 + BK <= kend) issue(kt % NST, k0);
+    else issue_tail(kt % NST, k0, kend);
+  };
+  // blocks of this wave's quarter that hold results
+  const int ni = min(TQ, max(0, (M - m0 - wm * (BM / 2) + 15) >> 4));
+  const int nj = min(TQ, max(0, (N - n0 - wn * (BM / 2) + 15) >> 4));
+#pragma unroll
+  for (int st = 0; st < NST - 1; ++st)
+    if (st < nk) stage(st);
+  // the waves of a workgroup meet in the same barriers whichever loop they run
+  auto loop = [&](auto whole) {
+    for (int kt = 0; kt < nk; ++kt) {
+      // this stage has landed for every wave (of the stages after it up to
+      // NST - 2 may be in flight), and every wave has read the one whose
+      // place the next stage takes
+      if (NST > 2 && kt + NST - 2 < nk) wait_vmcnt<(NST - 2) * 2 * Q>();
+      else wait_vmcnt<0>();
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+      if (kt + NST - 1 < nk) stage(kt + NST - 1);
+      const char* s = S + (kt % NST) * 2 * OP;
+      if constexpr (decltype(whole)::value) {
+#pragma unroll
+        for (int ks = 0; ks < BK / 4; ++ks) {
+          T af[TQ], bf[TQ];
+#pragma unroll
+          for (int i = 0; i < TQ; ++i) af[i] = operand(s, !TA, wm, i, ks);
+#pragma unroll
+          for (int j = 0; j < TQ; ++j) bf[j] = operand(s + OP, TB, wn, j, ks);
+#pragma unroll
+          for (int i = 0; i < TQ; ++i)
+#pragma unroll
+            for (int j = 0; j < TQ; ++j) acc[i][j] = mfma16(bf[j], af[i], acc[i][j]);
+        }
+      } else if (ni > 0 && nj > 0) {
+#pragma unroll 1
+        for (int ks = 0; ks < BK / 4; ++ks) {
+          T af[TQ];
+#pragma unroll
+          for (int i = 0; i < TQ; ++i) af[i] = operand(s, !TA, wm, i, ks);
+#pragma unroll
+          for (int j = 0; j < TQ; ++j) {
+            if (j >= nj) break;
+            const T bf = operand(s + OP, TB, wn, j, ks);
+#pragma unroll
+            for (int i = 0; i < TQ; ++i)
+              if (i < ni) acc[i][j] = mfma16(bf, af[i], acc[i][j]);
+          }
         }
       }
     }
-  }
+  };
+  if (ni == TQ && nj == TQ) loop(std::true_type{});
+  else loop(std::false_type{});
+  store_tile<T, TQ, TQ>(p, C, m0 + wm * (BM / 2), n0 + wn * (BM / 2), lane, acc);
 }
 
 static int g_force_tile = 0;
@@ -293,6 +504,46 @@ static void launch_shape(hipStream_t s, bool ta, bool tb, GemmParams<T>& p, int 
   XK_HIP(hipGetLastError());
 }
 
+template <typename T, int BM, int NST>
+static void launch_dma(hipStream_t s, bool ta, bool tb, GemmParams<T>& p, int batch)
+{
+  p.tiles_m = (p.m + BM - 1) / BM;
+  p.tiles_n = (p.n + BM - 1) / BM;
+  const long ntiles = (p.tri == TRI_FULL || p.trap) ? (long)p.tiles_m * p.tiles_n
+                                                    : (long)p.tiles_m * (p.tiles_m + 1) / 2;
+  XK_CHECK(ntiles < (1L << 31), "gemm grid too large");
+  dim3 grid((unsigned)ntiles, 1, (unsigned)batch), block(256);
+  if (!ta && !tb) hipLaunchKernelGGL((gemm_dma_kernel<T, BM, NST, false, false>), grid, block, 0, s, p);
+  else if (!ta && tb) hipLaunchKernelGGL((gemm_dma_kernel<T, BM, NST, false, true>), grid, block, 0, s, p);
+  else if (ta && !tb) hipLaunchKernelGGL((gemm_dma_kernel<T, BM, NST, true, false>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((gemm_dma_kernel<T, BM, NST, true, true>), grid, block, 0, s, p);
+  XK_HIP(hipGetLastError());
+}
+
+// Tile of gemm_dma_kernel for t128 / t64 tiles of 128 / 64 of inner dimension
+// k.  Rates with the chip full: FP64 70-71 TFLOP/s with 128 x 128 tiles (two
+// workgroups per CU), 66 with 64 x 64 (five per CU); FP32 136 and 122.  A last
+// round that fills at most half of its places takes about 0.65 of a round
+// with 128 (one workgroup per CU runs faster alone), one of a part f 0.5 +
+// 0.5 f with 64; filling the ring and storing cost as much as 120 and 57 of
+// k.  Measured, 128 / 64: FP64 4096^3 62.4 / 59.3, 2048^3 53.9 / 55.5, 1536^3
+// 31.8 / 42.0, 2500^2 x 512 43.1 / 46.5; FP32 4096^3 118 / 105, 3000^3 86 / 98.
+// 32 x 32 when 64 x 64 leaves CUs with one workgroup or none: FP64 512^3 17.3
+// against 9.2, 1024^3 39.3 / 38, 1536^3 42.5 / 42; FP32 512^3 23.3 / 14.2, 1024^3
+// 64.4 / 64.9.  (With registers between memory and LDS, tiles as now: 8192^3
+// 58.5, 4096^3 51.6, 1024^3 31.4, 512^3 12.8; FP32 133, 111, 47.7, 11.0.)
+template <typename T>
+static int dma_tile(long t128, long t64, int k)
+{
+  if (t64 < (sizeof(T) == 8 ? 512 : 256)) return 32;
+  const double r128 = t128 / 512.0, r64 = t64 / 1280.0;
+  const double w128 = std::floor(r128), w64 = std::floor(r64);
+  const double f128 = r128 - w128, f64 = r64 - w64;
+  const double c128 = (w128 + (f128 == 0 ? 0 : f128 <= 0.5 ? 0.65 : 1.0)) * 512 * 128 * 128 * (k + 120.0);
+  const double c64 = (w64 + (f64 == 0 ? 0 : 0.5 + 0.5 * f64)) * 1280 * 64 * 64 * (k + 57.0);
+  return c128 / (sizeof(T) == 8 ? 70.5 : 136.0) < c64 / (sizeof(T) == 8 ? 66.0 : 122.0) ? 128 : 64;
+}
+
 template <typename T>
 void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, const T* A, long lda,
           const T* B, long ldb, T beta, T* C, long ldc, int tri, int batch, long sA, long sB, long sC, int kmode)
@@ -314,26 +565,35 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, c
   p.vecA = aligned(A, lda, sA);
   p.vecB = aligned(B, ldb, sB);
   const bool ta = transA != NoTrans, tb = transB != NoTrans;
+  auto tiles = [&](int t) {
+    const long a = (m + t - 1) / t, b = (n + t - 1) / t;
+    return (p.tri != TRI_FULL && !p.trap ? a * (a + 1) / 2 : a * b) * batch;
+  };
   int bm = g_force_tile;
-  if (bm == 0) {
-    // FP64: 64 x 64 tiles at every size (measured on MI355X: 55.8 vs 47.1
-    // TFLOP/s at 16384^3, more resident waves per CU); FP32: 128 x 128 once
-    // there are enough tiles to fill the chip
-    long t128 = (long)((m + 127) / 128) * ((n + 127) / 128) * batch;
-    bm = (sizeof(T) == 8 || m <= 64 || n <= 64 || t128 < 160) ? 64 : 128;
-    // FP64 products too small to give every CU two 64 x 64 tiles (the
-    // latency-bound steps of TRSM sweeps and diagonal-block chains): 32 x 32
-    // tiles, four times the workgroups; the k order per element, hence the
-    // result, is the same
-    long t64 = (long)((m + 63) / 64) * ((n + 63) / 64);
-    if (p.tri != TRI_FULL && !p.trap) t64 = t64 / 2 + (m + 63) / 64;
-    if (sizeof(T) == 8 && t64 * batch < 512) bm = 32;
+  // 32-bit offsets inside a tile
+  const bool dma = p.vecA && p.vecB && lda < (1L << 21) && ldb < (1L << 21);
+  if (dma) {
+    if (bm == 0) bm = dma_tile<T>(tiles(128), tiles(64), k);
+    if (bm == 128) launch_dma<T, 128, 2>(s, ta, tb, p, batch);
+    else if (bm == 32) launch_dma<T, 32, 4>(s, ta, tb, p, batch);
+    else launch_dma<T, 64, 2>(s, ta, tb, p, batch);
+    return;
   }
-  if (bm == 128) launch_shape<T, 128, 16>(s, ta, tb, p, batch);
-  else if (bm == 32) {
-    if constexpr (sizeof(T) == 8) launch_shape<T, 32, 16>(s, ta, tb, p, batch);
+  // operands at odd offsets (row panels of an odd tile size): the tiles of
+  // the register-staged kernel by the same reasons, FP64 55.8 against 47.1
+  // TFLOP/s with 64 and 128 (more resident waves per CU), FP32 128 once they
+  // fill the chip
+  if (bm == 0) {
+    bm = sizeof(T) == 8 || tiles(128) < 160 ? 64 : 128;
+    if (sizeof(T) == 8 && tiles(64) < 512) bm = 32;
+  }
+  if constexpr (sizeof(T) == 8) {
+    if (bm == 32) launch_shape<T, 32, 16>(s, ta, tb, p, batch);
     else launch_shape<T, 64, 16>(s, ta, tb, p, batch);
-  } else launch_shape<T, 64, 16>(s, ta, tb, p, batch);
+  } else {
+    if (bm == 128) launch_shape<T, 128, 16>(s, ta, tb, p, batch);
+    else launch_shape<T, 64, 16>(s, ta, tb, p, batch);
+  }
 }
 
 template void gemm<double>(hipStream_t, int, int, int, int, int, double, const double*, long, const double*, long,

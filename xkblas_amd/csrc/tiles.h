@@ -4,6 +4,14 @@
 
 namespace xk {
 
+// Workgroup ids are dealt round-robin to the 8 XCDs: the id within a
+// contiguous range for each XCD, for any total.
+__device__ __forceinline__ int xcd_range(int pid, int total)
+{
+  const int x = pid & 7, q = total >> 3, r = total & 7;
+  return x * q + min(x, r) + (pid >> 3);
+}
+
 // Lower triangle of T x T tiles (i >= j), total = T (T + 1) / 2 workgroups.
 // Workgroup ids are dealt round-robin to the 8 XCDs: the id is remapped so
 // that each XCD gets a contiguous range, and the range is walked in groups of
@@ -13,7 +21,7 @@ namespace xk {
 template <int GM>
 __device__ __forceinline__ void tri_tile(int pid, int total, int T, int& i, int& j)
 {
-  if ((total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);
+  pid = xcd_range(pid, total);
   auto before = [](int h) { return (GM * GM * h * (h - 1)) / 2 + h * (GM * (GM + 1)) / 2; };
   // before(g) = a g^2 + b g: first guess from the quadratic, then exact
   const float a = 0.5f * GM * GM, b = 0.5f * GM * (GM + 1) - a;

@@ -70,11 +70,13 @@ static double tune_run(int op, int mode, int ta, int tb, int m, int n, int k, in
   Exec x = r.exec();
   x.mode = mode;
   hipStream_t s = x.s;
-  const long lda = std::max(op == 0 ? (ta == NoTrans ? m : k) : (op == 1 ? n : m), 1);
+  // columns as the tile cache keeps them: 256-byte aligned
+  auto padded = [](int rows) { return (std::max(rows, 1) * (long)sizeof(T) + 255) / 256 * 256 / (long)sizeof(T); };
+  const long lda = padded(op == 0 ? (ta == NoTrans ? m : k) : (op == 1 ? n : m));
   const long acols = op == 0 ? (ta == NoTrans ? k : m) : (op == 1 ? k : m);
-  const long ldb = std::max(op == 0 ? (tb == NoTrans ? k : n) : m, 1);
+  const long ldb = padded(op == 0 ? (tb == NoTrans ? k : n) : m);
   const long bcols = op == 0 ? (tb == NoTrans ? n : k) : n;
-  const long ldc = std::max(op == 1 ? n : m, 1);
+  const long ldc = padded(op == 1 ? n : m);
   const long ccols = n;
   T* A = (T*)arena(0, sizeof(T) * lda * std::max(acols, 1L));
   T* B = (T*)arena(1, sizeof(T) * ldb * std::max(bcols, 1L));
@@ -128,7 +130,7 @@ extern "C" {
 // inner k), 2 TRSM (Left, Lower, NoTrans, Non-unit, B m x n, block order nb),
 // 3 POTRF (lower, order m, block order nb).  dtype 0 FP64, 1 FP32; mode is
 // the math mode (split modes apply to FP64).  tile: GEMM macro tile (0 auto,
-// 32 (FP64; FP32 runs 64), 64, 128); split_count: 0 auto; split_kernel: 0 / 1.  Returns the best of
+// 32, 64, 128); split_count: 0 auto; split_kernel: 0 / 1.  Returns the best of
 // `iters` kernel times in ms, or a negative value on bad arguments.
 double xkblas_tune_time(int op, int dtype, int mode, int transA, int transB, int m, int n, int k, int tile, int nb,
                         int split_count, int split_kernel, int iters)

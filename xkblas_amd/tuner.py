@@ -56,7 +56,7 @@ def candidates(op, dtype, mode, m, n, k):
         if mode in SPLIT_MODES and dtype == 0:
             kernels = (0, 1) if mode == 2 else (0,)
             return [{"tile": 0, "nb": 0, "split": c, "kernel": kv} for c in split_counts(mode, k) for kv in kernels]
-        tiles = (32, 64, 128) if dtype == 0 else (64, 128)
+        tiles = (0, 32, 64, 128)  # 0: the library's own choice
         return [{"tile": t, "nb": 0, "split": 0, "kernel": 0} for t in tiles]
     dim = m
     nbs = [b for b in (64, 128, 256, 512, 1024, 2048, 4096) if b <= max(64, dim) and (b < 4096 or dim >= 16384)]
