@@ -71,3 +71,38 @@ def test_tiles_give_the_same_bits(xk, ta, tb, dtype):
     xk.lib().xkblas_set_param(0, 0)
     for C in out[1:]:
         assert np.array_equal(out[0], C)
+
+
+@pytest.mark.parametrize("ta,tb", OPS)
+def test_last_round_in_quarters(xk, ta, tb):
+    """A little more than one round of 128 x 128 tiles: whole tiles and
+    quarters together give what 64 x 64 tiles give, bit for bit."""
+    r = rng(4)
+    M, N, K = 2950, 2930, 2001
+    A = uniform(r, *((M, K) if ta == 111 else (K, M)), dtype=np.float32)
+    B = uniform(r, *((K, N) if tb == 111 else (N, K)), dtype=np.float32)
+    out = []
+    for t in (0, 64):
+        xk.lib().xkblas_set_gemm_tile(t)
+        C = np.zeros((M, N), dtype=np.float32, order="F")
+        xk.gemm(ta, tb, 1.0, A, B, 0.0, C)
+        xk.invalidate()
+        out.append(C)
+    xk.lib().xkblas_set_gemm_tile(0)
+    assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("uplo", [121, 122])
+def test_last_round_of_a_triangle_in_quarters(xk, uplo):
+    A = uniform(rng(6), 4070, 2001, dtype=np.float32)
+    out = []
+    for t in (0, 64):
+        xk.lib().xkblas_set_gemm_tile(t)
+        C = np.full((4070, 4070), 7, dtype=np.float32, order="F")
+        xk.syrk(uplo, 111, 1.0, A, 0.5, C)
+        xk.invalidate()
+        out.append(C)
+    xk.lib().xkblas_set_gemm_tile(0)
+    assert np.array_equal(out[0], out[1])
+    assert np.all((np.triu(out[0], 1) if uplo == 122 else np.tril(out[0], -1))[np.triu_indices(4070, 1) if uplo == 122
+                  else np.tril_indices(4070, -1)] == 7)

@@ -23,6 +23,7 @@
 // rastered in groups of 8 tile rows so that concurrently running tiles of one
 // XCD share op(A) panels in its L2.
 #include "common.h"
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include "tiles.h"
@@ -52,6 +53,7 @@ struct GemmParams {
   int tiles_m, tiles_n;
   int tri;
   int trap;        // triangle-masked output that is not square: full tile raster, tiles outside it leave at once
+  int whole;       // tiles of gemm_dma_mixed_kernel's first part
   int kmode;       // inner range per tile for a triangular operand (KRANGE_*)
   int vecA, vecB;  // 16-byte vector loads allowed (base and ld aligned)
   int prio;        // raise the waves' issue priority (latency-bound chain steps)
@@ -88,38 +90,53 @@ __device__ __forceinline__ void load_run(const T* p, T (&r)[V])
   }
 }
 
+// Tile (tm, tn) at place `at` of the raster: groups of 8 tile rows, column by
+// column inside a group; a square triangle's tiles only.
+template <typename T>
+__device__ __forceinline__ void tile_raster(const GemmParams<T>& p, int at, int& tm, int& tn)
+{
+  if (p.tri == TRI_FULL || p.trap) {
+    constexpr int GM = 8;
+    const int group = GM * p.tiles_n;
+    const int g = at / group;
+    const int first = g * GM;
+    const int gm = min(p.tiles_m - first, GM);
+    const int r = at - g * group;
+    tm = first + r % gm;
+    tn = r / gm;
+  } else {
+    int i, j;
+    tri_raster<8>(at, p.tiles_m, i, j);
+    if (p.tri == TRI_LOWER) { tm = i; tn = j; }
+    else { tm = j; tn = i; }
+  }
+}
+
+// Whether a BM x BN tile at (m0, n0) holds anything to write.
+template <int BM, int BN, typename T>
+__device__ __forceinline__ bool tile_holds(const GemmParams<T>& p, int m0, int n0)
+{
+  if (m0 >= p.m || n0 >= p.n) return false;
+  return p.tri == TRI_FULL || (p.tri == TRI_LOWER ? m0 + BM > n0 : n0 + BN > m0);
+}
+
 // First row and column of this workgroup's BM x BN tile; false when there is
 // nothing of it to write.
 template <int BM, int BN, typename T>
 __device__ __forceinline__ bool tile_origin(const GemmParams<T>& p, int& m0, int& n0)
 {
-  int pid = blockIdx.x, tm, tn;
-  const int total = gridDim.x;
-  if (p.tri == TRI_FULL || p.trap) {
-    // a limited inner range makes the work per tile grow along the tile
-    // rows or columns: no XCD blocking then (consecutive ids go to
-    // different XCDs, which then share light and heavy tiles alike), and
-    // the heaviest tiles are dispatched first
-    if (p.kmode == KRANGE_ALL) pid = xcd_range(pid, total);
-    constexpr int GM = 8;
-    const int group = GM * p.tiles_n;
-    const int g = pid / group;
-    const int first = g * GM;
-    const int gm = min(p.tiles_m - first, GM);
-    const int r = pid - g * group;
-    tm = first + r % gm;
-    tn = r / gm;
-    if (p.kmode == KRANGE_A_LOWER) tm = p.tiles_m - 1 - tm;
-    else if (p.kmode == KRANGE_B_UPPER) tn = p.tiles_n - 1 - tn;
-  } else {
-    int i, j;
-    tri_tile<8>(pid, total, p.tiles_m, i, j);
-    if (p.tri == TRI_LOWER) { tm = i; tn = j; }
-    else { tm = j; tn = i; }
-  }
+  int at = blockIdx.x, tm, tn;
+  // a limited inner range makes the work per tile grow along the tile rows or
+  // columns: no XCD blocking then (consecutive ids go to different XCDs, which
+  // then share light and heavy tiles alike), and the heaviest tiles are
+  // dispatched first
+  if (p.kmode == KRANGE_ALL) at = xcd_range(at, gridDim.x);
+  tile_raster(p, at, tm, tn);
+  if (p.kmode == KRANGE_A_LOWER) tm = p.tiles_m - 1 - tm;
+  else if (p.kmode == KRANGE_B_UPPER) tn = p.tiles_n - 1 - tn;
   m0 = tm * BM;
   n0 = tn * BN;
-  return !(p.trap && (p.tri == TRI_LOWER ? m0 + BM <= n0 : n0 + BN <= m0));
+  return tile_holds<BM, BN>(p, m0, n0);
 }
 
 // C = alpha acc + beta C on the selected triangle: the wave's TM x TN blocks
@@ -312,7 +329,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams<T> p)
 // that hold results.
 // The inner order per element is gemm_kernel's: the same bits.
 template <typename T, int BM, int NST, bool TA, bool TB>
-__global__ __launch_bounds__(256, 2) void gemm_dma_kernel(GemmParams<T> p)
+__device__ __forceinline__ void dma_tile_body(const GemmParams<T>& p, char* S, int m0, int n0)
 {
   constexpr int SZ = sizeof(T), E = 16 / SZ, BK = 128 / SZ;
   constexpr int OP = BM * 128;      // bytes of one operand's stage
@@ -320,7 +337,6 @@ __global__ __launch_bounds__(256, 2) void gemm_dma_kernel(GemmParams<T> p)
   constexpr int Q = BM / 32;        // load instructions per wave, operand and stage
   constexpr int TQ = BM / 32;       // 16 x 16 blocks of a wave's quarter, each way
   typedef typename AccT<T>::type acc_t;
-  __shared__ __attribute__((aligned(1024))) char S[NST * 2 * OP];
   if (p.prio) __builtin_amdgcn_s_setprio(3);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -329,8 +345,6 @@ __global__ __launch_bounds__(256, 2) void gemm_dma_kernel(GemmParams<T> p)
   const T* __restrict__ B = p.B + (long)blockIdx.z * p.sB;
   T* __restrict__ C = p.C + (long)blockIdx.z * p.sC;
   const int M = p.m, N = p.n, K = p.k;
-  int m0, n0;
-  if (!tile_origin<BM, BM>(p, m0, n0)) return;
 
   // block permutation of k-major row k: rows that the lanes of one read take
   // together (k .. k + 3) fall into different banks
@@ -478,6 +492,35 @@ __global__ __launch_bounds__(256, 2) void gemm_dma_kernel(GemmParams<T> p)
   store_tile<T, TQ, TQ>(p, C, m0 + wm * (BM / 2), n0 + wn * (BM / 2), lane, acc);
 }
 
+template <typename T, int BM, int NST, bool TA, bool TB>
+__global__ __launch_bounds__(256, 2) void gemm_dma_kernel(GemmParams<T> p)
+{
+  __shared__ __attribute__((aligned(1024))) char S[NST * 2 * BM * 128];
+  int m0, n0;
+  if (tile_origin<BM, BM>(p, m0, n0)) dma_tile_body<T, BM, NST, TA, TB>(p, S, m0, n0);
+}
+
+// 128 x 128 tiles for the first p.whole places of the raster (whole rounds
+// over the chip), then the rest as quarters of 64 x 64 with a ring of four
+// stages in the same LDS: the last round takes about its share of the work
+// instead of a tile's whole time.
+template <typename T, bool TA, bool TB>
+__global__ __launch_bounds__(256, 2) void gemm_dma_mixed_kernel(GemmParams<T> p)
+{
+  __shared__ __attribute__((aligned(1024))) char S[2 * 2 * 128 * 128];
+  const int pid = blockIdx.x;
+  int tm, tn;
+  if (pid < p.whole) {
+    tile_raster(p, xcd_range(pid, p.whole), tm, tn);
+    if (tile_holds<128, 128>(p, tm * 128, tn * 128)) dma_tile_body<T, 128, 2, TA, TB>(p, S, tm * 128, tn * 128);
+  } else {
+    const int at = xcd_range(pid - p.whole, gridDim.x - p.whole);
+    tile_raster(p, p.whole + (at >> 2), tm, tn);
+    const int m0 = tm * 128 + (at & 1) * 64, n0 = tn * 128 + (at & 2) * 32;
+    if (tile_holds<64, 64>(p, m0, n0)) dma_tile_body<T, 64, 4, TA, TB>(p, S, m0, n0);
+  }
+}
+
 static int g_force_tile = 0;
 void gemm_set_tile(int bm) { g_force_tile = bm; }
 
@@ -520,28 +563,55 @@ static void launch_dma(hipStream_t s, bool ta, bool tb, GemmParams<T>& p, int ba
   XK_HIP(hipGetLastError());
 }
 
+template <typename T>
+static void launch_mixed(hipStream_t s, bool ta, bool tb, GemmParams<T>& p, int whole, long tiles)
+{
+  p.tiles_m = (p.m + 127) / 128;
+  p.tiles_n = (p.n + 127) / 128;
+  p.whole = whole;
+  XK_CHECK(4 * tiles < (1L << 31), "gemm grid too large");
+  dim3 grid((unsigned)(whole + 4 * (tiles - whole))), block(256);
+  if (!ta && !tb) hipLaunchKernelGGL((gemm_dma_mixed_kernel<T, false, false>), grid, block, 0, s, p);
+  else if (!ta && tb) hipLaunchKernelGGL((gemm_dma_mixed_kernel<T, false, true>), grid, block, 0, s, p);
+  else if (ta && !tb) hipLaunchKernelGGL((gemm_dma_mixed_kernel<T, true, false>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((gemm_dma_mixed_kernel<T, true, true>), grid, block, 0, s, p);
+  XK_HIP(hipGetLastError());
+}
+
 // Tile of gemm_dma_kernel for t128 / t64 tiles of 128 / 64 of inner dimension
-// k.  Rates with the chip full: FP64 70-71 TFLOP/s with 128 x 128 tiles (two
-// workgroups per CU), 66 with 64 x 64 (five per CU); FP32 136 and 122.  A last
-// round that fills at most half of its places takes about 0.65 of a round
-// with 128 (one workgroup per CU runs faster alone), one of a part f 0.5 +
-// 0.5 f with 64; filling the ring and storing cost as much as 120 and 57 of
-// k.  Measured, 128 / 64: FP64 4096^3 62.4 / 59.3, 2048^3 53.9 / 55.5, 1536^3
-// 31.8 / 42.0, 2500^2 x 512 43.1 / 46.5; FP32 4096^3 118 / 105, 3000^3 86 / 98.
+// k; mixed: the last round of 128 x 128 tiles goes in quarters.  Rates with the
+// chip full: FP64 70-71 TFLOP/s with 128 x 128 tiles (two workgroups per CU),
+// 66 with 64 x 64 (five per CU); FP32 136 and 120.  A last round that fills a
+// part f of its places takes about 0.6 + 0.95 f of a round with 128 (up to
+// 1.12; a workgroup alone on its CU runs faster, but two of the last ones may
+// share one) and 0.1 + 1.2 f in quarters, an only round 0.62 up to half of the
+// places; with 64 0.5 + 0.5 f.  Filling the ring and storing cost as much as
+// 150 and 57 of k.  Measured, 128 / 64: FP64 4096^3 62.4 / 59.3, 2048^3 53.9 /
+// 55.5, 1536^3 31.8 / 42.0, 2500^2 x 512 43.1 / 46.5, 12000 x 1000 x 3000 47.7 /
+// 59.0; mixed / 128 / 64: FP64 triangle 8192^2 x 16384 67.4 / 60.8 / 64, FP32
+// 131.6 / 120.5 / 114, 4096 x 4100 x 8192 126 / 107 / 110, 3000^3 119 / 91 / 107.
 // 32 x 32 when 64 x 64 leaves CUs with one workgroup or none: FP64 512^3 17.3
 // against 9.2, 1024^3 39.3 / 38, 1536^3 42.5 / 42; FP32 512^3 23.3 / 14.2, 1024^3
 // 64.4 / 64.9.  (With registers between memory and LDS, tiles as now: 8192^3
 // 58.5, 4096^3 51.6, 1024^3 31.4, 512^3 12.8; FP32 133, 111, 47.7, 11.0.)
 template <typename T>
-static int dma_tile(long t128, long t64, int k)
+static int dma_tile(long t128, long t64, int k, bool may_mix, bool& mixed)
 {
+  mixed = false;
   if (t64 < (sizeof(T) == 8 ? 512 : 256)) return 32;
   const double r128 = t128 / 512.0, r64 = t64 / 1280.0;
   const double w128 = std::floor(r128), w64 = std::floor(r64);
   const double f128 = r128 - w128, f64 = r64 - w64;
-  const double c128 = (w128 + (f128 == 0 ? 0 : f128 <= 0.5 ? 0.65 : 1.0)) * 512 * 128 * 128 * (k + 120.0);
+  double last = 0;
+  if (w128 == 0) last = f128 <= 0.5 ? 0.62 : 1.06;
+  else if (f128 > 0) {
+    const double plain = std::min(1.12, 0.6 + 0.95 * f128), quarters = 0.1 + 1.2 * f128;
+    mixed = may_mix && quarters < plain;
+    last = mixed ? quarters : plain;
+  }
+  const double c128 = (w128 + last) * 512 * 128 * 128 * (k + 150.0);
   const double c64 = (w64 + (f64 == 0 ? 0 : 0.5 + 0.5 * f64)) * 1280 * 64 * 64 * (k + 57.0);
-  return c128 / (sizeof(T) == 8 ? 70.5 : 136.0) < c64 / (sizeof(T) == 8 ? 66.0 : 122.0) ? 128 : 64;
+  return c128 / (sizeof(T) == 8 ? 70.5 : 136.0) < c64 / (sizeof(T) == 8 ? 66.0 : 120.0) ? 128 : 64;
 }
 
 template <typename T>
@@ -573,7 +643,12 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, c
   // 32-bit offsets inside a tile
   const bool dma = p.vecA && p.vecB && lda < (1L << 21) && ldb < (1L << 21);
   if (dma) {
-    if (bm == 0) bm = dma_tile<T>(tiles(128), tiles(64), k);
+    bool mixed = false;
+    if (bm == 0) bm = dma_tile<T>(tiles(128), tiles(64), k, batch == 1 && kmode == KRANGE_ALL, mixed);
+    if (bm == 128 && mixed) {
+      launch_mixed<T>(s, ta, tb, p, (int)(tiles(128) / 512 * 512), tiles(128));
+      return;
+    }
     if (bm == 128) launch_dma<T, 128, 2>(s, ta, tb, p, batch);
     else if (bm == 32) launch_dma<T, 32, 4>(s, ta, tb, p, batch);
     else launch_dma<T, 64, 2>(s, ta, tb, p, batch);

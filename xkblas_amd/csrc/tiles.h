@@ -18,10 +18,10 @@ __device__ __forceinline__ int xcd_range(int pid, int total)
 // GM tile rows, column by column inside a group, so the workgroups of one XCD
 // that run together share the row panels of their group and a few column
 // panels in its L2.  Group g (full) holds GM (g GM) + GM (GM + 1) / 2 tiles.
+// tri_raster takes the place in that range, tri_tile the workgroup id.
 template <int GM>
-__device__ __forceinline__ void tri_tile(int pid, int total, int T, int& i, int& j)
+__device__ __forceinline__ void tri_raster(int pid, int T, int& i, int& j)
 {
-  pid = xcd_range(pid, total);
   auto before = [](int h) { return (GM * GM * h * (h - 1)) / 2 + h * (GM * (GM + 1)) / 2; };
   // before(g) = a g^2 + b g: first guess from the quadratic, then exact
   const float a = 0.5f * GM * GM, b = 0.5f * GM * (GM + 1) - a;
@@ -43,6 +43,12 @@ __device__ __forceinline__ void tri_tile(int pid, int total, int T, int& i, int&
   }
   j = r0 + jj;
   i = r0 + jj + rr;
+}
+
+template <int GM>
+__device__ __forceinline__ void tri_tile(int pid, int total, int T, int& i, int& j)
+{
+  tri_raster<GM>(xcd_range(pid, total), T, i, j);
 }
 
 }  // namespace xk
