@@ -75,3 +75,43 @@ def test_pipelined_then_resident_reuse(xk):
     assert np.array_equal(top, C[:300])
     assert np.array_equal(C, Cs)
     np.testing.assert_allclose(C, A @ B, rtol=0, atol=1e-12)
+
+
+@pytest.mark.parametrize("ta,tb", [(N_, N_), (T_, N_), (N_, T_), (T_, T_)])
+@pytest.mark.parametrize("mode,dtype", [(0, np.float64), (0, np.float32), (2, np.float64)])
+def test_resident_product_in_panels_equals_one_launch(xk, ta, tb, mode, dtype):
+    """A large result of resident operands is computed in column panels so
+    that its copy back runs beside the product: the same bits as one launch,
+    for a whole copy back, a part of it first, and a second product that
+    follows before the copy back (which then reads and waits correctly)."""
+    M, N, K = 2000, 2900 if dtype == np.float32 else 1900, 600
+    r = rng(5 + ta + 2 * tb + mode)
+    A = uniform(r, *((M, K) if ta == N_ else (K, M)), dtype=dtype)
+    B = uniform(r, *((K, N) if tb == N_ else (N, K)), dtype=dtype)
+    L = xk.lib()
+    xk.invalidate()
+    L.xkblas_set_param(700, 0)
+    L.xkblas_set_modemath(mode)
+    out = []
+    try:
+        for pipeline in (0, 1):
+            L.xkblas_set_pipeline(pipeline)
+            C, D = np.zeros((M, N), dtype, order="F"), np.zeros((M, 40), dtype, order="F")
+            E = uniform(rng(9), N, 40, dtype=dtype)
+            for beta in (0.0, -0.5):
+                xk.gemm(ta, tb, 1.5, A, B, beta, C, sync=False)
+            xk.gemm(N_, N_, 1.0, C, E, 0.0, D, sync=False)
+            L.xkblas_memory_coherent_async(0, 0, 300, 1000, C.ctypes.data, M, C.itemsize)
+            L.xkblas_sync()
+            top = C[:300, :1000].copy()
+            xk.coherent(C)
+            xk.coherent(D)
+            xk.gemm(ta, tb, 1.0, A, B, 0.0, C)  # all operands resident, copied back at once
+            out.append((top, D, C))
+            xk.invalidate()
+    finally:
+        L.xkblas_set_pipeline(1)
+        L.xkblas_set_modemath(0)
+        L.xkblas_set_param(0, 0)
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)

@@ -615,6 +615,16 @@ static int dma_tile(long t128, long t64, int k, bool may_mix, bool& mixed)
 }
 
 template <typename T>
+int gemm_tile_of(int m, int n, int k)
+{
+  auto tiles = [&](int t) { return (long)((m + t - 1) / t) * ((n + t - 1) / t); };
+  bool mixed;
+  return dma_tile<T>(tiles(128), tiles(64), k, true, mixed);
+}
+template int gemm_tile_of<double>(int, int, int);
+template int gemm_tile_of<float>(int, int, int);
+
+template <typename T>
 void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, const T* A, long lda,
           const T* B, long ldb, T beta, T* C, long ldc, int tri, int batch, long sA, long sB, long sC, int kmode)
 {

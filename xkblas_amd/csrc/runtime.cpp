@@ -227,7 +227,26 @@ void Runtime::drop(Replica* r)
   }
   cache_used -= r->bytes;
   if (r->info_slot >= 0) free_info.push_back(r->info_slot);
+  release(r);
+}
+
+void Runtime::release(Replica* r)
+{
+  unstamped.erase(std::remove(unstamped.begin(), unstamped.end(), r), unstamped.end());
+  if (r->written) XK_HIP(hipEventDestroy(r->written));
   delete r;
+}
+
+// An event behind the mirrors written by the last call, before other work
+// follows on the compute stream: their copies back wait for it alone.
+void Runtime::stamp_written()
+{
+  for (Replica* r : unstamped) {
+    if (!r->written) XK_HIP(hipEventCreateWithFlags(&r->written, hipEventDisableTiming));
+    XK_HIP(hipEventRecord(r->written, s_comp));
+    r->stamped = true;
+  }
+  unstamped.clear();
 }
 
 // Retired mirrors, at a public synchronisation point (no call is running and
@@ -244,7 +263,7 @@ void Runtime::free_retired()
     if (r->dev) XK_HIP(hipFree(r->dev));
     cache_used -= r->bytes;
     if (r->info_slot >= 0) free_info.push_back(r->info_slot);
-    delete r;
+    release(r);
   }
   retired.clear();
 }
@@ -361,6 +380,7 @@ void Runtime::clear_panels(Replica* r)
 {
   for (auto& pe : r->panels) XK_HIP(hipEventDestroy(pe.ev));  // released once complete
   r->panels.clear();
+  r->panel_cols = false;
 }
 
 // Mark tiles as written on the device (host copy stale).  Any later write
@@ -369,6 +389,8 @@ void Runtime::mark_written(Replica* r, int r0, int c0, int m, int n, int uplo)
 {
   if (m <= 0 || n <= 0) return;
   clear_panels(r);
+  if (r->stamped || std::find(unstamped.begin(), unstamped.end(), r) == unstamped.end()) unstamped.push_back(r);
+  r->stamped = false;
   const int ti0 = r0 / r->nb, ti1 = (r0 + m - 1) / r->nb;
   const int tj0 = c0 / r->nb, tj1 = (c0 + n - 1) / r->nb;
   for (int tj = tj0; tj <= tj1; ++tj)
@@ -384,37 +406,48 @@ void Runtime::mark_written(Replica* r, int r0, int c0, int m, int n, int uplo)
 void Runtime::writeback(Replica* r, int r0, int c0, int m, int n, int uplo)
 {
   if (m <= 0 || n <= 0) return;
-  if (!r->panels.empty()) {
-    // a product pipelined by row panels: each panel's rows go back once
-    // that panel is computed, under the computation of the next ones
-    int lo = 0;
-    const std::vector<Replica::PanelEvent> pv = r->panels;
-    for (const auto& pe : pv) {
-      const int a = std::max(lo, r0), b = std::min(pe.end, r0 + m);
-      if (a < b) {
-        XK_HIP(hipStreamWaitEvent(s_d2h, pe.ev, 0));
-        writeback_rows(r, a, c0, b - a, n, uplo);
-      }
-      lo = pe.end;
-    }
-    if (lo < r0 + m) {
+  const int nb = r->nb;
+  // whole tiles
+  const int lo = r0 / nb * nb, hi = std::min(r->M, (r0 + m + nb - 1) / nb * nb);
+  const int clo = c0 / nb * nb, chi = std::min(r->N, (c0 + n + nb - 1) / nb * nb);
+  bool any = false;
+  auto copy = [&](int a, int b) {  // rows or columns [a, b)
+    any |= r->panel_cols ? copy_back(r, lo, hi, a, b, uplo) : copy_back(r, a, b, clo, chi, uplo);
+  };
+  int done = r->panel_cols ? clo : lo;
+  const int end = r->panel_cols ? chi : hi;
+  // a product in panels: each panel goes back once it is computed, under the
+  // computation of the next ones
+  for (const auto& pe : r->panels) {
+    const int b = std::min(pe.end, end);
+    if (done >= b) continue;
+    XK_HIP(hipStreamWaitEvent(s_d2h, pe.ev, 0));
+    copy(done, b);
+    done = b;
+  }
+  if (done < end) {
+    if (r->stamped) {
+      XK_HIP(hipStreamWaitEvent(s_d2h, r->written, 0));
+    } else {
       XK_HIP(hipEventRecord(ev_comp, s_comp));
       XK_HIP(hipStreamWaitEvent(s_d2h, ev_comp, 0));
-      writeback_rows(r, std::max(lo, r0), c0, r0 + m - std::max(lo, r0), n, uplo);
     }
-    return;
+    copy(done, end);
   }
-  XK_HIP(hipEventRecord(ev_comp, s_comp));
-  XK_HIP(hipStreamWaitEvent(s_d2h, ev_comp, 0));
-  writeback_rows(r, r0, c0, m, n, uplo);
+  if (!any) return;
+  for (int tj = clo / nb; tj < (chi + nb - 1) / nb; ++tj)
+    for (int ti = lo / nb; ti < (hi + nb - 1) / nb; ++ti)
+      if (!(uplo == Lower && ti < tj) && !(uplo == Upper && ti > tj)) r->state[tj * r->mt + ti] |= HOST_VALID;
+  XK_HIP(hipEventRecord(ev_d2h, s_d2h));
+  pending_d2h = true;
 }
 
-// The D2H copies of writeback (the stream's ordering is set by the caller).
-void Runtime::writeback_rows(Replica* r, int r0, int c0, int m, int n, int uplo)
+// The D2H copies of writeback for rows [row_lo, row_hi) and columns [col_lo,
+// col_hi) (the stream's ordering is set by the caller); whether there were any.
+bool Runtime::copy_back(Replica* r, int row_lo, int row_hi, int col_lo, int col_hi, int uplo)
 {
-  if (m <= 0 || n <= 0) return;
-  const int ti0 = r0 / r->nb, ti1 = (r0 + m - 1) / r->nb;
-  const int tj0 = c0 / r->nb, tj1 = (c0 + n - 1) / r->nb;
+  const int ti0 = row_lo / r->nb, ti1 = (row_hi - 1) / r->nb;
+  const int tj0 = col_lo / r->nb, tj1 = (col_hi - 1) / r->nb;
   bool any = false;
   for (int tj = tj0; tj <= tj1; ++tj) {
     int ti = ti0;
@@ -427,21 +460,17 @@ void Runtime::writeback_rows(Replica* r, int r0, int c0, int m, int n, int uplo)
       if (!wanted(ti)) { ++ti; continue; }
       int te = ti;
       while (te + 1 <= ti1 && wanted(te + 1)) ++te;
-      const int row0 = ti * r->nb, row1 = std::min(r->M, (te + 1) * r->nb);
-      const int col0 = tj * r->nb, col1 = std::min(r->N, (tj + 1) * r->nb);
+      const int row0 = std::max(row_lo, ti * r->nb), row1 = std::min(row_hi, (te + 1) * r->nb);
+      const int col0 = std::max(col_lo, tj * r->nb), col1 = std::min(col_hi, (tj + 1) * r->nb);
       char* dst = (char*)r->host + ((size_t)row0 + (size_t)col0 * r->ld) * r->elt;
       const char* src = r->dev + ((size_t)row0 + (size_t)col0 * r->ldd) * r->elt;
       copy_d2h(dst, r->ld * r->elt, src, r->ldd * r->elt, (size_t)(row1 - row0) * r->elt, (size_t)(col1 - col0));
       stats.d2h_bytes += (double)(row1 - row0) * (col1 - col0) * r->elt;
-      for (int t = ti; t <= te; ++t) r->state[tj * r->mt + t] |= HOST_VALID;
       any = true;
       ti = te + 1;
     }
   }
-  if (any) {
-    XK_HIP(hipEventRecord(ev_d2h, s_d2h));
-    pending_d2h = true;
-  }
+  return any;
 }
 
 // ---------------------------------------------------------------- staging
@@ -610,6 +639,7 @@ void Runtime::copy_d2h(char* dst, size_t dpitch, const char* src, size_t spitch,
 // Order the compute stream after the pending copies.
 void Runtime::before_compute()
 {
+  if (!unstamped.empty()) stamp_written();
   if (pending_h2d) {
     XK_HIP(hipEventRecord(ev_h2d, s_h2d));
     XK_HIP(hipStreamWaitEvent(s_comp, ev_h2d, 0));
@@ -1227,6 +1257,46 @@ bool pipeline_enabled()
   return g_pipeline != 0;
 }
 
+// Column panels (their last columns + 1) in which a product of resident
+// operands runs so that each panel can go back to the host while the next ones
+// are computed; empty: in one launch.  A large result takes a good part of the
+// product's own time to copy (57 GB/s measured: 2.1 ms beside the 4.4 ms of an
+// FP64 5003 x 3001 x 9011, 38 ms beside the 98 ms of a split-BF16 16384^3);
+// columns, because whole columns copy at that rate (9 KB pieces of 32 KB
+// columns at half of it).
+// MFMA modes: panels of about 300 tiles of 128 x 128 (0.6 of what the chip
+// holds) and 250 us, the first of half that, dealt in turn to two streams: two
+// panels, out of step, are in flight at any time, so that few CUs wait for a
+// panel's last tiles.  With the copy (one launch / panels): FP64 4096^3 4.67 /
+// 3.54 ms, 5003 x 3001 x 9011 7.22 / 5.57, 8192 x 8192 x 2000 14.0 / 10.2; a
+// caller who leaves the result on the device: 1.99 / 2.55, 4.53 / 4.65, 3.88 /
+// 4.04 ms (panels of 520 tiles 2.01, 4.66, 3.92, with the copy 4.00, 6.67, 10.1).
+// Split modes (planes): panels of at most 1/8 that add no round of 256 x 256
+// tiles over the 256 CUs.
+std::vector<int> result_panels(int M, int N, int K, size_t elt, int planes)
+{
+  std::vector<int> ends;
+  if ((double)M * N * elt < 17e6) return ends;  // 0.3 ms
+  if (planes) {
+    auto rounds = [&](int n) { return (int)(((long)((M + 255) / 256) * ((n + 255) / 256) * planes + 255) / 256); };
+    for (int p = 8; p >= 2; --p) {
+      const int h = (N / p + 255) / 256 * 256;
+      if (h >= N || (N + h - 1) / h * rounds(h) > 1.02 * rounds(N)) continue;
+      for (int e = h; e < N; e += h) ends.push_back(e);
+      break;
+    }
+  } else {
+    const int tm = (M + 127) / 128, tn = (N + 127) / 128;
+    const double us = 2.0 * M * N * K / (elt == 8 ? 62e6 : 118e6);
+    const int per = std::max({1, (300 + tm / 2) / tm, (tn + 11) / 12, (int)(tn * 250.0 / us)}), first = std::max(1, per / 2);
+    const int cnt = (tn - first + per / 2) / per;
+    if (cnt < 1) return ends;
+    for (int i = 0; i < cnt; ++i) ends.push_back(128 * (first + (int)((long)(tn - first) * i / cnt)));
+  }
+  if (!ends.empty()) ends.push_back(N);
+  return ends;
+}
+
 template <typename T>
 int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, const T* alpha, const T* A, int LDA,
                const T* B, int LDB, const T* beta, T* C, int LDC)
@@ -1264,18 +1334,66 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
   // one launch (in the split modes the row scalings span the whole inner
   // dimension and B's residue planes are computed once), so the result is
   // the same bit for bit.
-  const int panels = (M + nb - 1) / nb;
+  // With the operands resident, column panels let a result's copy back run
+  // under the product (result_panels).
   const bool rowsA = transA == NoTrans;
-  const bool pipe = use_ab && rA != rC && rB != rC && panels > 1 && pipeline_enabled() &&
-                    (!r.all_valid(rA, 0, 0, Am, An) || (readC && !r.all_valid(rC, 0, 0, M, N)));
-  if (pipe) {
+  const bool split = sizeof(T) == 8 && split_enabled<T>(x);
+  std::vector<int> ends;  // of the panels; empty: one launch
+  bool resident = false;
+  if (use_ab && rA != rC && rB != rC && pipeline_enabled()) {
+    resident = r.all_valid(rA, 0, 0, Am, An) && r.all_valid(rB, 0, 0, Bm, Bn) &&
+               (!readC || r.all_valid(rC, 0, 0, M, N));
+    if (resident) {
+      ends = result_panels(M, N, K, sizeof(T), split ? split_plane_count(K, x.nsplit, x.mode == XKBLAS_SPLIT_FP8_MATH) : 0);
+    } else if (M > nb && (!r.all_valid(rA, 0, 0, Am, An) || (readC && !r.all_valid(rC, 0, 0, M, N)))) {
+      for (int e = nb; e < M; e += nb) ends.push_back(e);
+      ends.push_back(M);
+    }
+  }
+  if (!ends.empty() && resident) {
+    if (split) split_cache_register((const double*)rA->dev, rA->ldd, M, K, rowsA);
+    Exec xs[2] = {x, x};  // the panels go in turn to two streams
+    const int old_tile = gemm_get_tile();
+    std::vector<Replica::PanelEvent> pev;
+    r.before_compute();
+    r.prof_begin(sizeof(T) == 8 ? "gemm_f64" : "gemm_f32", flops);
+    if (!split) {
+      xs[1].s = r.s_diag;
+      XK_HIP(hipEventRecord(r.ev_pot0, x.s));
+      XK_HIP(hipStreamWaitEvent(xs[1].s, r.ev_pot0, 0));
+      if (!old_tile) gemm_set_tile(gemm_tile_of<T>(M, N, K));  // the whole product's
+    }
+    int j0 = 0;
+    for (size_t p = 0; p < ends.size(); ++p) {
+      const T* Bp = (const T*)rB->dev + (transB == NoTrans ? (long)j0 * rB->ldd : (long)j0);
+      dev_gemm<T>(xs[p & 1], transA, transB, M, ends[p] - j0, K, *alpha, (const T*)rA->dev, rA->ldd, Bp, rB->ldd,
+                  *beta, (T*)rC->dev + (long)j0 * rC->ldd, rC->ldd);
+      hipEvent_t ev;
+      XK_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+      XK_HIP(hipEventRecord(ev, xs[p & 1].s));
+      pev.push_back(Replica::PanelEvent{ends[p], ev});
+      j0 = ends[p];
+    }
+    if (!split) {
+      gemm_set_tile(old_tile);
+      const size_t odd = (pev.size() & ~(size_t)1) - 1;  // the last panel of the other stream
+      XK_HIP(hipStreamWaitEvent(x.s, pev[odd].ev, 0));
+    }
+    r.prof_end();
+    if (split) split_cache_clear();
+    r.mark_written(rC, 0, 0, M, N, 0);
+    rC->panels = pev;
+    rC->panel_cols = true;
+    return 0;
+  }
+  if (!ends.empty()) {
     r.fetch(rB, 0, 0, Bm, Bn);
-    const bool split = sizeof(T) == 8 && split_enabled<T>(x);
     if (split) split_cache_register((const double*)rB->dev, rB->ldd, N, K, transB != NoTrans);
     std::vector<Replica::PanelEvent> pev;
     r.prof_begin(sizeof(T) == 8 ? "gemm_f64" : "gemm_f32", flops);
-    for (int p = 0; p < panels; ++p) {
-      const int r0 = p * nb, rows = std::min(nb, M - r0);
+    int r0 = 0;
+    for (int end : ends) {
+      const int rows = end - r0;
       if (rowsA) r.fetch(rA, r0, 0, rows, K);
       else r.fetch(rA, 0, r0, K, rows);
       if (readC) r.fetch(rC, r0, 0, rows, N);
@@ -1286,7 +1404,8 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
       hipEvent_t ev;
       XK_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
       XK_HIP(hipEventRecord(ev, x.s));
-      pev.push_back(Replica::PanelEvent{r0 + rows, ev});
+      pev.push_back(Replica::PanelEvent{end, ev});
+      r0 = end;
     }
     r.prof_end();
     if (split) split_cache_clear();

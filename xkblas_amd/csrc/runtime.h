@@ -32,14 +32,20 @@ struct Replica {
   // drops the mirrors of the calling thread only (each thread's descriptor
   // list in the reference, blas/xkblas.c:1855-1908)
   std::thread::id owner;
-  // Rows [.., end) of the mirror are final once `ev` completes on the
-  // compute stream (a product pipelined by row panels): the copy back of a
-  // row panel waits only for its own event.  Empty otherwise.
+  // Rows (panel_cols: columns) [.., end) of the mirror are final once `ev`
+  // completes (a product computed in panels): the copy back of a panel waits
+  // only for its own event.  Empty otherwise.
   struct PanelEvent {
     int end;
     hipEvent_t ev;
   };
   std::vector<PanelEvent> panels;
+  bool panel_cols = false;
+  // The last write of the mirror is complete with `written` on the compute
+  // stream once `stamped`; before that, with whatever the stream holds now.
+  // The event is recorded only when another call follows the write.
+  hipEvent_t written = nullptr;
+  bool stamped = false;
 };
 
 struct ProfEntry {
@@ -78,6 +84,7 @@ struct Runtime {
   hipEvent_t ev_comp = nullptr, ev_h2d = nullptr, ev_d2h = nullptr;
   hipEvent_t ev_pot0 = nullptr, ev_pot1 = nullptr;  // POTRF's lookahead ordering
   bool pending_h2d = false, pending_d2h = false;
+  std::vector<Replica*> unstamped;  // mirrors written by the last call on the compute stream
 
   std::unordered_map<const void*, Replica*> map;
   size_t cache_used = 0, cache_limit = 0;
@@ -147,7 +154,9 @@ struct Runtime {
   void fetch(Replica* r, int r0, int c0, int m, int n);
   void mark_written(Replica* r, int r0, int c0, int m, int n, int uplo);
   void writeback(Replica* r, int r0, int c0, int m, int n, int uplo);
-  void writeback_rows(Replica* r, int r0, int c0, int m, int n, int uplo);
+  bool copy_back(Replica* r, int row_lo, int row_hi, int col_lo, int col_hi, int uplo);
+  void stamp_written();
+  void release(Replica* r);
   bool all_valid(const Replica* r, int r0, int c0, int m, int n) const;
   void clear_panels(Replica* r);
   std::vector<Replica*>& begin_call();
