@@ -373,3 +373,45 @@ def test_cpotrf_fp32(xk):
     xk.invalidate()
     F = np.tril(A).astype(np.complex128)
     assert np.abs(H - F @ F.conj().T).max() / np.abs(H).max() < 1e-5
+
+
+@pytest.mark.parametrize("ta", OPS)
+@pytest.mark.parametrize("tb", OPS)
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+def test_gemm_real_scalars_exact(xk, ta, tb, dtype):
+    """Real alpha and beta take the form without packing B or C: exact on
+    Gaussian integers, at sizes where rows, columns and the inner dimension
+    end inside a tile, and C not read with beta = 0."""
+    for M, N, K in [(1, 1, 1), (33, 17, 9), (64, 65, 40), (130, 31, 77)]:
+        r = rng(M + N + K)
+        z = lambda m, n: np.asfortranarray((r.integers(-4, 5, (m, n)) + 1j * r.integers(-4, 5, (m, n))).astype(dtype))
+        A = z(M, K) if ta == 111 else z(K, M)
+        B = z(K, N) if tb == 111 else z(N, K)
+        C0 = z(M, N)
+        C = C0.copy(order="F")
+        D = np.full((M, N), np.nan, dtype=dtype, order="F")
+        xk.gemm(ta, tb, 2.0, A, B, -3.0, C)
+        xk.gemm(ta, tb, 1.0, A, B, 0.0, D)
+        xk.invalidate()
+        P = _op(A, ta) @ _op(B, tb)
+        assert np.array_equal(C, 2 * P - 3 * C0), (M, N, K)
+        assert np.array_equal(D, P), (M, N, K)
+
+
+@pytest.mark.parametrize("ta", OPS)
+@pytest.mark.parametrize("uplo", [121, 122])
+@pytest.mark.parametrize("n", [1, 8, 63, 65, 300])
+def test_ztrsm_diagonal_of_any_phase(xk, uplo, ta, n):
+    """Diagonal entries of every phase (real, negative, imaginary), one alpha
+    of each kind; bar as test_ztrsm."""
+    r = rng(n + uplo + ta)
+    T = _tri(n, uplo) * (r.uniform(0, 1, (n, n)) + 1j * r.uniform(0, 1, (n, n))) / n
+    T[np.diag_indices(n)] = np.resize([1.0, -1.0, 1j, -1j, 0.6 - 0.8j, -0.6 + 0.8j], n)
+    B0 = _c(r, n, 5)
+    for alpha in (0.8 - 0.2j, -2.0):
+        A, X = np.asfortranarray(np.where(_tri(n, uplo), T, np.nan)), B0.copy(order="F")
+        xk.trsm(141, uplo, ta, 131, alpha, A, X)
+        xk.invalidate()
+        ref = np.linalg.solve(_op(T, ta), alpha * B0)
+        err = _inf(X - ref) / ((_inf(_op(T, ta)) + _inf(ref)) * max(n, 5) * EPS)
+        assert err <= 10.0, err

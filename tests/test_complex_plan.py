@@ -133,3 +133,69 @@ def test_real_form_cholesky_is_rho_of_complex_factor():
     # the diagonal blocks of the real factor are l_ii I: the odd rows' entry
     # left of the diagonal is zero
     np.testing.assert_allclose(np.diag(R, -1)[0::2], 0, atol=1e-12)
+
+
+def rho_of(A, sigma=1):
+    """[rho(a_ij)] of a rectangular matrix (cplx_rho_kernel)."""
+    M = np.empty((2 * A.shape[0], 2 * A.shape[1]))
+    M[0::2, 0::2] = M[1::2, 1::2] = A.real
+    M[1::2, 0::2] = sigma * A.imag
+    M[0::2, 1::2] = -sigma * A.imag
+    return M
+
+
+def pairs(X):
+    """An interleaved complex matrix as the real one it is in memory."""
+    out = np.empty((2 * X.shape[0], X.shape[1]))
+    out[0::2], out[1::2] = X.real, X.imag
+    return out
+
+
+def unpair(X):
+    return X[0::2] + 1j * X[1::2]
+
+
+@pytest.mark.parametrize("ta,tb", list(itertools.product([N_, T_, C_], repeat=2)))
+def test_rho_plan_matches_complex_product(ta, tb):
+    """The product with real scalars: rho(A) (Trans: of conj A), B as it lies
+    in memory or dealt into real and imaginary columns (cplx_deal_kernel)."""
+    r = np.random.default_rng(ta * 3 + tb)
+    m, n, k = 7, 5, 6
+    c = lambda p, q: r.standard_normal((p, q)) + 1j * r.standard_normal((p, q))
+    A = c(m, k) if ta == N_ else c(k, m)
+    B = c(k, n) if tb == N_ else c(n, k)
+    C = c(m, n)
+    op = lambda X, t: X if t == N_ else (X.T if t == T_ else X.conj().T)
+    YA = rho_of(A, -1 if ta == T_ else 1)
+    X = YA if ta == N_ else YA.T
+    if tb == N_:
+        Y = pairs(B)
+    else:
+        D = np.empty((n, 2 * k))
+        D[:, 0::2], D[:, 1::2] = B.real, (-1 if tb == C_ else 1) * B.imag
+        Y = D.T
+    got = unpair(1.5 * (X @ Y) - 0.5 * pairs(C))
+    np.testing.assert_allclose(got, 1.5 * (op(A, ta) @ op(B, tb)) - 0.5 * C, atol=1e-12)
+
+
+@pytest.mark.parametrize("ta", [N_, T_, C_])
+@pytest.mark.parametrize("lower", [True, False])
+def test_real_triangular_solve_plan(ta, lower):
+    """The left solve: T = T' D with |D| = 1 and a real positive diagonal in
+    T', rho(T') triangular, the rows scaled before or after as dev_ctrsm does."""
+    r = np.random.default_rng(ta + lower)
+    n, nrhs = 6, 3
+    c = lambda p, q: r.standard_normal((p, q)) + 1j * r.standard_normal((p, q))
+    T = (np.tril if lower else np.triu)(c(n, n)) + np.diag(3 * np.exp(1j * r.uniform(0, 6.28, n)))
+    B, alpha = c(n, nrhs), 0.8 - 0.2j
+    d = T.diagonal() / np.abs(T.diagonal())
+    R = rho_of(T * d.conj()[None, :])
+    np.testing.assert_allclose(np.triu(R, 1) if lower else np.tril(R, -1), 0, atol=1e-14)
+    if ta == N_:
+        X = alpha * d.conj()[:, None] * unpair(np.linalg.solve(R, pairs(B)))
+    elif ta == C_:
+        X = unpair(np.linalg.solve(R.T, pairs(alpha * d[:, None] * B)))
+    else:
+        X = unpair(np.linalg.solve(R.T, pairs(np.conj(alpha) * d[:, None] * B.conj()))).conj()
+    op = T if ta == N_ else (T.T if ta == T_ else T.conj().T)
+    np.testing.assert_allclose(op @ X, alpha * B, atol=1e-12)

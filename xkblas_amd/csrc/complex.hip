@@ -9,6 +9,10 @@
 // transposed or conjugated operand they build the transpose of the block
 // matrix, which the GEMM then reads transposed — and fold alpha, beta back
 // into the interleaved C.  All are single HBM passes.
+// With rows and columns in pairs the block operand is rho(X), rho(z) = [re
+// -im; im re], and the interleaved Y and C are the other two operands as they
+// lie in memory (real matrices of twice as many rows): with real alpha and
+// beta only rho(X) is built.  rho(Z)^T = rho(Z^H).
 #include "kernels.h"
 #include <algorithm>
 
@@ -47,6 +51,90 @@ __global__ __launch_bounds__(256) void cplx_pack_b_kernel(int vertical, int rows
   Y[i + (long)j * ldy] = b.re;
   if (vertical) Y[i + rows + (long)j * ldy] = b.im;
   else Y[i + (long)(j + cols) * ldy] = s * b.im;
+}
+
+// Y (2 rows x 2 cols) <- rho of the rows x cols complex A (s = -1: of conj A).
+template <typename T>
+__global__ __launch_bounds__(256) void cplx_rho_kernel(int rows, int cols, int j0, T s, const Cplx<T>* __restrict__ A,
+                                                       long lda, T* __restrict__ Y, long ldy)
+{
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int j = j0 + (int)blockIdx.y;
+  if (i >= rows || j >= cols) return;
+  const Cplx<T> a = A[i + (long)j * lda];
+  Cplx<T>* y = reinterpret_cast<Cplx<T>*>(Y + (long)(2 * j) * ldy) + i;  // ldy is even
+  *y = Cplx<T>{a.re, s * a.im};
+  y = reinterpret_cast<Cplx<T>*>(Y + (long)(2 * j + 1) * ldy) + i;
+  *y = Cplx<T>{-s * a.im, a.re};
+}
+
+// Y (rows x 2 cols) <- the columns' real parts and s times their imaginary
+// parts in turn: read transposed, the interleaved form of B^T (s = -1: B^H).
+template <typename T>
+__global__ __launch_bounds__(256) void cplx_deal_kernel(int rows, int cols, int j0, T s, const Cplx<T>* __restrict__ B,
+                                                        long ldb, T* __restrict__ Y, long ldy)
+{
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int j = j0 + (int)blockIdx.y;
+  if (i >= rows || j >= cols) return;
+  const Cplx<T> b = B[i + (long)j * ldb];
+  Y[i + (long)(2 * j) * ldy] = b.re;
+  Y[i + (long)(2 * j + 1) * ldy] = s * b.im;
+}
+
+// Real triangular form of a complex triangular matrix T for its solves: T = T'
+// D with D diagonal of modulus one and a real positive diagonal in T', so that
+// rho(T') is triangular itself.  R (2n x 2n, uplo triangle) <- rho(T'), D its
+// n diagonal entries (1 when unit: the diagonal is not read).
+template <typename T>
+__global__ __launch_bounds__(256) void cplx_trsm_form_kernel(int uplo, int unit, int n, int j0,
+                                                             const Cplx<T>* __restrict__ A, long lda,
+                                                             T* __restrict__ R, long ldr, Cplx<T>* __restrict__ D)
+{
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int j = j0 + (int)blockIdx.y;
+  if (i >= n || (uplo == Lower ? i < j : i > j)) return;
+  Cplx<T> d{T(1), T(0)};
+  T h = T(1);
+  if (!unit) {
+    const Cplx<T> t = A[j + (long)j * lda];
+    h = t.im == T(0) ? fabs(t.re) : hypot(t.re, t.im);
+    if (t.im == T(0)) d.re = t.re < T(0) ? T(-1) : T(1);
+    else d = Cplx<T>{t.re / h, t.im / h};
+  }
+  Cplx<T> z{h, T(0)};
+  if (i == j) {
+    D[j] = d;
+  } else {
+    const Cplx<T> a = A[i + (long)j * lda];  // times conj(d)
+    z = d.im == T(0) ? Cplx<T>{a.re * d.re, a.im * d.re}
+                     : Cplx<T>{a.re * d.re + a.im * d.im, a.im * d.re - a.re * d.im};
+  }
+  T* r = R + 2 * i + (long)(2 * j) * ldr;
+  r[0] = z.re;
+  r[1] = z.im;
+  r[ldr] = -z.im;
+  r[ldr + 1] = z.re;
+}
+
+// B(i, j) <- alpha B(i, j) D(i), with conj(B) when conj_b, conj(D) when
+// conj_d; D null: 1.
+template <typename T>
+__global__ __launch_bounds__(256) void cplx_scale_rows_kernel(int m, int n, int j0, int conj_b, int conj_d, T ar, T ai,
+                                                              const Cplx<T>* __restrict__ D, Cplx<T>* __restrict__ B,
+                                                              long ldb)
+{
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int j = j0 + (int)blockIdx.y;
+  if (i >= m || j >= n) return;
+  Cplx<T> b = B[i + (long)j * ldb];
+  if (conj_b) b.im = -b.im;
+  auto times = [&](T re, T im) {
+    b = im == T(0) ? Cplx<T>{b.re * re, b.im * re} : Cplx<T>{b.re * re - b.im * im, b.re * im + b.im * re};
+  };
+  if (D) times(D[i].re, conj_d ? -D[i].im : D[i].im);
+  times(ar, ai);
+  B[i + (long)j * ldb] = b;
 }
 
 // Two real blocks of the rows x cols complex B side by side (vertical = 0:
@@ -203,7 +291,7 @@ __global__ __launch_bounds__(256) void cplx_realform_kernel(int uplo, int n, int
 // The complex factor and inverse back from the real ones: l_ij = R[2i][2j] +
 // i R[2i+1][2j] for i >= j (a real diagonal), to A's stored triangle (Upper:
 // U(j, i) = conj(l_ij)); likewise inv(L) from Rinv to Tinv (Upper: inv(U) =
-// inv(L)^H).  Tinv's other triangle is not written.
+// inv(L)^H) unless that is null.  Tinv's other triangle is not written.
 template <typename T>
 __global__ __launch_bounds__(256) void cplx_fromreal_kernel(int uplo, int n, int j0, const T* __restrict__ R, long ldr,
                                                             Cplx<T>* __restrict__ A, long lda,
@@ -215,6 +303,11 @@ __global__ __launch_bounds__(256) void cplx_fromreal_kernel(int uplo, int n, int
   if (i >= n || j > i) return;
   const long e = 2 * i + (long)(2 * j) * ldr;
   Cplx<T> l{R[e], i == j ? T(0) : R[e + 1]};
+  if (!Tinv) {
+    if (uplo == Lower) A[i + (long)j * lda] = l;
+    else A[j + (long)i * lda] = Cplx<T>{l.re, -l.im};
+    return;
+  }
   Cplx<T> v{Rinv[e], i == j ? T(0) : Rinv[e + 1]};
   if (uplo == Lower) {
     A[i + (long)j * lda] = l;
@@ -249,6 +342,50 @@ void cplx_pack_b(hipStream_t s, int vertical, int sign, int rows, int cols, cons
   over_columns(rows, cols, [&](dim3 g, int j0) {
     hipLaunchKernelGGL((cplx_pack_b_kernel<T>), g, dim3(256), 0, s, vertical, rows, cols, j0, T(sign),
                        (const Cplx<T>*)B, ldb, Y, ldy);
+  });
+  XK_HIP(hipGetLastError());
+}
+
+template <typename T>
+void cplx_rho(hipStream_t s, int sigma, int rows, int cols, const T* A, long lda, T* Y, long ldy)
+{
+  if (rows <= 0 || cols <= 0) return;
+  over_columns(rows, cols, [&](dim3 g, int j0) {
+    hipLaunchKernelGGL((cplx_rho_kernel<T>), g, dim3(256), 0, s, rows, cols, j0, T(sigma), (const Cplx<T>*)A, lda, Y,
+                       ldy);
+  });
+  XK_HIP(hipGetLastError());
+}
+
+template <typename T>
+void cplx_deal(hipStream_t s, int sign, int rows, int cols, const T* B, long ldb, T* Y, long ldy)
+{
+  if (rows <= 0 || cols <= 0) return;
+  over_columns(rows, cols, [&](dim3 g, int j0) {
+    hipLaunchKernelGGL((cplx_deal_kernel<T>), g, dim3(256), 0, s, rows, cols, j0, T(sign), (const Cplx<T>*)B, ldb, Y,
+                       ldy);
+  });
+  XK_HIP(hipGetLastError());
+}
+
+template <typename T>
+void cplx_trsm_form(hipStream_t s, int uplo, int unit, int n, const T* A, long lda, T* R, long ldr, T* D)
+{
+  if (n <= 0) return;
+  over_columns(n, n, [&](dim3 g, int j0) {
+    hipLaunchKernelGGL((cplx_trsm_form_kernel<T>), g, dim3(256), 0, s, uplo, unit, n, j0, (const Cplx<T>*)A, lda, R,
+                       ldr, (Cplx<T>*)D);
+  });
+  XK_HIP(hipGetLastError());
+}
+
+template <typename T>
+void cplx_scale_rows(hipStream_t s, int m, int n, int conj_b, int conj_d, const T* alpha, const T* D, T* B, long ldb)
+{
+  if (m <= 0 || n <= 0) return;
+  over_columns(m, n, [&](dim3 g, int j0) {
+    hipLaunchKernelGGL((cplx_scale_rows_kernel<T>), g, dim3(256), 0, s, m, n, j0, conj_b, conj_d, alpha[0], alpha[1],
+                       (const Cplx<T>*)D, (Cplx<T>*)B, ldb);
   });
   XK_HIP(hipGetLastError());
 }
@@ -322,6 +459,10 @@ void cplx_fromreal(hipStream_t s, int uplo, int n, const T* R, long ldr, T* A, l
 }
 
 #define XK_INST(T)                                                                                         \
+  template void cplx_rho<T>(hipStream_t, int, int, int, const T*, long, T*, long);                          \
+  template void cplx_deal<T>(hipStream_t, int, int, int, const T*, long, T*, long);                         \
+  template void cplx_trsm_form<T>(hipStream_t, int, int, int, const T*, long, T*, long, T*);                \
+  template void cplx_scale_rows<T>(hipStream_t, int, int, int, int, const T*, const T*, T*, long);          \
   template void cplx_realform<T>(hipStream_t, int, int, const T*, long, T*, long);                         \
   template void cplx_fromreal<T>(hipStream_t, int, int, const T*, long, T*, long, const T*, T*, long);      \
   template void cplx_trtri_leaf<T>(hipStream_t, int, int, int, const T*, long, long, T*, long, long, int); \

@@ -103,6 +103,20 @@ template <typename T>
 void cplx_pack_a(hipStream_t s, int sigma, int rows, int cols, const T* A, long lda, T* Y, long ldy);
 template <typename T>
 void cplx_pack_b(hipStream_t s, int vertical, int sign, int rows, int cols, const T* B, long ldb, T* Y, long ldy);
+// Y (2 rows x 2 cols) <- rho(A) (sigma -1: rho(conj A)), rho(z) = [re -im; im
+// re] per element, ldy even; Y (rows x 2 cols) <- B's columns dealt into their
+// real and (times sign) imaginary parts.
+template <typename T>
+void cplx_rho(hipStream_t s, int sigma, int rows, int cols, const T* A, long lda, T* Y, long ldy);
+template <typename T>
+void cplx_deal(hipStream_t s, int sign, int rows, int cols, const T* B, long ldb, T* Y, long ldy);
+// The triangle A = T' D (D of modulus one, T' with a real positive diagonal):
+// R (2n x 2n, uplo triangle) <- rho(T'), D its n entries; and B(i, j) <- alpha
+// B(i, j) D(i) with conj(B) / conj(D) as asked (D null: 1).
+template <typename T>
+void cplx_trsm_form(hipStream_t s, int uplo, int unit, int n, const T* A, long lda, T* R, long ldr, T* D);
+template <typename T>
+void cplx_scale_rows(hipStream_t s, int m, int n, int conj_b, int conj_d, const T* alpha, const T* D, T* B, long ldb);
 // Y <- [sr Br, si Bi] (rows x 2 cols) or, vertical, [sr Br; si Bi] (2 rows x
 // cols); swap puts the si Bi block first.
 template <typename T>
@@ -128,7 +142,7 @@ template <typename T>
 void cplx_realform(hipStream_t s, int uplo, int n, const T* A, long lda, T* R, long ldr);
 // From the real forms rho(L) (R) and rho(inv(L)) (Rinv, same leading
 // dimension): L to A's uplo triangle (Upper: U = L^H) and inv(L) to Tinv's
-// (Upper: inv(U)).
+// (Upper: inv(U)); Rinv and Tinv null: the factor only.
 template <typename T>
 void cplx_fromreal(hipStream_t s, int uplo, int n, const T* R, long ldr, T* A, long lda, const T* Rinv, T* Tinv,
                    long ldinv);
