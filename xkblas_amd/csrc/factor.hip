@@ -176,18 +176,18 @@ __device__ __forceinline__ void pin(T& x)
 
 // Cholesky factor and inverse of one 16 x 16 tile by one wave.  In: d[c] =
 // A(i, c), the whole symmetric row i = lane % 16 (the four rows of 16 lanes
-// hold the same data).  Out: l[c] = L(i, c) and d[c] = inv(L)(i, c), zero
-// above the diagonal.  Returns this lane's pivot.
+// hold the same data).  Out, below the diagonal: l[c] = L(i, c) sqrt(p_c) and
+// d[c] = inv(L)(i, c) sqrt(p_i), p the pivots.  Returns this lane's pivot.
 // Elimination without roots: W A = U with W unit lower triangular, the
 // columns of W taking the place of the eliminated columns, so that each of
 // the 16 steps is one reciprocal and 15 row updates from row j; the pivots'
-// roots follow once, for all 16 pivots at a time: L(i, j) = A_j(i, j) /
-// sqrt(p_j), inv(L) = diag(1 / sqrt(p)) W.
+// roots are left to the caller, who takes them once, for all 16 pivots at a
+// time: L(i, j) = A_j(i, j) / sqrt(p_j), inv(L) = diag(1 / sqrt(p)) W.
 // A step's chain is pivot (broadcast) -> mantissa -> reciprocal -> two
 // corrections -> multiplier -> next pivot: 8 dependent instructions.  The
 // updates of the step before stand between them, in this order (one wave,
 // in-order issue; ordered by the compiler, a leaf of 128 took 39.6 us instead
-// of 33.4).
+// of 33.4 of then).
 template <typename T>
 __device__ __forceinline__ T factor16(T (&d)[16], T (&l)[16], int i)
 {
@@ -242,14 +242,6 @@ __device__ __forceinline__ T factor16(T (&d)[16], T (&l)[16], int i)
       m = fma(q, e, q);
     }
 #undef XK_UPD
-  });
-  T sq, rs;
-  sqrt_rcp(piv, sq, rs);
-  for_each<16>([&](auto jc) {
-    constexpr int j = decltype(jc)::value;
-    const T rj = row_bcast<j>(rs);
-    l[j] = i > j ? l[j] * rj : (i == j ? sq : T(0));
-    d[j] = i > j ? d[j] * rs : (i == j ? rs : T(0));
   });
   return piv;
 }
@@ -322,24 +314,35 @@ __device__ __forceinline__ void leaf_load(T* S, int uplo, int n, int nt, const T
 // or 8), one workgroup of NT waves, all products on MFMA tiles.
 // The chain of step k is wave 0's alone: factor and invert diagonal tile k in
 // registers (factor16), form panel tile (k + 1, k) = A inv(L_kk)^T and update
-// diagonal tile k + 1 with it, which is then ready for step k + 1.  Beside
-// the next factor16 the other waves update the remaining trailing tiles and
-// form row k of the inverse, inv(L)(k, j) = -inv(L_kk) sum_t L(k, t)
-// inv(L)(t, j), kept transposed (Z) in the places of row k of L, which
-// nothing reads any more.  Two barriers a step, ordering LDS only.
-// Bound by latency: 16 orders take 4 us, 2.1 of them the 16 dependent pivots;
-// order 128 33 us (FP64), where two leaves of order 64 with scalar panels and
-// the six launches that joined them took 130.
-// LDS: 20.5 KB (FP64, NT = 4), 73.7 KB (NT = 8).
+// diagonal tile k + 1 with it, which is then ready for step k + 1.  Behind it
+// the other waves form the rest of the panel and row k of the inverse,
+// inv(L)(k, j) = inv(L_kk) S(k, j), update the remaining trailing tiles and the
+// sums S(i, j) = -sum_t L(i, t) inv(L)(t, j) of the rows below, and write the
+// results to memory.  S and the inverse are kept transposed, in the places of
+// L, whose column k nothing reads after step k.
+// The waves meet in counters in LDS instead of barriers, so that wave 0 waits
+// only for what its next step reads: diagonal tiles done (by wave 0), panel
+// tiles and rows of the inverse done (all waves), updates of the two tiles that
+// wave 0 takes next, waves done with the step (all but wave 0; their loads of A
+// are step 0 of this count).  The waves of a workgroup are resident together
+// and none leaves before its last count, so every wait ends.
+// Bound by latency: a step takes 6.7k cycles, 3.0k of them the 16 dependent
+// pivots.  Order 128 takes 27.5 us (FP64); it took 33.4 with two barriers a
+// step, the stores to memory on wave 0's way and the sums formed whole when
+// their row came up, and two leaves of order 64 with scalar panels and the six
+// launches that joined them took 130.
+// LDS: 27.4 KB (FP64, NT = 4), 80.7 KB (NT = 8).
 template <typename T, int NT>
-__global__ __launch_bounds__(64 * NT) void potrf_leaf_kernel(int uplo, int n, T* A, long lda, long sA, T* Tinv,
-                                                             long ldinv, long sInv, int* info, int base, int pair)
+__global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(4)))
+void potrf_leaf_kernel(int uplo, int n, T* A, long lda, long sA, T* Tinv, long ldinv, long sInv, int* info, int base,
+                       int pair)
 {
   typedef typename LeafV<T>::type V;
+  constexpr int NW = NT - 1;  // waves beside wave 0
   __shared__ T S[NT * (NT + 1) / 2 * TS];
-  // the latency-bound step of the diagonal chain may share its CU with
-  // update GEMM waves: its waves issue first
-  __builtin_amdgcn_s_setprio(2);
+  __shared__ T LK[3 * TS], RT[3 * 32];  // factor16's l, the pivots' roots and their reciprocals, for the stores of L_kk
+  __shared__ int done[4];
+  enum { DIAG, PANEL, NEXT, TRAIL };
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ti = lane & 15, g = lane >> 4;
   const int nt = (n + 15) >> 4;
@@ -352,92 +355,189 @@ __global__ __launch_bounds__(64 * NT) void potrf_leaf_kernel(int uplo, int n, T*
       else M[k + (long)i * ld] = v;
     }
   };
-  leaf_load<T, NT>(S, uplo, n, nt, A, lda, true, false);
+  // One more of c is done.  The LDS executes a wave's operations in order, so
+  // whoever sees the count sees this wave's writes before it: it is enough
+  // that the compiler keeps the order, nothing is waited for.
+  auto signal = [&](int c) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    if (lane == 0) __hip_atomic_fetch_add(&done[c], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  // until c has reached `count` and c2 `count2`
+  auto wait2 = [&](int c, int count, int c2, int count2) {
+    for (;;) {
+      const int a = __hip_atomic_load(&done[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      const int b = __hip_atomic_load(&done[c2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (__builtin_amdgcn_readfirstlane(a) >= count && __builtin_amdgcn_readfirstlane(b) >= count2) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  if (threadIdx.x < 4) done[threadIdx.x] = 0;
   lds_barrier();
-  int fail = INT_MAX;  // first order with a non-positive pivot (wave 0)
-  V z = {0, 0, 0, 0};  // this wave's tile of the inverse's current row
-  for (int k = 0; k < nt; ++k) {
-    const int c0 = k * 16;
-    T* Dk = S + tile_slot(k, k);
-    V dk;
-    if (wave == 0) {
-      __builtin_amdgcn_s_setprio(3);
+  leaf_load<T, NT>(S, uplo, n, nt, A, lda, true, false);  // wave 0: tile (0, 0)
+  if (wave == 0) {
+    // the latency-bound step of the diagonal chain, which may share its CU
+    // with update GEMM waves: its instructions issue first
+    __builtin_amdgcn_s_setprio(3);
+    int fail = INT_MAX;  // first order with a non-positive pivot
+    for (int k = 0; k < nt; ++k) {
+      const int c0 = k * 16;
+      T* Dk = S + tile_slot(k, k);
       T d[16], l[16];
 #pragma unroll
       for (int c = 0; c < 16; ++c) d[c] = Dk[ti + 16 * col_pos<T>(c)];
       const T piv = factor16(d, l, ti);
       const unsigned long long bad = __ballot(!(piv > T(0)) && c0 + ti < n);
       if (bad && fail == INT_MAX) fail = c0 + __ffsll(bad) - 1;
-      dk = row_to_tile(d, g);
-      tile_store(Dk, lane, dk);
-      const V lk = row_to_tile(l, g);
+      T sq, rs;
+      sqrt_rcp(piv, sq, rs);
+      V dk = row_to_tile(d, g);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int col = tile_col<T>(g, r);
+        dk[r] = ti > col ? dk[r] * rs : (ti == col ? rs : T(0));
+      }
+      tile_store(Dk, lane, dk);
+      signal(DIAG);
+      const V lk = row_to_tile(l, g);
+      // for the stores of L_kk
+      auto keep = [&]() {
+        tile_store(LK + k % 3 * TS, lane, lk);
+        if (g < 2) RT[k % 3 * 32 + lane] = g ? rs : sq;
+        signal(PANEL);
+      };
+      if (k + 1 == nt) {
+        keep();
+        break;
+      }
+      // tiles (k + 1, k) and (k + 1, k + 1), there with all updates before k
+      T* P = S + tile_slot(k + 1, k);
+      T* C = S + tile_slot(k + 1, k + 1);
+      wait2(TRAIL, NW, NEXT, 2 * k);
+      const V a = tile_load(P, lane), c = tile_load(C, lane);
+      const V z = {0, 0, 0, 0};
+      const V lp = tile_xyt(z, a, dk);
+      tile_store(P, lane, lp);
+      keep();
+      tile_store(C, lane, tile_xyt(c, lp, -lp));
+    }
+    // pair: orders 2i, 2i + 1 stand for order i of a complex block
+    if (lane == 0 && fail != INT_MAX) atomicMin(info, pair ? (base + fail) / 2 + 1 : base + fail + 1);
+    return;
+  }
+  signal(TRAIL);           // its tile row is loaded
+  // Trailing tiles are counted from the last, column after column, rows
+  // falling: those of step k are the first of one list for all steps, dealt to
+  // waves 1 .. in turn.  A wave keeps its tiles in registers until the step
+  // that takes them, tile (i, q) up to step lim - 1.
+  constexpr int MT = (NT * (NT - 1) / 2 - 1 + NW - 1) / NW;
+  V c[MT];
+  int ci[MT], cq[MT], lim[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    int e = 0, r = wave - 1 + NW * m;
+    while (r > e) r -= ++e;
+    ci[m] = nt - 1 - r;
+    cq[m] = nt - 1 - e;
+    lim[m] = ci[m] == cq[m] ? cq[m] - 1 : cq[m];
+  }
+  const V zero = {0, 0, 0, 0};
+  V s = zero;
+  for (int k = 0; k < nt; ++k) {
+    const int c0 = k * 16, h = nt - 1 - k;
+    const int pi = k + 1 + wave;  // this wave's tile row of the panel (wave 0: k + 1)
+    V lp = zero, z = zero;
+    wait2(DIAG, k + 1, TRAIL, (k + 1) * NW);
+    const V dk = tile_load(S + tile_slot(k, k), lane);
+    // S(k - 1 + wave, k - 1), now that column k - 1 of L has been read
+    if (Tinv && wave > 1 && k > 0 && k - 1 + wave < nt) tile_store(S + tile_slot(k - 1 + wave, k - 1), lane, s);
+    if (pi < nt) {
+      T* P = S + tile_slot(pi, k);
+      lp = tile_xyt(zero, tile_load(P, lane), dk);
+      tile_store(P, lane, lp);
+    }
+    // row k of the inverse, one tile a wave: column k - 1 is wave 1's
+    const int j = wave == 1 ? k - 1 : wave - 2;
+    const bool inv = Tinv && j >= 0 && (wave == 1 || j < k - 1);
+    if (inv) {
+      if (wave > 1) s = tile_load(S + tile_slot(k, j), lane);
+      z = tile_xyt(zero, s, dk);
+      tile_store(S + tile_slot(k, j), lane, z);
+    }
+    signal(PANEL);
+    if (k == 0) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        if (lim[m] > 0) c[m] = tile_load(S + tile_slot(ci[m], cq[m]), lane);
+    }
+    wait2(PANEL, (k + 1) * NT, DIAG, 0);
+    // trailing updates, those that wave 0 waits for first
+#pragma unroll
+    for (int m = MT - 1; m >= 0; --m)
+      if (lim[m] > k) {
+        const V x = tile_load(S + tile_slot(ci[m], k), lane), y = tile_load(S + tile_slot(cq[m], k), lane);
+        c[m] = tile_xyt(c[m], x, -y);
+        if (lim[m] == k + 1) tile_store(S + tile_slot(ci[m], cq[m]), lane, c[m]);
+        if (ci[m] == k + 2) signal(NEXT);
+      }
+    if (Tinv) {
+      // S(i, j) -= L(i, k) inv(L)(k, j) for j < k < i, the waves with fewer
+      // trailing tiles first; v / h by a multiplication
+      const int rh = (int)(0x13161a202b408000ull >> (8 * h)) & 255;
+      int v = wave - 1 - (h * (h + 1) / 2 - 1) % NW;
+      for (v = v < 0 ? v + NW : v; v < k * h; v += NW) {
+        const int jj = v * rh >> 7, i = k + 1 + v - jj * h;
+        T* C = S + tile_slot(i, jj);
+        const V x = tile_load(S + tile_slot(k, jj), lane), y = tile_load(S + tile_slot(i, k), lane);
+        tile_store(C, lane, tile_xyt(tile_load(C, lane), x, -y));
+      }
+      // S(k + wave, k) = -L(k + wave, k) inv(L_kk)
+      if (wave <= h)
+        s = tile_xyt(zero, tile_load_t(S + tile_slot(k, k), lane), -tile_load(S + tile_slot(k + wave, k), lane));
+    }
+    // the last wave, without panel tiles, writes the diagonal tile and wave 0's panel tile
+    const bool mine = wave == NW;
+    V lk, l0;
+    if (mine) {
+      lk = tile_load(LK + k % 3 * TS, lane);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int col = tile_col<T>(g, r);
+        const T root = RT[k % 3 * 32 + (ti > col ? 16 + col : ti)];
+        lk[r] = ti > col ? lk[r] * root : root;
+      }
+      if (h) l0 = tile_load(S + tile_slot(k + 1, k), lane);
+    }
+    signal(TRAIL);
+    // to memory: tile rows `row` .., columns col0 .., or their mirror image;
+    // only the last tile row has orders beyond n
+    auto put_tile = [&](T* M, long ld, int row, int col0, bool mirror, const V& t) {
+      if (row + ti >= n) return;
+      const bool down = (uplo == Lower) != mirror;
+      T* q = M + (down ? row + ti + col0 * ld : (row + ti) * ld + col0);
+      const long step = down ? ld : 1;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) q[tile_col<T>(g, r) * step] = t[r];
+    };
+    if (pi < nt) {
+      put_tile(A, lda, pi * 16, c0, false, lp);
+      if (Tinv) put_tile(Tinv, ldinv, pi * 16, c0, true, zero);
+    }
+    if (mine && h) {
+      put_tile(A, lda, c0 + 16, c0, false, l0);
+      if (Tinv) put_tile(Tinv, ldinv, c0 + 16, c0, true, zero);
+    }
+    if (inv && h) put_tile(Tinv, ldinv, j * 16, c0, true, z);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int col = tile_col<T>(g, r);
+      if (inv && !h) put(Tinv, ldinv, c0 + col, j * 16 + ti, z[r]);
+      if (mine) {
         if (col <= ti) put(A, lda, c0 + ti, c0 + col, lk[r]);
         if (Tinv) put(Tinv, ldinv, c0 + ti, c0 + col, dk[r]);
       }
     }
-    lds_barrier();
-    // row k - 1 of the inverse takes the place of row k - 1 of L
-    if (wave > 0 && wave < k) tile_store(S + tile_slot(k - 1, wave - 1), lane, z);
-    if (wave > 0) dk = tile_load(Dk, lane);
-    // panel: tile row k + 1 + wave
-    V lp = {0, 0, 0, 0};
-    const int pi = k + 1 + wave;
-    if (pi < nt) {
-      T* P = S + tile_slot(pi, k);
-      lp = tile_xyt(lp, tile_load(P, lane), dk);
-      tile_store(P, lane, lp);
-    }
-    lds_barrier();
-    if (wave == 0) {
-      if (k + 1 < nt) {
-        T* C = S + tile_slot(k + 1, k + 1);
-        V c = tile_load(C, lane);
-        c = tile_xyt(c, lp, -lp);
-        tile_store(C, lane, c);
-      }
-    } else {
-      // trailing tiles (i, j), k < j <= i, but the first, dealt to waves 1 ..
-      int t = wave;  // tile index in column order, (k + 1, k + 1) is 0
-      for (int j = k + 1; j < nt; ++j) {
-        const int h = nt - j;
-        for (; t < h; t += NT - 1) {
-          const int i = j + t;
-          T* C = S + tile_slot(i, j);
-          V c = tile_load(C, lane);
-          const V x = tile_load(S + tile_slot(i, k), lane), y = tile_load(S + tile_slot(j, k), lane);
-          c = tile_xyt(c, x, -y);
-          tile_store(C, lane, c);
-        }
-        t -= h;
-      }
-      // row k of the inverse, block column j = wave - 1
-      const int j = wave - 1;
-      if (j < k && Tinv) {
-        V s = {0, 0, 0, 0};
-        s = tile_xyt(s, tile_load_t(S + tile_slot(j, j), lane), tile_load(S + tile_slot(k, j), lane));
-        for (int u = j + 1; u < k; ++u)
-          s = tile_xyt(s, tile_load(S + tile_slot(u, j), lane), tile_load(S + tile_slot(k, u), lane));
-        z = V{0, 0, 0, 0};
-        z = tile_xyt(z, s, -dk);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) put(Tinv, ldinv, c0 + tile_col<T>(g, r), j * 16 + ti, z[r]);
-      }
-    }
-    // the panel's factor entries, and zeros across the diagonal of the inverse
-    if (pi < nt) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = c0 + tile_col<T>(g, r);
-        put(A, lda, pi * 16 + ti, col, lp[r]);
-        if (Tinv) put(Tinv, ldinv, col, pi * 16 + ti, T(0));
-      }
-    }
   }
-  // pair: orders 2i, 2i + 1 stand for order i of a complex block
-  if (threadIdx.x == 0 && fail != INT_MAX) atomicMin(info, pair ? (base + fail) / 2 + 1 : base + fail + 1);
 }
 
 // Inverse of one triangular block of order <= 16 NT, one workgroup of NT
