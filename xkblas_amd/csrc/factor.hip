@@ -324,8 +324,11 @@ __device__ __forceinline__ void leaf_load(T* S, int uplo, int n, int nt, const T
 // only for what its next step reads: diagonal tiles done (by wave 0), panel
 // tiles and rows of the inverse done (all waves), updates of the two tiles that
 // wave 0 takes next, waves done with the step (all but wave 0; their loads of A
-// are step 0 of this count).  The waves of a workgroup are resident together
-// and none leaves before its last count, so every wait ends.
+// are step 0 of this count).  A count stands for a step only while no wave can
+// add the next step's before all have added this one's: a wave that adds to one
+// has waited for the step before to be complete in it.  The waves of a
+// workgroup are resident together and none leaves before its last count, so
+// every wait ends.
 // Bound by latency: a step takes 6.7k cycles, 3.0k of them the 16 dependent
 // pivots.  Order 128 takes 27.5 us (FP64); it took 33.4 with two barriers a
 // step, the stores to memory on wave 0's way and the sums formed whole when
@@ -407,6 +410,9 @@ void potrf_leaf_kernel(int uplo, int n, T* A, long lda, long sA, T* Tinv, long l
         signal(PANEL);
       };
       if (k + 1 == nt) {
+        // nothing above waits for the other waves in this step: their part of
+        // the step before has to be counted before this one's
+        wait2(PANEL, k * NT, DIAG, 0);
         keep();
         break;
       }
