@@ -281,6 +281,22 @@ static void potrf_panels(const Exec& x, int uplo, int n, T* A, long lda, int* in
   if (lookahead) gemm_set_priority_stream(nullptr);
 }
 
+// Block order of a factorization with split products when the program sets
+// none.  A block is factored and inverted in FP64 (n^3 / 3 each at the FP64
+// rate, behind the chain of its leaves); the products between blocks run at the
+// split rate, less so with a shorter inner dimension.  Order 2048 against the
+// tile rule's half of n, DPOTRF, split BF16: n = 8192 7.4 against 8.6 ms,
+// 12288 15.4 against 21.4; against 1024: even at 8192, 16.4 at 12288; against
+// 3072: 8.0 and 16.4.
+// whole: refinement behind it, where a factor in one block saves more than
+// reduced products: solve with 8 right-hand sides, n = 4096 3.6 ms in one block
+// and 4.4 in two, 4500 4.5 and 5.1 in three, 5000 5.4 and 5.6, 6000 7.5 and 6.7.
+int split_potrf_order(int n, int nb, bool whole)
+{
+  if (whole && n <= 4608) return n;
+  return std::min(nb, 2048);
+}
+
 template <typename T>
 void dev_potrf(const Exec& x, int uplo, int n, T* A, long lda, int nb, int* info,
                const PotrfHooks<T>* hooks)
@@ -307,7 +323,8 @@ void dev_potrf(const Exec& x, int uplo, int n, T* A, long lda, int nb, int* info
     return;
   }
   // inverses of two consecutive diagonal blocks (ping-pong for lookahead)
-  T* inv = (T*)scratch(WS_INV, sizeof(T) * (size_t)2 * nb * nb);
+  const int ninv = nt > 1 ? 2 : 1;
+  T* inv = (T*)scratch(WS_INV, sizeof(T) * (size_t)ninv * nb * nb);
   const bool lookahead = x.s_diag != nullptr && nt > 1;
   hipStream_t sd = lookahead ? x.s_diag : x.s;
   // trailing updates of two panels at once (inner dimension 2 nb): longer
@@ -343,7 +360,7 @@ void dev_potrf(const Exec& x, int uplo, int n, T* A, long lda, int nb, int* info
   if (lookahead) gemm_set_priority_stream(sd);
   // the inverses' blocks above the diagonal are never written with nonzeros:
   // one fill here replaces a fill per recursion node
-  fill_zero<T>(sd, nb, 2 * nb, inv, nb);
+  fill_zero<T>(sd, nb, ninv * nb, inv, nb);
   // the diagonal keep_nb sub-blocks of block k's inverse are the inverses of
   // the factor's diagonal blocks of order keep_nb
   auto keep = [&](int k, const T* ik) {

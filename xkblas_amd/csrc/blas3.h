@@ -69,6 +69,9 @@ struct PotrfHooks {
 template <typename T>
 void dev_potrf(const Exec& x, int uplo, int n, T* A, long lda, int nb, int* info,
                const PotrfHooks<T>* hooks = nullptr);
+// nb of a dev_potrf with split products, of the tile rule's nb; whole: a solve
+// with refinement follows
+int split_potrf_order(int n, int nb, bool whole);
 // trailing updates of dev_potrf: 1 paired (default, also for -1), 0 one per panel
 void potrf_set_pairing(int v);
 

@@ -1518,7 +1518,8 @@ int potrf_async(const char* fn, int uplo, int N, T* A, int LDA)
   int* dinfo = r.d_info + rA->info_slot;
   fill_int(x.s, dinfo, 1, INT_MAX);
   r.prof_begin(sizeof(T) == 8 ? "potrf_f64" : "potrf_f32", (double)N * N * N / 3.0 + (double)N * N / 2.0 + N / 6.0);
-  dev_potrf<T>(x, uplo, N, (T*)rA->dev, rA->ldd, nb, dinfo);
+  const int order = r.nb || !split_enabled<T>(x) ? nb : split_potrf_order(N, nb, false);
+  dev_potrf<T>(x, uplo, N, (T*)rA->dev, rA->ldd, order, dinfo);
   r.prof_end();
   XK_HIP(hipMemcpyAsync(r.h_info + rA->info_slot, dinfo, sizeof(int), hipMemcpyDeviceToHost, x.s));
   r.mark_written(rA, 0, 0, N, N, uplo);
@@ -2216,8 +2217,9 @@ int xkblas_dposv_ir(int uplo, int N, int NRHS, const double* A, int LDA, const d
   xl.mode = XKBLAS_SPLIT_BF16_MATH;
   xl.nsplit = g_ir_moduli;
   r.prof_begin("posv_ir_f64", (double)N * N * N / 3.0 + 2.0 * N * N * (double)NRHS);
+  const int order = r.nb ? nb : split_potrf_order(N, nb, true);
   const int info = dev_posv_ir(x, xl, xf, uplo, N, NRHS, (const double*)rA->dev, rA->ldd, (const double*)rB->dev,
-                               rB->ldd, (double*)rX->dev, rX->ldd, nb, g_ir_itermax, iter);
+                               rB->ldd, (double*)rX->dev, rX->ldd, order, g_ir_itermax, iter);
   r.prof_end();
   r.mark_written(rX, 0, 0, N, NRHS, 0);
   return info;
