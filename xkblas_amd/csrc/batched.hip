@@ -10,14 +10,15 @@
 // launches on one stream: an int fill of the counter (no memset node, so the
 // pair can be captured in a hipGraph) and the persistent kernel.
 //
+// The first items go to the workgroups by position, the others from the counter.
 // GEMM tile: 4 waves, 2 x 2 of 32 x 32 quarters as 16 x 16 MFMA blocks
-// (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32), 16-deep k slices through
-// LDS, edges zero-filled.
+// (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32), 32-deep k slices through
+// LDS, rows beyond the matrix repeated, the end of the inner dimension zero.
 // TRSM panel (Left, Lower, NoTrans, Non-unit; B m x ncols with ncols <= 64),
 // left-looking over 64-row blocks: one MFMA tile forms alpha B_kb minus the
-// solved blocks' contribution straight into LDS, four 16-row sub-blocks are
-// solved with the solutions in registers (1 / L_ii precomputed), and the
-// block is written back for the next one, all inside the workgroup.
+// solved blocks' contribution straight into LDS, then each wave solves 16 of
+// the columns by itself, 16 rows at a time (rows in lanes, DPP), and the block
+// is written back for the next one, all inside the workgroup.
 // Shared memory is 40 KB per workgroup, so four fit on a CU.
 #include "common.h"
 #include "kernels.h"
@@ -59,12 +60,18 @@ template <typename T> struct BAcc;
 template <> struct BAcc<double> { typedef bd4 type; };
 template <> struct BAcc<float> { typedef bf4 type; };
 
-constexpr int TB_BM = 64, TB_BK = 16, TB_LD = TB_BM + 2;
+// Operands by pointers into global memory: a load through a pointer of unknown
+// kind also counts as an LDS access, and every wait for LDS data would wait
+// for the prefetched slices too.
+template <typename T> using GlobalC = const __attribute__((address_space(1))) T*;
+template <typename T> using Global = __attribute__((address_space(1))) T*;
+
+constexpr int TB_BM = 64, TB_BK = 32, TB_LD = TB_BM + 2;
 
 // Shared memory of one workgroup, in doubles: 40 KB, so that four
 // workgroups fit in the 160 KB of a CU.  Overlaid uses:
-//   GEMM staging  2 buffers x (A, B) x 16 x 66            4224
-//   TRSM          X block 64 x 64 (swizzled) + L strip 64 x 16   5120
+//   GEMM staging  (A, B) x 32 x 66                         4224
+//   TRSM          X block, 64 columns of 65                4160
 //   item index    one int at the start, between items
 constexpr int BATCH_SMEM = 5120;
 
@@ -78,94 +85,139 @@ __device__ __forceinline__ int item_tid()
   return t;
 }
 
+// A barrier for LDS data alone: loads from memory stay in flight over it.
+__device__ __forceinline__ void slice_barrier()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// One operand of a tile: this thread's elements of each 32-deep slice of op(A)
+// (`rows` of m) or op(B) (`rows` of n), by pointers that move on one slice at a
+// time.  along: the tile's rows are contiguous in memory, else the inner index
+// is.  Rows beyond the matrix repeat its last one: they only reach results that
+// are not stored.
+template <typename T, int TBM>
+struct SliceLoad {
+  static constexpr int V = TBM / 16, SH = TBM == 64 ? 6 : 5;  // V elements of each half of a slice
+  GlobalC<T> p[V];
+  T* lds;     // place of element 0
+  long step;  // half a slice
+  int k0;     // inner index of element 0
+  bool along;
+
+  __device__ __forceinline__ SliceLoad(GlobalC<T> A, long ld, bool along_, int row0, int rows, int tid, T* buf)
+      : along(along_)
+  {
+    const int i0 = along ? tid & (TBM - 1) : tid >> 4;
+    k0 = along ? tid >> SH : tid & 15;
+    step = along ? 16 * ld : 16;
+    lds = buf + k0 * TB_LD + i0;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const int i = min(row0 + i0 + (along ? 0 : 16 * v), rows - 1), k = k0 + (along ? 256 / TBM * v : 0);
+      p[v] = along ? A + i + (long)k * ld : A + k + (long)i * ld;
+    }
+  }
+  // the next slice; left: what is left of the inner dimension
+  __device__ __forceinline__ void load(T (&r)[2 * V], int left, GlobalC<T> A)
+  {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        GlobalC<T> q = p[v];
+        if (left < TB_BK) q = k0 + (along ? 256 / TBM * v : 0) + 16 * h < left ? q : A;
+        r[h * V + v] = *q;
+        p[v] += step;
+      }
+  }
+  __device__ __forceinline__ void store(const T (&r)[2 * V], int left) const
+  {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      T* d = lds + 16 * h * TB_LD;
+      if (left < TB_BK) {
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+          d[along ? 256 / TBM * v * TB_LD : 16 * v] =
+              k0 + (along ? 256 / TBM * v : 0) + 16 * h < left ? r[h * V + v] : T(0);
+      } else if (along) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) d[256 / TBM * v * TB_LD] = r[h * V + v];
+      } else {
+#pragma unroll
+        for (int v = 0; v < V; ++v) d[16 * v] = r[h * V + v];
+      }
+    }
+  }
+};
+
 // Main loop of the TBM x TBM tile (TBM = 64 or 32) at (m0, n0) of alpha
 // op(A) op(B): 4 waves as 2 x 2 quarters of TBM/2 x TBM/2, each TQ x TQ MFMA
-// blocks of 16 x 16 (TQ = TBM / 32); 16-deep k slices double-buffered in
-// LDS, the next slice prefetched into registers while the current one is
-// multiplied.  Ends with a barrier after the last LDS read, so the caller
-// may overwrite `smem` at once.
+// blocks of 16 x 16 (TQ = TBM / 32); one 32-deep k slice in LDS, the next in
+// flight to registers while it is multiplied.  Ends with a barrier after the
+// last LDS read, so the caller may overwrite `smem` at once.  A slice takes
+// 4.5k cycles alone, 2.0k of them products (FP64, 64 x 64); four workgroups of
+// a CU share the rest.  2048 products of order 512: FP64 49.6 TFLOP/s, 44.8
+// with 16-deep slices in two buffers and addresses formed for each element.
 template <typename T, int TBM>
-__device__ __forceinline__ void tile_mainloop(int ta, int tb, int M, int N, int K, const T* __restrict__ A, long lda,
-                                              const T* __restrict__ B, long ldb, int m0, int n0, T* smem,
+__device__ __forceinline__ void tile_mainloop(int ta, int tb, int M, int N, int K, GlobalC<T> A, long lda,
+                                              GlobalC<T> B, long ldb, int m0, int n0, T* smem,
                                               typename BAcc<T>::type (&acc)[TBM / 32][TBM / 32])
 {
-  constexpr int TQ = TBM / 32, WT = TBM / 2;
-  constexpr int V = TBM * TB_BK / 256;  // elements of each slice per thread
-  constexpr int SH = TBM == 64 ? 6 : 5;  // log2(TBM)
-  T(*As)[TB_BK][TB_LD] = reinterpret_cast<T(*)[TB_BK][TB_LD]>(smem);
-  T(*Bs)[TB_BK][TB_LD] = reinterpret_cast<T(*)[TB_BK][TB_LD]>(smem + 2 * TB_BK * TB_LD);
+  constexpr int TQ = TBM / 32, WT = TBM / 2, V = TBM / 16;
+  T* As = smem;
+  T* Bs = smem + TB_BK * TB_LD;
   typedef typename BAcc<T>::type acc_t;
   const int tid = item_tid(), lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
-  T ra[V], rb[V];
-  auto load = [&](int k0) {
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-      const int e = tid + 256 * v;  // 0 .. TBM * 16 - 1
-      // op(A) element (i, kk): i = e % TBM, kk = e / TBM (coalesced when !ta)
-      int i = e & (TBM - 1), kk = e >> SH;
-      if (ta) { kk = e & 15; i = e >> 4; }
-      const int gi = m0 + i, gk = k0 + kk;
-      T x = T(0);
-      if (gi < M && gk < K) x = ta ? A[gk + (long)gi * lda] : A[gi + (long)gk * lda];
-      ra[v] = x;
-      // op(B) element (kk, j)
-      int j = e >> 4, kb = e & 15;
-      if (tb) { j = e & (TBM - 1); kb = e >> SH; }
-      const int gj = n0 + j, gkb = k0 + kb;
-      T y = T(0);
-      if (gj < N && gkb < K) y = tb ? B[gj + (long)gkb * ldb] : B[gkb + (long)gj * ldb];
-      rb[v] = y;
-    }
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-      const int e = tid + 256 * v;
-      int i = e & (TBM - 1), kk = e >> SH;
-      if (ta) { kk = e & 15; i = e >> 4; }
-      As[buf][kk][i] = ra[v];
-      int j = e >> 4, kb = e & 15;
-      if (tb) { j = e & (TBM - 1); kb = e >> SH; }
-      Bs[buf][kb][j] = rb[v];
-    }
-  };
 #pragma unroll
   for (int i = 0; i < TQ; ++i)
 #pragma unroll
     for (int j = 0; j < TQ; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
-  const int nk = (K + TB_BK - 1) / TB_BK;
+  if (K <= 0) return;
   const int lr = lane & 15, lk = lane >> 4;
-  if (nk > 0) {
-    load(0);
-    store(0);
-    __syncthreads();
-    int buf = 0;
-    for (int kt = 0; kt < nk; ++kt) {
-      const bool more = kt + 1 < nk;
-      if (more) load((kt + 1) * TB_BK);
+  SliceLoad<T, TBM> la(A, lda, !ta, m0, M, tid, As), lb(B, ldb, tb, n0, N, tid, Bs);
+  const T* ar = As + lk * TB_LD + wm * WT + lr;
+  const T* br = Bs + lk * TB_LD + wn * WT + lr;
+  T ra[2 * V], rb[2 * V];
+  la.load(ra, K, A);
+  lb.load(rb, K, B);
+  for (int left = K; left > 0; left -= TB_BK) {
+    la.store(ra, left);
+    lb.store(rb, left);
+    slice_barrier();
+    if (left > TB_BK) {
+      la.load(ra, left - TB_BK, A);
+      lb.load(rb, left - TB_BK, B);
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int ks = 0; ks < TB_BK / 4; ++ks) {
+    for (int h = 0; h < 2; ++h) {
+      if (16 * h >= left) break;
+#pragma unroll
+      for (int ks = 4 * h; ks < 4 * h + 4; ++ks) {
         T af[TQ], bf[TQ];
 #pragma unroll
-        for (int i = 0; i < TQ; ++i) af[i] = As[buf][ks * 4 + lk][wm * WT + i * 16 + lr];
+        for (int i = 0; i < TQ; ++i) af[i] = ar[ks * 4 * TB_LD + i * 16];
 #pragma unroll
-        for (int j = 0; j < TQ; ++j) bf[j] = Bs[buf][ks * 4 + lk][wn * WT + j * 16 + lr];
+        for (int j = 0; j < TQ; ++j) bf[j] = br[ks * 4 * TB_LD + j * 16];
 #pragma unroll
         for (int i = 0; i < TQ; ++i)
 #pragma unroll
           for (int j = 0; j < TQ; ++j) acc[i][j] = bmfma(bf[j], af[i], acc[i][j]);
       }
-      if (more) store(buf ^ 1);
-      __syncthreads();
-      buf ^= 1;
     }
+    __builtin_amdgcn_sched_barrier(0);
+    slice_barrier();
   }
 }
 
 template <typename T>
-__device__ __forceinline__ void tile64_mainloop(int ta, int tb, int M, int N, int K, const T* __restrict__ A, long lda,
-                                                const T* __restrict__ B, long ldb, int m0, int n0, T* smem,
+__device__ __forceinline__ void tile64_mainloop(int ta, int tb, int M, int N, int K, GlobalC<T> A, long lda,
+                                                GlobalC<T> B, long ldb, int m0, int n0, T* smem,
                                                 typename BAcc<T>::type (&acc)[2][2])
 {
   tile_mainloop<T, 64>(ta, tb, M, N, K, A, lda, B, ldb, m0, n0, smem, acc);
@@ -186,137 +238,199 @@ __device__ __forceinline__ int tile_col(int wave, int lane, int j, int r)
 
 // C tile (tm, tn) of the TBM x TBM tiling of C <- alpha op(A) op(B) + beta C.
 template <typename T, int TBM>
-__device__ void gemm_tile(int ta, int tb, int M, int N, int K, T alpha, const T* __restrict__ A, long lda,
-                          const T* __restrict__ B, long ldb, T beta, T* __restrict__ C, long ldc, int tm, int tn,
-                          T* smem)
+__device__ void gemm_tile(int ta, int tb, int M, int N, int K, T alpha, GlobalC<T> A, long lda, GlobalC<T> B, long ldb,
+                          T beta, Global<T> C, long ldc, int tm, int tn, T* smem)
 {
   constexpr int TQ = TBM / 32;
   typename BAcc<T>::type acc[TQ][TQ];
   const int m0 = tm * TBM, n0 = tn * TBM;
   tile_mainloop<T, TBM>(ta, tb, M, N, K, A, lda, B, ldb, m0, n0, smem, acc);
   const int tid = item_tid(), lane = tid & 63, wave = tid >> 6;
+  // C is read whole before it is written: one wait for all, where a load and
+  // its use in turn behind each bounds test cost 16 memory latencies a tile
+  T c[TQ][TQ][4];
+  if (beta != T(0)) {
 #pragma unroll
-  for (int i = 0; i < TQ; ++i) {
-    const int gm = m0 + tile_row<T, TBM>(wave, lane, i);
-#pragma unroll
-    for (int j = 0; j < TQ; ++j) {
+    for (int j = 0; j < TQ; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int gn = n0 + tile_col<T, TBM>(wave, lane, j, r);
-        if (gm < M && gn < N) {
-          T* c = C + gm + (long)gn * ldc;
-          T v = alpha * acc[i][j][r];
-          if (beta != T(0)) v += beta * *c;
-          *c = v;
-        }
+        const GlobalC<T> q = C + (long)min(n0 + tile_col<T, TBM>(wave, lane, j, r), N - 1) * ldc;
+#pragma unroll
+        for (int i = 0; i < TQ; ++i) c[i][j][r] = q[min(m0 + tile_row<T, TBM>(wave, lane, i), M - 1)];
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < TQ; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int gn = n0 + tile_col<T, TBM>(wave, lane, j, r);
+#pragma unroll
+      for (int i = 0; i < TQ; ++i) {
+        const int gm = m0 + tile_row<T, TBM>(wave, lane, i);
+        T v = alpha * acc[i][j][r];
+        if (beta != T(0)) v += beta * c[i][j][r];
+        if (gm < M && gn < N) C[gm + (long)gn * ldc] = v;
       }
     }
+}
+
+// d += (y of lane J of this lane's row of 16 lanes) * m
+template <int J>
+__device__ __forceinline__ void fmac_row(double& d, double y, double m)
+{
+  asm volatile("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(d) : "v"(y), "v"(m), "n"(J));
+}
+template <int J>
+__device__ __forceinline__ void fmac_row(float& d, float y, float m)
+{
+  asm volatile("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(d) : "v"(y), "v"(m), "n"(J));
+}
+
+// L x = d for one 16 x 16 block of L: lane i of each row of 16 lanes holds row
+// i of -L (l; zero from the diagonal on), 1 / L(i, i) and row i of four columns
+// of d.  Row J of the solution is taken when it is complete: what the later
+// steps do to it (zero times an infinite solution) stays out.
+template <typename T, typename V, int J, int END>
+__device__ __forceinline__ void solve16(V& d, V& x, const T (&l)[16], T rinv, int i)
+{
+  if constexpr (J < END) {
+    V y;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) y[r] = d[r] * rinv;
+    // two wait states between a vector write and its DPP read: the compiler
+    // does not look into fmac_row, the selections stand between
+    asm volatile("" : "+v"(y));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[r] = i == J ? y[r] : x[r];
+    asm volatile("" : "+v"(x));
+    if constexpr (J < 15) {
+      const T m = l[J];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        T t = d[r];
+        fmac_row<J>(t, y[r], m);
+        d[r] = t;
+      }
+    }
+    solve16<T, V, J + 1, END>(d, x, l, rinv, i);
   }
 }
 
 // One 64-column panel of a lower-triangular solve L X = alpha B, in place,
 // left-looking over 64-row blocks kb:
-//   X_kb <- alpha B_kb - L[kb, 0:kb] X[0:kb]   one MFMA tile, k = 64 kb, into LDS
-//   X_kb <- L_kk^-1 X_kb                       in LDS, 16-row sub-blocks
+//   X_kb <- alpha B_kb - L[kb, 0:kb] X[0:kb]   one MFMA tile, into LDS
+//   X_kb <- L_kk^-1 X_kb                       16 columns a wave, no barriers
 //   X_kb -> global                             (read back by later blocks)
-// The X block lives in LDS as Xs[i * 64 + (c ^ i)] (row i, column c): rows
-// and columns are both conflict-free permutations of the banks.  L_kk's lower
-// triangle is read into registers before the block's GEMM and handed to LDS
-// one 16-column strip at a time: Ld[i * 16 + (q ^ (i & 15))] = L(i, 16 s + q),
-// with 1 / L(i, i) in place of the diagonal.  Per strip s, wave 0 (lane =
-// column) solves rows 16 s .. 16 s + 15 with the 16 solutions in registers,
-// then all four waves subtract their contribution from the rows below.
+// A wave takes its 64 x 16 part from LDS in the layout of four MFMA blocks and
+// goes down it in strips of 16 rows: solve16 on the strip, whose solutions then
+// reach the operand layout through their place in LDS, and one product for each
+// block below, with L from memory (requested half a strip ahead).
+// Bound by latency: a block takes 9.0k cycles per 64 of the inner dimension and
+// 24k besides (19k the strips).  Order 1024 with 64 columns alone: 636 us; with
+// one wave solving a strip of all columns for the others, three barriers a
+// strip, and B read one element after the other: 755 us.  Products by single
+// waves straight from memory, without LDS (each wave then loads what the four
+// now share): 550 us alone, but 1250 instead of 799 for 1024 solves.
 template <typename T>
 __device__ void trsm_panel(const BatchProblem& p, int panel, T* smem)
 {
-  const int m = p.m;
-  const int c0 = panel * 64;
-  const int nc = min(64, p.n - c0);
-  const T* L = reinterpret_cast<const T*>(p.A);
-  T* Bp = reinterpret_cast<T*>(p.C) + (long)c0 * p.ldc;
+  typedef typename BAcc<T>::type V;
+  constexpr int XLD = 65;
+  const int tid = item_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i = lane & 15, g = lane >> 4;
+  const int m = p.m, ncp = min(64, p.n - panel * 64), nc = ncp - wave * 16;
+  const GlobalC<T> L = (GlobalC<T>)(uintptr_t)p.A;
+  const Global<T> Bq = (Global<T>)(uintptr_t)p.C + (long)panel * 64 * p.ldc, Bp = Bq + (long)wave * 16 * p.ldc;
   const long ldl = p.lda, ldb = p.ldc;
   const T alpha = (T)p.alpha;
   T* Xs = smem;
-  T* Ld = smem + 64 * 64;
-  const int nb = (m + 63) / 64;
-  for (int kb = 0; kb < nb; ++kb) {
-    const int tid = item_tid(), lane = tid & 63, wave = tid >> 6;
-    const int r0 = kb * 64, h = min(64, m - r0);
-    // L_kk(lane, 4 v + wave), lower triangle; padding rows get a unit diagonal
-    T lreg[16];
+  T* Xt = smem + wave * 16 * XLD;
+  auto col = [&](int r) { return sizeof(T) == 8 ? g + 4 * r : 4 * g + r; };
+  for (int kb = 0; kb < m; kb += 64) {
+    // addresses are formed anew for each block and strip, not carried along
+    int r0 = kb;
+    asm volatile("" : "+s"(r0));
+    const int h = min(64, m - r0);
+    {
+      V t[2][2];
+      tile64_mainloop<T>(0, 0, h, ncp, r0, L + r0, ldl, Bq, ldb, 0, 0, smem, t);
+      T v[2][2][4];  // B, read whole as in gemm_tile
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int q = 4 * v + wave;
-      T x = T(0);
-      if (lane < h && q < lane) x = L[(r0 + lane) + (long)(r0 + q) * ldl];
-      else if (q == lane) x = lane < h ? L[(r0 + lane) + (long)(r0 + q) * ldl] : T(1);
-      lreg[v] = x;
-    }
-    typename BAcc<T>::type acc[2][2];
-    tile64_mainloop<T>(0, 0, h, nc, r0, L + r0, ldl, Bp, ldb, 0, 0, smem, acc);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = tile_row<T>(wave, lane, i);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int col = tile_col<T>(wave, lane, j, r);
-          T v = T(0);
-          if (row < h && col < nc) v = alpha * Bp[(r0 + row) + (long)col * ldb] - acc[i][j][r];
-          Xs[row * 64 + (col ^ row)] = v;
+          const GlobalC<T> q = Bq + r0 + (long)min(tile_col<T>(wave, lane, b, r), ncp - 1) * ldb;
+#pragma unroll
+          for (int a = 0; a < 2; ++a) v[a][b][r] = q[min(tile_row<T>(wave, lane, a), h - 1)];
         }
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const int row = tile_row<T>(wave, lane, a);
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int c = tile_col<T>(wave, lane, b, r);
+            Xs[c * XLD + row] = row < h && c < ncp ? alpha * v[a][b][r] - t[a][b][r] : T(0);
+          }
       }
     }
+    __syncthreads();
+    V acc[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      if (16 * s >= h) break;
-      // strip s of L_kk: this thread holds columns q = 4 v + wave, v = 4 s .. 4 s + 3
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[b][r] = Xs[(wave * 16 + col(r)) * XLD + 16 * b + i];
+    // strips of 16 rows; acc[0] is the strip's, acc[b] that of the b-th below
+#pragma unroll 1
+    for (int sb = 0; sb < h; sb += 16) {
+      int s = sb;
+      asm volatile("" : "+s"(s));
+      const int row = r0 + s + i;
+      const GlobalC<T> D = L + min(row, m - 1) + (long)(r0 + s) * ldl;
+      const int last = m - 1 - r0 - s;
+      T l[16], lu[3][4];
+#pragma unroll
+      for (int q = 0; q < 15; ++q) {
+        const T v = D[(long)min(q, last) * ldl];
+        l[q] = q < i && row < m ? -v : T(0);
+      }
+      const T diag = row < m ? D[(long)min(i, last) * ldl] : T(1);
+      V x = {0, 0, 0, 0};
+      const T rinv = T(1) / diag;
+      solve16<T, V, 0, 8>(acc[0], x, l, rinv, i);
+      __builtin_amdgcn_sched_barrier(0);
+      // L of the rows below; rows beyond m stay inside the column behind, which
+      // the columns of this strip have where a row is below, and blocks beyond
+      // h repeat the last one
+      const int below = (h - s - 1) >> 4;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int q = 4 * u + wave;  // column inside the strip
-        T x = lreg[4 * s + u];
-        if (16 * s + q == lane) x = T(1) / x;
-        Ld[lane * 16 + (q ^ (lane & 15))] = x;
+        const GlobalC<T> q = L + min(row, m - 1) + (long)min(r0 + s + 4 * u + g, m - 1) * ldl;
+#pragma unroll
+        for (int b = 0; b < 3; ++b) lu[b][u] = q[16 * min(b + 1, below)];
       }
-      __syncthreads();
-      if (wave == 0) {
-        const int c = lane;
-        T x[16];
+      __builtin_amdgcn_sched_barrier(0);
+      solve16<T, V, 8, 16>(acc[0], x, l, rinv, i);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) x[r] = Xs[(16 * s + r) * 64 + (c ^ (16 * s + r))];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const T* lrow = Ld + (16 * s + r) * 16;
-          T v = x[r];
-#pragma unroll
-          for (int q = 0; q < r; ++q) v -= lrow[q ^ r] * x[q];
-          x[r] = v * lrow[0];  // lrow[r ^ r] = 1 / L(r, r)
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) Xs[(16 * s + r) * 64 + (c ^ (16 * s + r))] = x[r];
+      for (int r = 0; r < 4; ++r) {
+        const int c = col(r);
+        if (row < m && c < nc) Bp[row + (long)c * ldb] = x[r];
+        Xt[c * XLD + s + i] = x[r];
       }
-      __syncthreads();
-      if (16 * (s + 1) < h) {
-        const int c = lane;
-        T xq[16];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      T xo[4];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) xq[q] = Xs[(16 * s + q) * 64 + (c ^ (16 * s + q))];
-        for (int i = 16 * (s + 1) + wave; i < h; i += 4) {
-          const T* lrow = Ld + i * 16;
-          T v = Xs[i * 64 + (c ^ i)];
+      for (int u = 0; u < 4; ++u) xo[u] = -Xt[i * XLD + s + 4 * u + g];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-          for (int q = 0; q < 16; ++q) v -= lrow[q ^ (i & 15)] * xq[q];
-          Xs[i * 64 + (c ^ i)] = v;
+      for (int b = 0; b < 3; ++b) {
+        acc[b] = acc[b + 1];
+        if (s + 16 * (b + 1) < h) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) acc[b] = bmfma(xo[u], lu[b][u], acc[b]);
         }
       }
-      __syncthreads();
-    }
-    // X_kb back to global memory, coalesced along rows
-#pragma unroll 4
-    for (int v = 0; v < 16; ++v) {
-      const int i = lane, c = wave + 4 * v;
-      if (i < h && c < nc) Bp[(r0 + i) + (long)c * ldb] = Xs[i * 64 + (c ^ i)];
     }
     __syncthreads();  // X_kb visible to the workgroup's next block; Xs free
   }
@@ -327,20 +441,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void b
 {
   __shared__ double smem_d[BATCH_SMEM];
   int* next = reinterpret_cast<int*>(smem_d);
-  for (;;) {
-    if (threadIdx.x == 0) *next = atomicAdd(counter, 1);
-    __syncthreads();
-    const int it = __builtin_amdgcn_readfirstlane(*next);
-    __syncthreads();
-    if (it >= nitems) return;
+  // The first items, the longest, go by position: workgroups c, c + 256, .. share
+  // a CU, so that each CU starts with one of the longest; by the counter, in
+  // the order of arrival, some start with several (1024 solves of order 32 ..
+  // 1024, FP64: 1018 us, now 799).
+  for (int it = blockIdx.x; it < nitems;) {
     const BatchItem w = items[it];
     const BatchProblem p = probs[w.prob];
     if (p.kind == 0) {
       const int ta = p.ta != NoTrans, tb = p.tb != NoTrans;
       if (p.dtype == 0) {
-        const double* A = reinterpret_cast<const double*>(p.A);
-        const double* B = reinterpret_cast<const double*>(p.B);
-        double* C = reinterpret_cast<double*>(p.C);
+        const GlobalC<double> A = (GlobalC<double>)(uintptr_t)p.A;
+        const GlobalC<double> B = (GlobalC<double>)(uintptr_t)p.B;
+        const Global<double> C = (Global<double>)(uintptr_t)p.C;
         if (w.tile == 32)
           gemm_tile<double, 32>(ta, tb, p.m, p.n, p.k, p.alpha, A, p.lda, B, p.ldb, p.beta, C, p.ldc, w.tm, w.tn,
                                 smem_d);
@@ -348,9 +461,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void b
           gemm_tile<double, 64>(ta, tb, p.m, p.n, p.k, p.alpha, A, p.lda, B, p.ldb, p.beta, C, p.ldc, w.tm, w.tn,
                                 smem_d);
       } else {
-        const float* A = reinterpret_cast<const float*>(p.A);
-        const float* B = reinterpret_cast<const float*>(p.B);
-        float* C = reinterpret_cast<float*>(p.C);
+        const GlobalC<float> A = (GlobalC<float>)(uintptr_t)p.A;
+        const GlobalC<float> B = (GlobalC<float>)(uintptr_t)p.B;
+        const Global<float> C = (Global<float>)(uintptr_t)p.C;
         float* sm = reinterpret_cast<float*>(smem_d);
         if (w.tile == 32)
           gemm_tile<float, 32>(ta, tb, p.m, p.n, p.k, (float)p.alpha, A, p.lda, B, p.ldb, (float)p.beta, C, p.ldc,
@@ -368,6 +481,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void b
       __builtin_amdgcn_s_setprio(0);
     }
     __syncthreads();  // smem free for the next item index
+    if (threadIdx.x == 0) *next = (int)gridDim.x + atomicAdd(counter, 1);
+    __syncthreads();
+    it = __builtin_amdgcn_readfirstlane(*next);
+    __syncthreads();
   }
 }
 
@@ -405,9 +522,10 @@ struct BatchCost {
 // covers at most 3/4 of the area the 64 x 64 one does (a small m or n), 2 =
 // 32 x 32 only, 3 = 64 x 64 only, 0 (default) = rule 1 for FP64 problems and
 // 64 x 64 for FP32 ones (XKBLAS_BATCH_TILE).  On the uneven batch of 4096
-// GEMMs + 1024 TRSMs (MI355X, best of five per run, four runs), FP64: per
-// problem 1.54-1.70 ms (mean 1.60) vs 64 x 64 1.56-1.80 (mean 1.70); FP32:
-// 64 x 64 1.06-1.10 vs per problem 1.13-1.14 ms.
+// GEMMs + 1024 TRSMs (MI355X, two draws of sizes), FP64: per problem 1342 and
+// 1407 us, 64 x 64 1312 and 1378, 32 x 32 1790 and 1846 (the documented default
+// stays, 2 % from the best); FP32: 64 x 64 857 and 896, per problem 923 and
+// 958, 32 x 32 1444 and 1489.
 static int g_batch_tile = getenv("XKBLAS_BATCH_TILE") ? atoi(getenv("XKBLAS_BATCH_TILE")) : 0;
 
 static int gemm_item_tile(int m, int n, int dtype)
