@@ -30,6 +30,49 @@
 
 namespace xk {
 
+enum { WS_SPLITK = 31 };
+
+// Parts of the inner dimension of a product with few tiles: the parts are
+// multiplied side by side (one launch, each into its own partial result) and
+// summed by a second pass over the result.  They fill the CUs that the tiles
+// leave idle and the last round, at the cost of that pass and of filling the
+// rings more often: no part under 600 of k, under 192 when even 64 x 64 tiles
+// leave four CUs of five without one (48); no parts of a k under 512, nor where
+// the tiles fill the chip by themselves (768: 2048^3 316 us in one part, 317 in
+// two).  The partial results stay under 2.5 times the operands.  FP64, us, one
+// part / by this rule: 4096 x 200 x 8192 375 / 276, 8192 x 64 x 4096 130 / 95,
+// 512^2 x 2048 55.6 / 34.5, 1500^2 x 3000 333 / 270, 300^2 x 4000 102 / 31,
+// 200^2 x 10000 246 / 44, 1000 x 100 x 1000 23.4 / 16.5; lower triangles 517 x
+// 1500 42.5 / 22, 2048 x 8192 860 / 587, 1500 x 2000 135 / 111; unchanged 512^3,
+// 1024^3.  Shorter chains of sums round less: relative error against an
+// extended product, uniform operands, 300 x 200 x 1500 1.3e-15 / 5.0e-16, 200^2
+// x 10000 3.4e-15 / 6.3e-16, triangle 517 x 1500 1.0e-15 / 2.5e-16.
+int gemm_k_parts(int m, int n, int k, int tri)
+{
+  const long a = (m + 63) / 64, b = (n + 63) / 64, t64 = tri == TRI_FULL ? a * b : a * (a + 1) / 2;
+  if (k < 512 || t64 >= 768 || gemm_get_tile() != 0) return 1;  // a set tile: one product as it is
+  const long most = std::max(8L, std::min(32L, 512 / t64));
+  return (int)std::max(1L, std::min(most, (long)k / (t64 <= 48 ? 192 : 600)));
+}
+
+// gemm, in parts of the inner dimension (0: by gemm_k_parts).  For the
+// library's compute stream: the partial results have one place.
+template <typename T>
+static void gemm_parts(hipStream_t s, int ta, int tb, int m, int n, int k, T alpha, const T* A, long lda, const T* B,
+                       long ldb, T beta, T* C, long ldc, int tri = TRI_FULL, int parts = 0)
+{
+  if (parts == 0) parts = gemm_k_parts(m, n, k, tri);
+  if (parts < 2 || n > 65535) {
+    gemm<T>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tri);
+    return;
+  }
+  const int kc = ((k + parts - 1) / parts + 31) / 32 * 32, np = (k + kc - 1) / kc;
+  T* W = (T*)scratch(WS_SPLITK, sizeof(T) * (size_t)np * m * n);
+  gemm<T>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, T(0), W, m, tri, np, ta != NoTrans ? (long)kc : (long)kc * lda,
+          tb != NoTrans ? (long)kc * ldb : (long)kc, (long)m * n, 0, kc);
+  splitk_reduce<T>(s, m, n, np, W, beta, C, ldc, tri);
+}
+
 template <typename T>
 void dev_gemm(const Exec& x, int transA, int transB, int m, int n, int k, T alpha, const T* A, long lda,
               const T* B, long ldb, T beta, T* C, long ldc)
@@ -39,7 +82,7 @@ void dev_gemm(const Exec& x, int transA, int transB, int m, int n, int k, T alph
     split_gemm<T>(x, transA, transB, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, TRI_FULL);
     return;
   }
-  gemm<T>(x.s, transA, transB, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+  gemm_parts<T>(x.s, transA, transB, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, TRI_FULL, x.parts);
 }
 
 template <typename T>
@@ -54,7 +97,7 @@ void dev_syrk(const Exec& x, int uplo, int trans, int n, int k, T alpha, const T
     split_gemm<T>(x, ta, tb, n, n, k, alpha, A, lda, A, lda, beta, C, ldc, tri);
     return;
   }
-  gemm<T>(x.s, ta, tb, n, n, k, alpha, A, lda, A, lda, beta, C, ldc, tri);
+  gemm_parts<T>(x.s, ta, tb, n, n, k, alpha, A, lda, A, lda, beta, C, ldc, tri);
 }
 
 // Split point of a recursive step: a multiple of 64 near n/2.
@@ -183,7 +226,7 @@ static void potrf_diag(hipStream_t s, int uplo, int n, T* A, long lda, T* Tinv, 
   inverse_levels<T>(s, uplo, NonUnit, n, A, lda, 0, Tinv, ldinv, 0, 1, wslot, false);
 }
 
-enum { WS_TRSM = 4, WS_TRSMW = 5, WS_SPLITK = 31 };
+enum { WS_TRSM = 4, WS_TRSMW = 5 };
 
 // Products with few output tiles and a long inner dimension (the inverse
 // products and late updates of a TRSM sweep with few right-hand sides) are
@@ -728,9 +771,14 @@ static void cgemm_impl(const Exec& x, int transA, int transB, int m, int n, int 
     const long ldp = rup(2L * n);
     T* P = (T*)scratch(WS_ZP, sizeof(T) * (size_t)ldp * n);
     const int opu = ta ? Trans : NoTrans, opv = tb ? NoTrans : Trans;
-    if (one_launch) {
-      gemm<T>(x.s, opu, opv, n, n, 2 * k, T(1), U, ldu, V1, ldv, T(0), P, ldp, uplo == Lower ? TRI_LOWER : TRI_UPPER,
-              2, 0, (long)vsz, (long)n);
+    const int tri = uplo == Lower ? TRI_LOWER : TRI_UPPER;
+    if (one_launch && gemm_k_parts(n, n, 2 * k, tri) > 1) {
+      // parts fill the rounds better: n = 2048, k = 4096 1.50 -> 1.18 ms
+      gemm_parts<T>(x.s, opu, opv, n, n, 2 * k, T(1), U, ldu, V1, ldv, T(0), P, ldp, tri);
+      gemm_parts<T>(x.s, opu, opv, n, n, 2 * k, T(1), U, ldu, V2, ldv, T(0), P + n, ldp, tri);
+    } else if (one_launch) {
+      gemm<T>(x.s, opu, opv, n, n, 2 * k, T(1), U, ldu, V1, ldv, T(0), P, ldp, tri, 2, 0,
+              (long)vsz, (long)n);
     } else {
       dev_gemmt<T>(x, uplo, opu, opv, n, 2 * k, T(1), U, ldu, V1, same ? ldu : ldv, T(0), P, ldp);
       dev_gemmt<T>(x, uplo, opu, opv, n, 2 * k, T(1), U, ldu, V2, ldv, T(0), P + n, ldp);

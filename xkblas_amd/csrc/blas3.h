@@ -22,11 +22,15 @@ struct Exec {
   hipStream_t s_diag; // side stream for latency-bound diagonal-block work
   int mode;           // xkblas_mode_math_t
   int nsplit;         // CRT moduli for split modes (0 = automatic)
+  int parts = 0;      // of the inner dimension in dev_gemm: 0 by gemm_k_parts
   hipEvent_t ev0 = nullptr, ev1 = nullptr;  // POTRF's stream-ordering events (created per call when null)
 };
 
 // Scratch slots of dev_potrf.
 enum { WS_DIAG0 = 0, WS_DIAG1 = 1, WS_PANEL = 2, WS_INV = 3 };
+
+// parts of the inner dimension of a product (1: none)
+int gemm_k_parts(int m, int n, int k, int tri);
 
 template <typename T>
 void dev_gemm(const Exec& x, int transA, int transB, int m, int n, int k, T alpha, const T* A, long lda,

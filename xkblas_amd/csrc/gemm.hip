@@ -55,6 +55,7 @@ struct GemmParams {
   int trap;        // triangle-masked output that is not square: full tile raster, tiles outside it leave at once
   int whole;       // tiles of gemm_dma_mixed_kernel's first part
   int kmode;       // inner range per tile for a triangular operand (KRANGE_*)
+  int kpart;       // > 0: batch entry z multiplies the z-th kpart of the inner dimension
   int vecA, vecB;  // 16-byte vector loads allowed (base and ld aligned)
   int prio;        // raise the waves' issue priority (latency-bound chain steps)
   T alpha, beta;
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams<T> p)
   const T* __restrict__ B = p.B + (long)blockIdx.z * p.sB;
   T* __restrict__ C = p.C + (long)blockIdx.z * p.sC;
 
-  const int M = p.m, N = p.n, K = p.k;
+  const int M = p.m, N = p.n, K = p.kpart ? min(p.kpart, p.k - (int)blockIdx.z * p.kpart) : p.k;
   int m0, n0;
   if (!tile_origin<BM, BN>(p, m0, n0)) return;
 
@@ -344,7 +345,7 @@ __device__ __forceinline__ void dma_tile_body(const GemmParams<T>& p, char* S, i
   const T* __restrict__ A = p.A + (long)blockIdx.z * p.sA;
   const T* __restrict__ B = p.B + (long)blockIdx.z * p.sB;
   T* __restrict__ C = p.C + (long)blockIdx.z * p.sC;
-  const int M = p.m, N = p.n, K = p.k;
+  const int M = p.m, N = p.n, K = p.kpart ? min(p.kpart, p.k - (int)blockIdx.z * p.kpart) : p.k;
 
   // block permutation of k-major row k: rows that the lanes of one read take
   // together (k .. k + 3) fall into different banks
@@ -626,13 +627,13 @@ template int gemm_tile_of<float>(int, int, int);
 
 template <typename T>
 void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, const T* A, long lda,
-          const T* B, long ldb, T beta, T* C, long ldc, int tri, int batch, long sA, long sB, long sC, int kmode)
+          const T* B, long ldb, T beta, T* C, long ldc, int tri, int batch, long sA, long sB, long sC, int kmode, int kpart)
 {
   if (m <= 0 || n <= 0 || batch <= 0) return;
   if (tri != TRI_FULL)
     XK_CHECK(tri == TRI_LOWER ? m >= n : n >= m, "triangular gemm output must hold its whole diagonal");
   GemmParams<T> p;
-  p.m = m; p.n = n; p.k = k; p.tri = tri; p.kmode = kmode;
+  p.m = m; p.n = n; p.k = k; p.tri = tri; p.kmode = kmode; p.kpart = kpart;
   p.trap = tri != TRI_FULL && m != n;
   p.alpha = alpha; p.beta = beta;
   p.A = A; p.lda = lda; p.sA = sA;
@@ -654,7 +655,7 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, c
   const bool dma = p.vecA && p.vecB && lda < (1L << 21) && ldb < (1L << 21);
   if (dma) {
     bool mixed = false;
-    if (bm == 0) bm = dma_tile<T>(tiles(128), tiles(64), k, batch == 1 && kmode == KRANGE_ALL, mixed);
+    if (bm == 0) bm = dma_tile<T>(tiles(128), tiles(64), kpart ? kpart : k, batch == 1 && kmode == KRANGE_ALL, mixed);
     if (bm == 128 && mixed) {
       launch_mixed<T>(s, ta, tb, p, (int)(tiles(128) / 512 * 512), tiles(128));
       return;
@@ -682,8 +683,8 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, c
 }
 
 template void gemm<double>(hipStream_t, int, int, int, int, int, double, const double*, long, const double*, long,
-                           double, double*, long, int, int, long, long, long, int);
+                           double, double*, long, int, int, long, long, long, int, int);
 template void gemm<float>(hipStream_t, int, int, int, int, int, float, const float*, long, const float*, long,
-                          float, float*, long, int, int, long, long, long, int);
+                          float, float*, long, int, int, long, long, long, int, int);
 
 }  // namespace xk

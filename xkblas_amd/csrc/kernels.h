@@ -18,7 +18,7 @@ namespace xk {
 template <typename T>
 void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha,
           const T* A, long lda, const T* B, long ldb, T beta, T* C, long ldc,
-          int tri = TRI_FULL, int batch = 1, long sA = 0, long sB = 0, long sC = 0, int kmode = 0);
+          int tri = TRI_FULL, int batch = 1, long sA = 0, long sB = 0, long sC = 0, int kmode = 0, int kpart = 0);
 
 // The tile gemm() takes for a product with aligned operands.
 template <typename T>
@@ -64,7 +64,7 @@ void zero_triangle(hipStream_t s, int uplo, int n, T* A, long lda);
 // C <- beta C + sum over `parts` of the m x n partial products W (leading
 // dimension m, one every m n elements); beta == 0 never reads C.
 template <typename T>
-void splitk_reduce(hipStream_t s, int m, int n, int parts, const T* W, T beta, T* C, long ldc);
+void splitk_reduce(hipStream_t s, int m, int n, int parts, const T* W, T beta, T* C, long ldc, int tri = TRI_FULL);
 
 // Fill an int array with a value (stream-ordered, graph-capturable).
 void fill_int(hipStream_t s, int* p, int n, int v);

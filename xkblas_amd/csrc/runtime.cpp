@@ -1391,6 +1391,7 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
     if (split) split_cache_register((const double*)rB->dev, rB->ldd, N, K, transB != NoTrans);
     std::vector<Replica::PanelEvent> pev;
     r.prof_begin(sizeof(T) == 8 ? "gemm_f64" : "gemm_f32", flops);
+    x.parts = gemm_k_parts(M, N, K, TRI_FULL);  // the whole product's: the same bits by both ways
     int r0 = 0;
     for (int end : ends) {
       const int rows = end - r0;
