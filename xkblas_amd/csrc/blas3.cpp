@@ -269,12 +269,15 @@ static int g_potrf_pair = getenv("XKBLAS_POTRF_PAIR") ? (atoi(getenv("XKBLAS_POT
 static int potrf_pairing() { return g_potrf_pair; }
 void potrf_set_pairing(int v) { g_potrf_pair = v < 0 ? 1 : (v ? 1 : 0); }
 
-// Width of the block columns of potrf_panels: one block column while the
-// trailing products are shorter than the chain anyway (order 517: 0.20 ms
-// against 0.27 with two streams, 1024: 0.38 against 0.45), then 512 (order
-// 2048 / 8192 / 16384: 0.94 / 7.04 / 35.2 ms; 256: 0.99 / 7.26 / 37.4;
-// 1024: 0.92 / 7.13 / 35.3; FP32 order 8192: 4.92, 5.05, 5.17 ms).
-static int panel_width(int n) { return n <= 1024 ? n : 512; }
+// Width of the block columns of potrf_panels: one block column, whose updates
+// follow its panels on one stream, as long as a second stream costs more (events,
+// leaves that wait for room beside the trailing update) than its overlap gives:
+// one / columns of 512 on two streams, FP64 lower, order 1100 0.370 / 0.470 ms,
+// 2048 0.726 / 0.849, 3072 1.22 / 1.35, 4096 1.87 / 1.94, 4608 2.30 / 2.34, 6144
+// 3.80 / 3.71; FP32 2048 0.590 / 0.717, 4608 1.73 / 1.82.  Then 512: widths 384 to
+// 1024 are within 2 % of each other at 8192, 12288 and 16384 (6.2, 14.8, 30.2 ms),
+// and one last block column of the last 3072 or 4096 orders gives no more.
+static int panel_width(int n) { return n <= 4608 ? n : 512; }
 
 // Blocked Cholesky in the MFMA modes: block columns of panel_width(n) factored
 // over their whole height on the side stream (potrf_columns), beside the
