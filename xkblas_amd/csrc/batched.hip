@@ -15,10 +15,10 @@
 // (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32), 32-deep k slices through
 // LDS, rows beyond the matrix repeated, the end of the inner dimension zero.
 // TRSM panel (Left, Lower, NoTrans, Non-unit; B m x ncols with ncols <= 64),
-// left-looking over 64-row blocks: one MFMA tile forms alpha B_kb minus the
-// solved blocks' contribution straight into LDS, then each wave solves 16 of
-// the columns by itself, 16 rows at a time (rows in lanes, DPP), and the block
-// is written back for the next one, all inside the workgroup.
+// left-looking over 64-row blocks: one MFMA tile, 16 columns a wave, forms alpha
+// B_kb minus the solved blocks' contribution, then each wave solves its columns
+// by itself, 16 rows at a time (rows in lanes, DPP), and the block is written
+// back for the next one, all inside the workgroup.
 // Shared memory is 40 KB per workgroup, so four fit on a CU.
 #include "common.h"
 #include "kernels.h"
@@ -71,7 +71,7 @@ constexpr int TB_BM = 64, TB_BK = 32, TB_LD = TB_BM + 2;
 // Shared memory of one workgroup, in doubles: 40 KB, so that four
 // workgroups fit in the 160 KB of a CU.  Overlaid uses:
 //   GEMM staging  (A, B) x 32 x 66                         4224
-//   TRSM          X block, 64 columns of 65                4160
+//   TRSM          L_kk, 10 tiles of 256, and 4 x 16 columns of 17   3648
 //   item index    one int at the start, between items
 constexpr int BATCH_SMEM = 5120;
 
@@ -155,33 +155,33 @@ struct SliceLoad {
 };
 
 // Main loop of the TBM x TBM tile (TBM = 64 or 32) at (m0, n0) of alpha
-// op(A) op(B): 4 waves as 2 x 2 quarters of TBM/2 x TBM/2, each TQ x TQ MFMA
-// blocks of 16 x 16 (TQ = TBM / 32); one 32-deep k slice in LDS, the next in
+// op(A) op(B): 4 waves as 2 x 2 quarters of TBM/2 x TBM/2, or (TI = 4, TJ = 1)
+// as four strips of 16 columns, each TI x TJ MFMA blocks of 16 x 16; one 32-deep k slice in LDS, the next in
 // flight to registers while it is multiplied.  Ends with a barrier after the
 // last LDS read, so the caller may overwrite `smem` at once.  A slice takes
 // 4.5k cycles alone, 2.0k of them products (FP64, 64 x 64); four workgroups of
 // a CU share the rest.  2048 products of order 512: FP64 49.6 TFLOP/s, 44.8
 // with 16-deep slices in two buffers and addresses formed for each element.
-template <typename T, int TBM>
+template <typename T, int TBM, int TI = TBM / 32, int TJ = TBM / 32>
 __device__ __forceinline__ void tile_mainloop(int ta, int tb, int M, int N, int K, GlobalC<T> A, long lda,
                                               GlobalC<T> B, long ldb, int m0, int n0, T* smem,
-                                              typename BAcc<T>::type (&acc)[TBM / 32][TBM / 32])
+                                              typename BAcc<T>::type (&acc)[TI][TJ])
 {
-  constexpr int TQ = TBM / 32, WT = TBM / 2, V = TBM / 16;
+  constexpr int V = TBM / 16;
   T* As = smem;
   T* Bs = smem + TB_BK * TB_LD;
   typedef typename BAcc<T>::type acc_t;
   const int tid = item_tid(), lane = tid & 63, wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = TJ == 1 && TBM == 64 ? 0 : wave & 1, wn = TJ == 1 && TBM == 64 ? wave : wave >> 1;
 #pragma unroll
-  for (int i = 0; i < TQ; ++i)
+  for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int j = 0; j < TQ; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    for (int j = 0; j < TJ; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
   if (K <= 0) return;
   const int lr = lane & 15, lk = lane >> 4;
   SliceLoad<T, TBM> la(A, lda, !ta, m0, M, tid, As), lb(B, ldb, tb, n0, N, tid, Bs);
-  const T* ar = As + lk * TB_LD + wm * WT + lr;
-  const T* br = Bs + lk * TB_LD + wn * WT + lr;
+  const T* ar = As + lk * TB_LD + wm * 16 * TI + lr;
+  const T* br = Bs + lk * TB_LD + wn * 16 * TJ + lr;
   T ra[2 * V], rb[2 * V];
   la.load(ra, K, A);
   lb.load(rb, K, B);
@@ -199,28 +199,20 @@ __device__ __forceinline__ void tile_mainloop(int ta, int tb, int M, int N, int 
       if (16 * h >= left) break;
 #pragma unroll
       for (int ks = 4 * h; ks < 4 * h + 4; ++ks) {
-        T af[TQ], bf[TQ];
+        T af[TI], bf[TJ];
 #pragma unroll
-        for (int i = 0; i < TQ; ++i) af[i] = ar[ks * 4 * TB_LD + i * 16];
+        for (int i = 0; i < TI; ++i) af[i] = ar[ks * 4 * TB_LD + i * 16];
 #pragma unroll
-        for (int j = 0; j < TQ; ++j) bf[j] = br[ks * 4 * TB_LD + j * 16];
+        for (int j = 0; j < TJ; ++j) bf[j] = br[ks * 4 * TB_LD + j * 16];
 #pragma unroll
-        for (int i = 0; i < TQ; ++i)
+        for (int i = 0; i < TI; ++i)
 #pragma unroll
-          for (int j = 0; j < TQ; ++j) acc[i][j] = bmfma(bf[j], af[i], acc[i][j]);
+          for (int j = 0; j < TJ; ++j) acc[i][j] = bmfma(bf[j], af[i], acc[i][j]);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
     slice_barrier();
   }
-}
-
-template <typename T>
-__device__ __forceinline__ void tile64_mainloop(int ta, int tb, int M, int N, int K, GlobalC<T> A, long lda,
-                                                GlobalC<T> B, long ldb, int m0, int n0, T* smem,
-                                                typename BAcc<T>::type (&acc)[2][2])
-{
-  tile_mainloop<T, 64>(ta, tb, M, N, K, A, lda, B, ldb, m0, n0, smem, acc);
 }
 
 // Tile element of accumulator register r of block (i, j) held by `lane`:
@@ -317,25 +309,25 @@ __device__ __forceinline__ void solve16(V& d, V& x, const T (&l)[16], T rinv, in
 }
 
 // One 64-column panel of a lower-triangular solve L X = alpha B, in place,
-// left-looking over 64-row blocks kb:
-//   X_kb <- alpha B_kb - L[kb, 0:kb] X[0:kb]   one MFMA tile, into LDS
-//   X_kb <- L_kk^-1 X_kb                       16 columns a wave, no barriers
+// left-looking over 64-row blocks kb, 16 columns a wave:
+//   X_kb <- alpha B_kb - L[kb, 0:kb] X[0:kb]   four MFMA blocks a wave
+//   X_kb <- L_kk^-1 X_kb                       L_kk in LDS, no barriers
 //   X_kb -> global                             (read back by later blocks)
-// A wave takes its 64 x 16 part from LDS in the layout of four MFMA blocks and
-// goes down it in strips of 16 rows: solve16 on the strip, whose solutions then
-// reach the operand layout through their place in LDS, and one product for each
-// block below, with L from memory (requested half a strip ahead).
-// Bound by latency: a block takes 9.0k cycles per 64 of the inner dimension and
-// 24k besides (19k the strips).  Order 1024 with 64 columns alone: 636 us; with
-// one wave solving a strip of all columns for the others, three barriers a
-// strip, and B read one element after the other: 755 us.  Products by single
-// waves straight from memory, without LDS (each wave then loads what the four
-// now share): 550 us alone, but 1250 instead of 799 for 1024 solves.
+// A wave goes down its 64 x 16 part in strips of 16 rows: solve16 on the strip,
+// whose solutions reach the operand layout through LDS, and one product for each
+// block below.
+// Bound by latency.  Order 1024 with 64 columns alone: 566 us; with the products
+// in quarters of 32 x 32, redistributed through LDS, and each strip's part of L
+// from memory: 636; with one wave solving a strip of all columns for the others,
+// three barriers a strip, and B read one element after the other: 755.  1024
+// solves of order 32 to 1024: 739, 799 and 1406 us.  Products by single waves
+// straight from memory, without LDS (each wave then loads what the four now
+// share): 550 us alone, but 1250 for the 1024 solves.
 template <typename T>
 __device__ void trsm_panel(const BatchProblem& p, int panel, T* smem)
 {
   typedef typename BAcc<T>::type V;
-  constexpr int XLD = 65;
+  constexpr int XLD = 17;
   const int tid = item_tid(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 15, g = lane >> 4;
   const int m = p.m, ncp = min(64, p.n - panel * 64), nc = ncp - wave * 16;
@@ -343,96 +335,78 @@ __device__ void trsm_panel(const BatchProblem& p, int panel, T* smem)
   const Global<T> Bq = (Global<T>)(uintptr_t)p.C + (long)panel * 64 * p.ldc, Bp = Bq + (long)wave * 16 * p.ldc;
   const long ldl = p.lda, ldb = p.ldc;
   const T alpha = (T)p.alpha;
-  T* Xs = smem;
-  T* Xt = smem + wave * 16 * XLD;
+  T* Ls = smem;                             // tiles (a, b), b <= a, of L_kk by columns
+  T* Xt = smem + 2560 + wave * 16 * XLD;    // a strip's solution, for its transpose
   auto col = [&](int r) { return sizeof(T) == 8 ? g + 4 * r : 4 * g + r; };
   for (int kb = 0; kb < m; kb += 64) {
     // addresses are formed anew for each block and strip, not carried along
     int r0 = kb;
     asm volatile("" : "+s"(r0));
     const int h = min(64, m - r0);
-    {
-      V t[2][2];
-      tile64_mainloop<T>(0, 0, h, ncp, r0, L + r0, ldl, Bq, ldb, 0, 0, smem, t);
-      T v[2][2][4];  // B, read whole as in gemm_tile
+    V acc[4][1];
+    tile_mainloop<T, 64, 4, 1>(0, 0, h, ncp, r0, L + r0, ldl, Bq, ldb, 0, 0, smem, acc);
+    // L_kk to LDS, the diagonal's reciprocals in its place; rows and columns
+    // beyond m repeat the last: what they reach is not stored (a tile row at a
+    // time: all ten tiles in flight take the registers of the products)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+    for (int a = 0; a < 4; ++a) {
+      if (16 * a >= h) break;
+      const int ti = tid & 15, q = tid >> 4;
+      const GlobalC<T> Lr = L + min(r0 + 16 * a + ti, m - 1);
+      T x[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const GlobalC<T> q = Bq + r0 + (long)min(tile_col<T>(wave, lane, b, r), ncp - 1) * ldb;
+      for (int b = 0; b <= a; ++b) x[b] = Lr[(long)min(r0 + 16 * b + q, m - 1) * ldl];
+      if (ti == q) x[a] = T(1) / x[a];
 #pragma unroll
-          for (int a = 0; a < 2; ++a) v[a][b][r] = q[min(tile_row<T>(wave, lane, a), h - 1)];
-        }
+      for (int b = 0; b <= a; ++b) Ls[(a * (a + 1) / 2 + b) * 256 + q * 16 + ti] = x[b];
+    }
+    if (nc > 0) {
 #pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        const int row = tile_row<T>(wave, lane, a);
+      for (int r = 0; r < 4; ++r) {
+        const GlobalC<T> q = Bp + r0 + (long)min(col(r), nc - 1) * ldb;
+        T v[4];
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < 4; ++b) v[b] = q[min(16 * b + i, h - 1)];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int c = tile_col<T>(wave, lane, b, r);
-            Xs[c * XLD + row] = row < h && c < ncp ? alpha * v[a][b][r] - t[a][b][r] : T(0);
-          }
+        for (int b = 0; b < 4; ++b) acc[b][0][r] = 16 * b + i < h && col(r) < nc ? alpha * v[b] - acc[b][0][r] : T(0);
       }
     }
     __syncthreads();
-    V acc[4];
+    if (nc > 0) {
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+      for (int s = 0; s < 4; ++s) {
+        if (16 * s >= h) break;
+        const T* D = Ls + (s * (s + 1) / 2 + s) * 256;
+        T l[16];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[b][r] = Xs[(wave * 16 + col(r)) * XLD + 16 * b + i];
-    // strips of 16 rows; acc[0] is the strip's, acc[b] that of the b-th below
-#pragma unroll 1
-    for (int sb = 0; sb < h; sb += 16) {
-      int s = sb;
-      asm volatile("" : "+s"(s));
-      const int row = r0 + s + i;
-      const GlobalC<T> D = L + min(row, m - 1) + (long)(r0 + s) * ldl;
-      const int last = m - 1 - r0 - s;
-      T l[16], lu[3][4];
+        for (int q = 0; q < 16; ++q) {
+          const T v = D[q * 16 + i];
+          l[q] = q < i ? -v : T(0);
+        }
+        V x = {0, 0, 0, 0};
+        solve16<T, V, 0, 16>(acc[s][0], x, l, D[17 * i], i);
+        const int row = r0 + 16 * s + i;
 #pragma unroll
-      for (int q = 0; q < 15; ++q) {
-        const T v = D[(long)min(q, last) * ldl];
-        l[q] = q < i && row < m ? -v : T(0);
-      }
-      const T diag = row < m ? D[(long)min(i, last) * ldl] : T(1);
-      V x = {0, 0, 0, 0};
-      const T rinv = T(1) / diag;
-      solve16<T, V, 0, 8>(acc[0], x, l, rinv, i);
-      __builtin_amdgcn_sched_barrier(0);
-      // L of the rows below; rows beyond m stay inside the column behind, which
-      // the columns of this strip have where a row is below, and blocks beyond
-      // h repeat the last one
-      const int below = (h - s - 1) >> 4;
+        for (int r = 0; r < 4; ++r) {
+          const int c = col(r);
+          if (row < m && c < nc) Bp[row + (long)c * ldb] = x[r];
+          Xt[c * XLD + i] = x[r];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        T xo[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const GlobalC<T> q = L + min(row, m - 1) + (long)min(r0 + s + 4 * u + g, m - 1) * ldl;
+        for (int u = 0; u < 4; ++u) xo[u] = -Xt[i * XLD + 4 * u + g];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-        for (int b = 0; b < 3; ++b) lu[b][u] = q[16 * min(b + 1, below)];
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      solve16<T, V, 8, 16>(acc[0], x, l, rinv, i);
+        for (int b = s + 1; b < 4; ++b) {
+          if (16 * b >= h) break;
+          const T* E = Ls + (b * (b + 1) / 2 + s) * 256;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int c = col(r);
-        if (row < m && c < nc) Bp[row + (long)c * ldb] = x[r];
-        Xt[c * XLD + s + i] = x[r];
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      T xo[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) xo[u] = -Xt[i * XLD + s + 4 * u + g];
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-      for (int b = 0; b < 3; ++b) {
-        acc[b] = acc[b + 1];
-        if (s + 16 * (b + 1) < h) {
-#pragma unroll
-          for (int u = 0; u < 4; ++u) acc[b] = bmfma(xo[u], lu[b][u], acc[b]);
+          for (int u = 0; u < 4; ++u) acc[b][0] = bmfma(xo[u], E[(4 * u + g) * 16 + i], acc[b][0]);
         }
       }
     }
-    __syncthreads();  // X_kb visible to the workgroup's next block; Xs free
+    __syncthreads();  // X_kb visible to the workgroup's next block; Ls free
   }
 }
 
@@ -444,7 +418,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void b
   // The first items, the longest, go by position: workgroups c, c + 256, .. share
   // a CU, so that each CU starts with one of the longest; by the counter, in
   // the order of arrival, some start with several (1024 solves of order 32 ..
-  // 1024, FP64: 1018 us, now 799).
+  // 1024, FP64: 1018 us, then 799).
   for (int it = blockIdx.x; it < nitems;) {
     const BatchItem w = items[it];
     const BatchProblem p = probs[w.prob];
