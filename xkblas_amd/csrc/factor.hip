@@ -247,6 +247,9 @@ __device__ __forceinline__ T factor16(T (&d)[16], T (&l)[16], int i)
 }
 
 // Row i = lane % 16 of a lower triangular tile in l[]; y[c] = inv(L)(i, c).
+// Rows up to j keep their value in step j (a product by zero would not: row j
+// of a singular tile is infinite, and zero times that would reach the rows
+// above, whose solutions are finite).
 template <typename T>
 __device__ __forceinline__ void invert16(const T (&l)[16], T (&y)[16], int i, T rdiag)
 {
@@ -259,7 +262,8 @@ __device__ __forceinline__ void invert16(const T (&l)[16], T (&y)[16], int i, T 
     for_each<j + 1>([&](auto cc) {
       constexpr int c = decltype(cc)::value;
       y[c] = i == j ? y[c] * rdiag : y[c];
-      y[c] = fma(-m, row_bcast<j>(y[c]), y[c]);
+      const T below = fma(-m, row_bcast<j>(y[c]), y[c]);
+      y[c] = i > j ? below : y[c];
     });
   });
 }
