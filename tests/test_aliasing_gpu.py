@@ -117,3 +117,27 @@ def test_potrf_info_beyond_initial_slots(xk):
     finally:
         xk.invalidate()
     assert got == want
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("routine", ["gemm", "hemm"])
+def test_complex_product_into_its_operand(xk, routine, dtype):
+    """C <- A C with C given as both B and C (real scalars), in many rounds of
+    tiles: B is read before C is written.  Bar: |C - ref| <= 4 (k + 8) eps |A| |B|."""
+    n, m = 1500, 1700
+    r = rng(19)
+
+    def mat(rows, cols):
+        return np.asfortranarray((r.uniform(-1, 1, (rows, cols)) + 1j * r.uniform(-1, 1, (rows, cols))).astype(dtype))
+
+    A, B = mat(n, n), mat(n, m)
+    C = B.copy(order="F")
+    if routine == "gemm":
+        xk.gemm(N_, N_, 1.0, A, C, 0.0, C)
+    else:
+        A = np.asfortranarray(A + A.conj().T)
+        xk.hemm(141, 122, 1.0, A, C, 0.0, C)
+    xk.invalidate()
+    X, Y = A.astype(np.complex128), B.astype(np.complex128)
+    bar = 4 * (n + 8) * np.finfo(dtype).eps * (np.abs(X) @ np.abs(Y))
+    assert np.all(np.abs(C - X @ Y) <= bar)

@@ -789,12 +789,15 @@ static void cgemm_impl(const Exec& x, int transA, int transB, int m, int n, int 
     cplx_combine<T>(x.s, m, n, P, ldp, alpha, beta, C, ldc, uplo, herm);
     return;
   }
-  if (alpha[1] == T(0) && beta[1] == T(0)) {
+  if (alpha[1] == T(0) && beta[1] == T(0) && (B != C || transB != NoTrans)) {
     // real scalars: op(B) and C as they lie in memory, real with twice the
     // rows; rho(A) (Trans: rho(conj A)) read transposed for a transposed op,
     // a transposed B dealt into real and imaginary columns.  One pass over A
     // and the product, instead of two passes, the product and a pass over C
-    // (ZGEMM 4096 x 200 x 4096 0.95 -> 0.69 ms, 512 x 200 x 512 0.050 -> 0.035)
+    // (ZGEMM 4096 x 200 x 4096 0.95 -> 0.69 ms, 512 x 200 x 512 0.050 -> 0.035).
+    // Not for a product into its own operand B, which the tiles of C would
+    // overwrite under the tiles that still read it: the packed form below
+    // reads B before C is written.
     const bool ta = transA != NoTrans, tb = transB != NoTrans;
     const int ar = ta ? k : m, ac = ta ? m : k;
     const long ldya = rup(2L * ar);
