@@ -106,3 +106,23 @@ def test_last_round_of_a_triangle_in_quarters(xk, uplo):
     assert np.array_equal(out[0], out[1])
     assert np.all((np.triu(out[0], 1) if uplo == 122 else np.tril(out[0], -1))[np.triu_indices(4070, 1) if uplo == 122
                   else np.tril_indices(4070, -1)] == 7)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("ta,tb", OPS)
+def test_ring_ends_in_a_remainder_of_any_size(xk, ta, tb, dtype):
+    """The ring of four stages behind 2 to 9 whole ones, with remainders that leave
+    some waves nothing to load in the last: exact on integers."""
+    M, N = 901, 1030
+    r = rng(3)
+    xk.lib().xkblas_set_gemm_tile(32)
+    try:
+        for K in (33, 49, 50, 52, 63, 64, 65, 97, 100, 113, 127, 129, 145, 161, 289):
+            A = small_int(r, *((M, K) if ta == 111 else (K, M)), dtype=dtype)
+            B = small_int(r, *((K, N) if tb == 111 else (N, K)), dtype=dtype)
+            C = np.full((M, N), np.nan, dtype=dtype, order="F")
+            xk.gemm(ta, tb, 1.0, A, B, 0.0, C)
+            xk.invalidate()
+            assert np.array_equal(C, (A if ta == 111 else A.T) @ (B if tb == 111 else B.T)), K
+    finally:
+        xk.lib().xkblas_set_gemm_tile(0)
