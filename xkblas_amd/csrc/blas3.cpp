@@ -59,11 +59,11 @@ int gemm_k_parts(int m, int n, int k, int tri)
 // library's compute stream: the partial results have one place.
 template <typename T>
 static void gemm_parts(hipStream_t s, int ta, int tb, int m, int n, int k, T alpha, const T* A, long lda, const T* B,
-                       long ldb, T beta, T* C, long ldc, int tri = TRI_FULL, int parts = 0)
+                       long ldb, T beta, T* C, long ldc, int tri = TRI_FULL, int parts = 0, int tile = 0)
 {
   if (parts == 0) parts = gemm_k_parts(m, n, k, tri);
   if (parts < 2 || n > 65535) {
-    gemm<T>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tri);
+    gemm<T>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, tri, 1, 0, 0, 0, 0, 0, tile);
     return;
   }
   const int kc = ((k + parts - 1) / parts + 31) / 32 * 32, np = (k + kc - 1) / kc;
@@ -82,7 +82,7 @@ void dev_gemm(const Exec& x, int transA, int transB, int m, int n, int k, T alph
     split_gemm<T>(x, transA, transB, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, TRI_FULL);
     return;
   }
-  gemm_parts<T>(x.s, transA, transB, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, TRI_FULL, x.parts);
+  gemm_parts<T>(x.s, transA, transB, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, TRI_FULL, x.parts, x.tile);
 }
 
 template <typename T>

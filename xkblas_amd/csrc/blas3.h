@@ -23,6 +23,7 @@ struct Exec {
   int mode;           // xkblas_mode_math_t
   int nsplit;         // CRT moduli for split modes (0 = automatic)
   int parts = 0;      // of the inner dimension in dev_gemm: 0 by gemm_k_parts
+  int tile = 0;       // of dev_gemm in the MFMA modes: 0 by gemm's own rule
   hipEvent_t ev0 = nullptr, ev1 = nullptr;  // POTRF's stream-ordering events (created per call when null)
 };
 

@@ -612,7 +612,7 @@ static void launch_mixed(hipStream_t s, bool ta, bool tb, GemmParams<T>& p, int 
 // 64.4 / 64.9.  (With registers between memory and LDS, tiles as now: 8192^3
 // 58.5, 4096^3 51.6, 1024^3 31.4, 512^3 12.8; FP32 133, 111, 47.7, 11.0.)
 template <typename T>
-static int dma_tile(long t128, long t64, int k, bool may_mix, bool& mixed)
+static int dma_tile(long t128, long t64, int k, bool may_mix, bool& mixed, double* us = nullptr)
 {
   mixed = false;
   if (t64 < (sizeof(T) == 8 ? 512 : 256)) return 32;
@@ -626,24 +626,26 @@ static int dma_tile(long t128, long t64, int k, bool may_mix, bool& mixed)
     mixed = may_mix && quarters < plain;
     last = mixed ? quarters : plain;
   }
-  const double c128 = (w128 + last) * 512 * 128 * 128 * (k + 150.0);
-  const double c64 = (w64 + (f64 == 0 ? 0 : 0.5 + 0.5 * f64)) * 1280 * 64 * 64 * (k + 57.0);
-  return c128 / (sizeof(T) == 8 ? 70.5 : 136.0) < c64 / (sizeof(T) == 8 ? 66.0 : 120.0) ? 128 : 64;
+  const double c128 = (w128 + last) * 512 * 128 * 128 * (k + 150.0) / (sizeof(T) == 8 ? 35.25e6 : 68e6);
+  const double c64 = (w64 + (f64 == 0 ? 0 : 0.5 + 0.5 * f64)) * 1280 * 64 * 64 * (k + 57.0) / (sizeof(T) == 8 ? 33e6 : 60e6);
+  if (us) *us = std::min(c128, c64);
+  return c128 < c64 ? 128 : 64;
 }
 
 template <typename T>
-int gemm_tile_of(int m, int n, int k)
+int gemm_tile_of(int m, int n, int k, double* us)
 {
   auto tiles = [&](int t) { return (long)((m + t - 1) / t) * ((n + t - 1) / t); };
   bool mixed;
-  return dma_tile<T>(tiles(128), tiles(64), k, true, mixed);
+  return dma_tile<T>(tiles(128), tiles(64), k, true, mixed, us);
 }
-template int gemm_tile_of<double>(int, int, int);
-template int gemm_tile_of<float>(int, int, int);
+template int gemm_tile_of<double>(int, int, int, double*);
+template int gemm_tile_of<float>(int, int, int, double*);
 
 template <typename T>
 void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, const T* A, long lda,
-          const T* B, long ldb, T beta, T* C, long ldc, int tri, int batch, long sA, long sB, long sC, int kmode, int kpart)
+          const T* B, long ldb, T beta, T* C, long ldc, int tri, int batch, long sA, long sB, long sC, int kmode, int kpart,
+          int tile)
 {
   if (m <= 0 || n <= 0 || batch <= 0) return;
   if (tri != TRI_FULL)
@@ -671,7 +673,10 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, c
   const bool dma = p.vecA && p.vecB && lda < (1L << 21) && ldb < (1L << 21);
   if (dma) {
     bool mixed = false;
-    if (bm == 0) bm = dma_tile<T>(tiles(128), tiles(64), kpart ? kpart : k, batch == 1 && kmode == KRANGE_ALL, mixed);
+    if (bm == 0) {
+      bm = dma_tile<T>(tiles(128), tiles(64), kpart ? kpart : k, batch == 1 && kmode == KRANGE_ALL, mixed);
+      if (tile) bm = tile;
+    }
     if (bm == 128 && mixed) {
       launch_mixed<T>(s, ta, tb, p, (int)(tiles(128) / 512 * 512), tiles(128));
       return;
@@ -699,8 +704,8 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, c
 }
 
 template void gemm<double>(hipStream_t, int, int, int, int, int, double, const double*, long, const double*, long,
-                           double, double*, long, int, int, long, long, long, int, int);
+                           double, double*, long, int, int, long, long, long, int, int, int);
 template void gemm<float>(hipStream_t, int, int, int, int, int, float, const float*, long, const float*, long,
-                          float, float*, long, int, int, long, long, long, int, int);
+                          float, float*, long, int, int, long, long, long, int, int, int);
 
 }  // namespace xk

@@ -18,11 +18,13 @@ namespace xk {
 template <typename T>
 void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha,
           const T* A, long lda, const T* B, long ldb, T beta, T* C, long ldc,
-          int tri = TRI_FULL, int batch = 1, long sA = 0, long sB = 0, long sC = 0, int kmode = 0, int kpart = 0);
+          int tri = TRI_FULL, int batch = 1, long sA = 0, long sB = 0, long sC = 0, int kmode = 0, int kpart = 0,
+          int tile = 0);
 
-// The tile gemm() takes for a product with aligned operands.
+// The tile gemm() takes for a product with aligned operands, and about how
+// long the product runs (unless with 32 x 32 tiles).
 template <typename T>
-int gemm_tile_of(int m, int n, int k);
+int gemm_tile_of(int m, int n, int k, double* us);
 
 // Forces the macro-tile shape of gemm(): 0 = automatic, 32, 64
 // or 128.

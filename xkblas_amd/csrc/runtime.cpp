@@ -1294,6 +1294,7 @@ std::vector<int> result_panels(int M, int N, int K, size_t elt, int planes)
     }
     for (int e = width; width && e < N; e += width) ends.push_back(e);
   } else {
+    if (gemm_k_parts(M, N, K, TRI_FULL) > 1) return ends;  // in one launch: the partial results have one place
     const int tm = (M + 127) / 128, tn = (N + 127) / 128;
     const double us = 2.0 * M * N * K / (elt == 8 ? 62e6 : 118e6);
     const int per = std::max({1, (300 + tm / 2) / tm, (tn + 11) / 12, (int)(tn * 250.0 / us)}), first = std::max(1, per / 2);
@@ -1360,8 +1361,9 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
   }
   if (!ends.empty() && resident) {
     if (split) split_cache_register((const double*)rA->dev, rA->ldd, M, K, rowsA);
+    x.parts = 1;  // the whole product's, like the tile
+    if (!split) x.tile = gemm_tile_of<T>(M, N, K, nullptr);
     Exec xs[2] = {x, x};  // the panels go in turn to two streams
-    const int old_tile = gemm_get_tile();
     std::vector<Replica::PanelEvent> pev;
     r.before_compute();
     r.prof_begin(sizeof(T) == 8 ? "gemm_f64" : "gemm_f32", flops);
@@ -1369,7 +1371,6 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
       xs[1].s = r.s_diag;
       XK_HIP(hipEventRecord(r.ev_pot0, x.s));
       XK_HIP(hipStreamWaitEvent(xs[1].s, r.ev_pot0, 0));
-      if (!old_tile) gemm_set_tile(gemm_tile_of<T>(M, N, K));  // the whole product's
     }
     int j0 = 0;
     for (size_t p = 0; p < ends.size(); ++p) {
@@ -1383,7 +1384,6 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
       j0 = ends[p];
     }
     if (!split) {
-      gemm_set_tile(old_tile);
       const size_t odd = (pev.size() & ~(size_t)1) - 1;  // the last panel of the other stream
       XK_HIP(hipStreamWaitEvent(x.s, pev[odd].ev, 0));
     }
