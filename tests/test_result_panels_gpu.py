@@ -1,6 +1,7 @@
 """Products of resident operands in column panels and in one launch: the same
-bits where the panels must not be taken (parts of the inner dimension, whose
-partial results have one place)."""
+bits, at sizes where the panels are taken (several rounds over the chip, a last
+panel of another tile) and where they must not be (parts of the inner dimension,
+whose partial results have one place)."""
 import numpy as np
 import pytest
 
@@ -14,6 +15,9 @@ def _mat(r, m, n, dtype):
 
 
 @pytest.mark.parametrize("dtype,mode,op,m,n,k,beta", [
+    (np.float64, 0, "NN", 4100, 4200, 2600, -0.5), (np.float64, 0, "TT", 5003, 3001, 4003, 0.0),
+    (np.float32, 0, "NT", 6000, 6100, 3000, -0.5), (np.float32, 0, "TN", 4096, 4100, 1500, 0.0),
+    (np.float64, 3, "NT", 8192, 5400, 3000, -0.5),
     (np.float64, 0, "NN", 15411, 158, 8000, 0.0), (np.float64, 0, "TT", 15411, 158, 3000, -0.5)])
 def test_panels_equal_one_launch(xk, dtype, mode, op, m, n, k, beta):
     r = rng(m + k)

@@ -25,6 +25,10 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha,
 // long the product runs (unless with 32 x 32 tiles).
 template <typename T>
 int gemm_tile_of(int m, int n, int k, double* us);
+// Time of a full round over the chip of tiles of 128 x 128 (512 of them) or 64
+// x 64 (1280).
+template <typename T>
+double gemm_round_us(int tile, int k);
 
 // Forces the macro-tile shape of gemm(): 0 = automatic, 32, 64
 // or 128.

@@ -1260,49 +1260,94 @@ bool pipeline_enabled()
 // Column panels (their last columns + 1) in which a product of resident
 // operands runs so that each panel can go back to the host while the next ones
 // are computed; empty: in one launch.  A large result takes a good part of the
-// product's own time to copy (57 GB/s measured: 2.1 ms beside the 4.4 ms of an
-// FP64 5003 x 3001 x 9011, 38 ms beside the 98 ms of a split-BF16 16384^3);
+// product's own time to copy (57 GB/s measured: 2.1 ms beside the 4.2 ms of an
+// FP64 5003 x 3001 x 9011, 38 ms beside the 86 ms of a split-BF16 16384^3);
 // columns, because whole columns copy at that rate (9 KB pieces of 32 KB
 // columns at half of it).
-// MFMA modes: panels of about 300 tiles of 128 x 128 (0.6 of what the chip
-// holds) and 250 us, the first of half that, dealt in turn to two streams: two
-// panels, out of step, are in flight at any time, so that few CUs wait for a
-// panel's last tiles.  With the copy (one launch / panels): FP64 4096^3 4.67 /
-// 3.54 ms, 5003 x 3001 x 9011 7.22 / 5.57, 8192 x 8192 x 2000 14.0 / 10.2; a
-// caller who leaves the result on the device: 1.99 / 2.55, 4.53 / 4.65, 3.88 /
-// 4.04 ms (panels of 520 tiles 2.01, 4.66, 3.92, with the copy 4.00, 6.67, 10.1).
-// Split modes (planes): the count up to 8 with the shortest product (by rounds of
-// 256 x 256 tiles over the 256 CUs, 6 % more at most) and last copy.  BF16, with
-// the copy / left on the device, one launch and panels: 4843 x 7959 x 7432 14.3 and
-// 9.9 / 7.7 and 8.0 ms, 6000 x 5000 x 4000 8.5 and 6.0 / 3.6 and 3.9.
-std::vector<int> result_panels(int M, int N, int K, size_t elt, int planes)
+// Nothing says yet whether the result will be copied, so the panels may cost a
+// caller who leaves it on the device little, and are taken where the copied
+// result is there a tenth earlier: all but the last panel end where whole rounds
+// of the product's tiles over the chip do, at most 1.5 % of their places empty.
+// MFMA modes: rounds of 512 tiles of 128 or 1280 of 64 (`tile`; the last panel
+// takes its own).  A boundary, where the chip drains, costs 12 us with two
+// workgroups on a CU (128) and a tenth of a round more with five (64); 5 % in all.
+// One launch / panels, left on the device and copied back: FP64 4096^3 1.96 / 1.98
+// and 4.41 / 3.40 ms, 5003 x 3001 x 9011 4.15 / 4.32 and 6.37 / 5.02, 8192 x 8192 x
+// 2000 3.85 / 3.89 and 13.4 / 10.0; FP32 4096 x 4100 x 8192 2.18 / 2.23 and 3.45 /
+// 2.87.  (On two streams, in panels of 300 tiles, 2.6 ms left on the device for
+// 4096^3 and 1.9 instead of 1.4 for 3300 x 3300 x 4000.)
+// Split modes: rounds of 256 tiles of 256 over all planes.  A boundary costs up to
+// a round where the rounds end exactly (8192^3 BF16 0.1 ms) and two elsewhere
+// (4843 x 7959 x 7432 in two panels 6.46 -> 6.86 ms); 1 % in all.
+// BF16, as above: 16384^3 85.3 / 85.6 and 123.9 / 92.5; FP8 97.5 / 97.9 and 137.5 /
+// 101.1; smaller products in one launch.  (By rounds up to 6 % more, 4096^3 left on
+// the device took 1.91 ms instead of 1.71, 2430 x 2059 x 1300 0.48 instead of 0.38.)
+template <typename T>
+std::vector<int> result_panels(int M, int N, int K, int planes, int& tile)
 {
   std::vector<int> ends;
-  if ((double)M * N * elt < 17e6) return ends;  // 0.3 ms
+  tile = 0;
+  if ((double)M * N * sizeof(T) < 17e6) return ends;  // 0.3 ms
+  double us = 0;  // of the product in one launch
+  int bm = 256, places = 256;
   if (planes) {
-    auto rounds = [&](int n) { return (int)(((long)((M + 255) / 256) * ((n + 255) / 256) * planes + 255) / 256); };
-    const double prod = 2.0 * M * N * K * planes / (planes > 13 ? 2.7e15 : 1.15e15), copy = 8.0 * M * N / 57e9;
-    double best = prod + copy;
-    int width = 0;
-    for (int p = 8; p >= 2; --p) {
-      const int h = (N / p + 255) / 256 * 256;
-      const double more = (double)((N + h - 1) / h) * rounds(h) / rounds(N), t = prod * more + copy * h / N;
-      if (h < N && more <= 1.06 && t < best) {
-        best = t;
-        width = h;
+    us = 2.0 * M * N * K * planes / (planes > 13 ? 2.7e9 : 1.15e9);
+  } else {
+    if (gemm_get_tile() != 0 || gemm_k_parts(M, N, K, TRI_FULL) > 1) return ends;
+    bm = gemm_tile_of<T>(M, N, K, &us);
+    if (bm == 32) return ends;
+    places = bm == 128 ? 512 : 1280;
+  }
+  const int tn = (N + bm - 1) / bm;
+  const long column = (long)((M + bm - 1) / bm) * std::max(planes, 1);  // places of a column of tiles
+  const long rounds = column * tn / places, step = std::max(1L, rounds / 16);
+  std::vector<int> at{0};  // ends, in columns of tiles
+  double boundary = bm == 64 ? 12 + 0.1 * gemm_round_us<T>(64, K) : 12;
+  for (int exact = planes != 0; exact >= 0 && at.size() == 1; --exact) {
+    if (planes) boundary = us / std::max(1L, rounds) * (exact ? 1.0 : 2.0);
+    for (long q = step; q <= rounds && at.size() < 20; ++q) {
+      const long c = q * places / column;
+      if (c <= at.back() || c >= tn || (exact ? c * column != q * places : c * column * 1.015 < (double)q * places)) continue;
+      at.push_back((int)c);
+      q += step - 1;
+    }
+  }
+  const double may = planes ? 0.0105 : 0.05;
+  const int most = std::min(4, 1 + (int)(may * us / boundary)), cnt = (int)at.size();
+  if (most < 2 || cnt < 2) return ends;
+  // when the product is over up to an end
+  std::vector<double> over(cnt);
+  for (int i = 0; i < cnt; ++i)
+    over[i] = planes ? us * at[i] / tn : (at[i] * column + places - 1) / places * gemm_round_us<T>(bm, K);
+  const double copy = (double)M * bm * sizeof(T) / 57e3;
+  // back[p][i]: when p panels up to at[i] are copied
+  std::vector<std::vector<double>> back(most, std::vector<double>(cnt, 1e300));
+  std::vector<std::vector<int>> from(most, std::vector<int>(cnt, 0));
+  back[0][0] = 0;
+  double best = 0.9 * (us + copy * tn);
+  int panels = 0, last = 0;
+  for (int p = 1; p < most; ++p)
+    for (int i = 1; i < cnt; ++i) {
+      for (int h = 0; h < i; ++h) {
+        const double end = std::max(back[p - 1][h], over[i] + (p - 1) * boundary) + copy * (at[i] - at[h]);
+        if (end < back[p][i]) {
+          back[p][i] = end;
+          from[p][i] = h;
+        }
+      }
+      double rest = us - over[i];
+      if (!planes && gemm_tile_of<T>(M, N - at[i] * bm, K, &rest) == 32) continue;
+      const double prod = over[i] + rest + p * boundary, end = std::max(back[p][i], prod) + copy * (tn - at[i]);
+      if (end < best && prod <= (1 + may) * us) {
+        best = end;
+        panels = p;
+        last = i;
       }
     }
-    for (int e = width; width && e < N; e += width) ends.push_back(e);
-  } else {
-    if (gemm_k_parts(M, N, K, TRI_FULL) > 1) return ends;  // in one launch: the partial results have one place
-    const int tm = (M + 127) / 128, tn = (N + 127) / 128;
-    const double us = 2.0 * M * N * K / (elt == 8 ? 62e6 : 118e6);
-    const int per = std::max({1, (300 + tm / 2) / tm, (tn + 11) / 12, (int)(tn * 250.0 / us)}), first = std::max(1, per / 2);
-    const int cnt = (tn - first + per / 2) / per;
-    if (cnt < 1) return ends;
-    for (int i = 0; i < cnt; ++i) ends.push_back(128 * (first + (int)((long)(tn - first) * i / cnt)));
-  }
-  if (!ends.empty()) ends.push_back(N);
+  if (panels == 0) return ends;
+  for (int p = panels, i = last; p >= 1; i = from[p--][i]) ends.insert(ends.begin(), at[i] * bm);
+  ends.push_back(N);
+  if (!planes) tile = bm;
   return ends;
 }
 
@@ -1353,7 +1398,7 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
     resident = r.all_valid(rA, 0, 0, Am, An) && r.all_valid(rB, 0, 0, Bm, Bn) &&
                (!readC || r.all_valid(rC, 0, 0, M, N));
     if (resident) {
-      ends = result_panels(M, N, K, sizeof(T), split ? split_plane_count(K, x.nsplit, x.mode == XKBLAS_SPLIT_FP8_MATH) : 0);
+      ends = result_panels<T>(M, N, K, split ? split_plane_count(K, x.nsplit, x.mode == XKBLAS_SPLIT_FP8_MATH) : 0, x.tile);
     } else if (M > nb && (!r.all_valid(rA, 0, 0, Am, An) || (readC && !r.all_valid(rC, 0, 0, M, N)))) {
       for (int e = nb; e < M; e += nb) ends.push_back(e);
       ends.push_back(M);
@@ -1361,31 +1406,21 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
   }
   if (!ends.empty() && resident) {
     if (split) split_cache_register((const double*)rA->dev, rA->ldd, M, K, rowsA);
-    x.parts = 1;  // the whole product's, like the tile
-    if (!split) x.tile = gemm_tile_of<T>(M, N, K, nullptr);
-    Exec xs[2] = {x, x};  // the panels go in turn to two streams
     std::vector<Replica::PanelEvent> pev;
     r.before_compute();
     r.prof_begin(sizeof(T) == 8 ? "gemm_f64" : "gemm_f32", flops);
-    if (!split) {
-      xs[1].s = r.s_diag;
-      XK_HIP(hipEventRecord(r.ev_pot0, x.s));
-      XK_HIP(hipStreamWaitEvent(xs[1].s, r.ev_pot0, 0));
-    }
+    x.parts = 1;  // the whole product's
     int j0 = 0;
-    for (size_t p = 0; p < ends.size(); ++p) {
+    for (int end : ends) {
+      if (end == N) x.tile = 0;
       const T* Bp = (const T*)rB->dev + (transB == NoTrans ? (long)j0 * rB->ldd : (long)j0);
-      dev_gemm<T>(xs[p & 1], transA, transB, M, ends[p] - j0, K, *alpha, (const T*)rA->dev, rA->ldd, Bp, rB->ldd,
-                  *beta, (T*)rC->dev + (long)j0 * rC->ldd, rC->ldd);
+      dev_gemm<T>(x, transA, transB, M, end - j0, K, *alpha, (const T*)rA->dev, rA->ldd, Bp, rB->ldd, *beta,
+                  (T*)rC->dev + (long)j0 * rC->ldd, rC->ldd);
       hipEvent_t ev;
       XK_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-      XK_HIP(hipEventRecord(ev, xs[p & 1].s));
-      pev.push_back(Replica::PanelEvent{ends[p], ev});
-      j0 = ends[p];
-    }
-    if (!split) {
-      const size_t odd = (pev.size() & ~(size_t)1) - 1;  // the last panel of the other stream
-      XK_HIP(hipStreamWaitEvent(x.s, pev[odd].ev, 0));
+      XK_HIP(hipEventRecord(ev, x.s));
+      pev.push_back(Replica::PanelEvent{end, ev});
+      j0 = end;
     }
     r.prof_end();
     if (split) split_cache_clear();
