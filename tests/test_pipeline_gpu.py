@@ -115,3 +115,31 @@ def test_resident_product_in_panels_equals_one_launch(xk, ta, tb, mode, dtype):
         L.xkblas_set_param(0, 0)
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+def test_copies_back_of_short_and_long_calls(xk):
+    """Results of short calls (copied back behind the whole stream) and long ones
+    (behind their own event), with calls of the other kind between and a mirror
+    written by both in turn: exact on integers."""
+    n = 2400
+    r = rng(8)
+    A = np.asfortranarray(r.integers(-2, 3, (n, n)).astype(np.float64))
+    a = np.asfortranarray(r.integers(-2, 3, (n, 20)).astype(np.float64))
+    long_, short = A @ A, a @ a.T
+    C, D, E = (np.zeros((n, n), order="F") for _ in range(3))
+    for _ in range(3):
+        xk.gemm(N_, T_, 1.0, a, a, 0.0, C, sync=False)   # short
+        xk.gemm(N_, N_, 1.0, A, A, 0.0, D, sync=False)   # long
+        xk.gemm(N_, T_, 1.0, a, a, 0.0, E, sync=False)
+        xk.coherent(C)
+        assert np.array_equal(C, short)
+        xk.gemm(N_, N_, 1.0, A, A, 1.0, E, sync=False)   # the same mirror, long
+        xk.coherent(D)
+        assert np.array_equal(D, long_)
+        xk.gemm(N_, T_, 1.0, a, a, 1.0, E, sync=False)   # and short
+        xk.gemm(N_, N_, 1.0, A, A, 0.0, C, sync=False)
+        xk.coherent(E)
+        xk.coherent(C)
+        assert np.array_equal(E, long_ + 2 * short)
+        assert np.array_equal(C, long_)
+    xk.invalidate()

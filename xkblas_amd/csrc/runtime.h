@@ -43,7 +43,7 @@ struct Replica {
   bool panel_cols = false;
   // The last write of the mirror is complete with `written` on the compute
   // stream once `stamped`; before that, with whatever the stream holds now.
-  // The event is recorded only when another call follows the write.
+  // The event is recorded only when another call follows a long one's write.
   hipEvent_t written = nullptr;
   bool stamped = false;
 };
@@ -84,7 +84,8 @@ struct Runtime {
   hipEvent_t ev_comp = nullptr, ev_h2d = nullptr, ev_d2h = nullptr;
   hipEvent_t ev_pot0 = nullptr, ev_pot1 = nullptr;  // POTRF's lookahead ordering
   bool pending_h2d = false, pending_d2h = false;
-  std::vector<Replica*> unstamped;  // mirrors written by the last call on the compute stream
+  std::vector<Replica*> unstamped;  // mirrors written by the last call on the compute stream, if it was a long one
+  double call_flops = 0;            // of the running call
 
   std::unordered_map<const void*, Replica*> map;
   size_t cache_used = 0, cache_limit = 0;
