@@ -1290,14 +1290,18 @@ bool pipeline_enabled()
 // 101.1; smaller products in one launch.  (By rounds up to 6 % more, 4096^3 left on
 // the device took 1.91 ms instead of 1.71, 2430 x 2059 x 1300 0.48 instead of 0.38.)
 template <typename T>
-std::vector<int> result_panels(int M, int N, int K, int planes, int& tile)
+std::vector<int> result_panels(const Exec& x, int M, int N, int K, bool split, int& tile)
 {
   std::vector<int> ends;
   tile = 0;
   if ((double)M * N * sizeof(T) < 17e6) return ends;  // 0.3 ms
   double us = 0;  // of the product in one launch
-  int bm = 256, places = 256;
-  if (planes) {
+  int bm = 256, places = 256, planes = 0;
+  if (split) {
+    // fewer than 96 rounds of any count of moduli: the count takes 5 us of host time
+    const bool fp8 = x.mode == XKBLAS_SPLIT_FP8_MATH;
+    if ((long)((M + 255) / 256) * ((N + 255) / 256) * (fp8 ? 38 : 13) < 96 * 256) return ends;
+    planes = split_plane_count(K, x.nsplit, fp8);
     us = 2.0 * M * N * K * planes / (planes > 13 ? 2.7e9 : 1.15e9);
   } else {
     if (gemm_get_tile() != 0 || gemm_k_parts(M, N, K, TRI_FULL) > 1) return ends;
@@ -1405,7 +1409,7 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
     resident = r.all_valid(rA, 0, 0, Am, An) && r.all_valid(rB, 0, 0, Bm, Bn) &&
                (!readC || r.all_valid(rC, 0, 0, M, N));
     if (resident) {
-      ends = result_panels<T>(M, N, K, split ? split_plane_count(K, x.nsplit, x.mode == XKBLAS_SPLIT_FP8_MATH) : 0, x.tile);
+      ends = result_panels<T>(x, M, N, K, split, x.tile);
     } else if (M > nb && (!r.all_valid(rA, 0, 0, Am, An) || (readC && !r.all_valid(rC, 0, 0, M, N)))) {
       for (int e = nb; e < M; e += nb) ends.push_back(e);
       ends.push_back(M);
