@@ -1276,8 +1276,9 @@ bool pipeline_enabled()
 // result is there a tenth earlier: all but the last panel end where whole rounds
 // of the product's tiles over the chip do, at most 1.5 % of their places empty.
 // MFMA modes: rounds of 512 tiles of 128 or 1280 of 64 (`tile`; the last panel
-// takes its own).  A boundary, where the chip drains, costs 12 us with two
-// workgroups on a CU (128) and a tenth of a round more with five (64); 5 % in all.
+// takes its own).  A boundary, where the chip drains, costs 12 us (FP32: 30) with two
+// workgroups on a CU (128) and a tenth of a round more with five (64); 5 % in all,
+// FP32 2 %.
 // One launch / panels, left on the device and copied back: FP64 4096^3 1.96 / 1.98
 // and 4.41 / 3.40 ms, 5003 x 3001 x 9011 4.15 / 4.32 and 6.37 / 5.02, 8192 x 8192 x
 // 2000 3.85 / 3.89 and 13.4 / 10.0; FP32 4096 x 4100 x 8192 2.18 / 2.23 and 3.45 /
@@ -1313,7 +1314,7 @@ std::vector<int> result_panels(const Exec& x, int M, int N, int K, bool split, i
   const long column = (long)((M + bm - 1) / bm) * std::max(planes, 1);  // places of a column of tiles
   const long rounds = column * tn / places, step = std::max(1L, rounds / 16);
   std::vector<int> at{0};  // ends, in columns of tiles
-  double boundary = bm == 64 ? 12 + 0.1 * gemm_round_us<T>(64, K) : 12;
+  double boundary = (sizeof(T) == 8 ? 12 : 30) + (bm == 64 ? 0.1 * gemm_round_us<T>(64, K) : 0);
   for (int exact = planes != 0; exact >= 0 && at.size() == 1; --exact) {
     if (planes) boundary = us / std::max(1L, rounds) * (exact ? 1.0 : 2.0);
     for (long q = step; q <= rounds && at.size() < 20; ++q) {
@@ -1323,7 +1324,7 @@ std::vector<int> result_panels(const Exec& x, int M, int N, int K, bool split, i
       q += step - 1;
     }
   }
-  const double may = planes ? 0.0105 : 0.05;
+  const double may = planes ? 0.0105 : sizeof(T) == 8 ? 0.05 : 0.02;
   const int most = std::min(4, 1 + (int)(may * us / boundary)), cnt = (int)at.size();
   if (most < 2 || cnt < 2) return ends;
   // when the product is over up to an end
