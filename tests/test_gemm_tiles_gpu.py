@@ -126,3 +126,26 @@ def test_ring_ends_in_a_remainder_of_any_size(xk, ta, tb, dtype):
             assert np.array_equal(C, (A if ta == 111 else A.T) @ (B if tb == 111 else B.T)), K
     finally:
         xk.lib().xkblas_set_gemm_tile(0)
+
+
+@pytest.mark.parametrize("ta,tb", OPS)
+@pytest.mark.parametrize("dtype,M,N,K", [
+    (np.float64, 700, 901, 31), (np.float64, 700, 901, 32), (np.float64, 160, 7680, 127), (np.float64, 160, 7680, 128),
+    (np.float32, 1100, 1000, 63), (np.float32, 1100, 1000, 33), (np.float32, 1100, 1000, 64),
+    (np.float32, 7168, 7200, 576), (np.float32, 7100, 7300, 600)])
+def test_kernel_by_rule_gives_the_same_bits(xk, dtype, M, N, K, ta, tb):
+    """On both sides of the lines between the two kernels (short inner dimensions;
+    FP32 over many rounds, C's columns a multiple of 4 KB apart or not): what 64 x
+    64 tiles of the other kernel give, bit for bit."""
+    r = rng(K)
+    A = (r.random((K, M) if ta == 111 else (M, K), dtype=dtype) - dtype(0.5)).T
+    B = (r.random((N, K) if tb == 111 else (K, N), dtype=dtype) - dtype(0.5)).T
+    out = []
+    for t in (0, 64):
+        xk.lib().xkblas_set_gemm_tile(t)
+        C = np.ones((N, M), dtype=dtype).T
+        xk.gemm(ta, tb, 1.5, A, B, -0.5, C)
+        xk.invalidate()
+        out.append(C)
+    xk.lib().xkblas_set_gemm_tile(0)
+    assert np.array_equal(out[0], out[1])

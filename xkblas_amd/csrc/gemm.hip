@@ -641,6 +641,27 @@ static int dma_tile(long t128, long t64, int k, bool may_mix, bool& mixed, doubl
   return c128 < c64 ? 128 : 64;
 }
 
+// Whether the register-staged kernel is the faster one for aligned operands (us,
+// it / direct to LDS).
+// FP64: an inner dimension of less than two stages (4096^2 x 24 50.2 / 54.1, 1024^2
+// x 8 8.9 / 9.6), or of a few where 32 x 32 tiles are more than one fill of the
+// chip (160 x 7680 x 48 11.6 / 12.4, x 96 14.3 / 14.7).
+// FP32: a remainder of a first or second stage where 64 x 64 tiles fit the chip at
+// once (4096 x 512 x 48 12.5 / 14.4, 1024^2 x 16 9.7 / 11.5; 2048^2 x 16 23 / 16); and middling inner dimensions over
+// many rounds, where two workgroups on a CU hide less of each other's loads than
+// four, with both operands stored along their rows (12000^2 x 768 1909 / 2040) or
+// with C's columns a multiple of 4 KB apart, which meet in the same memory channels
+// (8192^2 x 768 881 / 985 and 914 with B along the inner dimension, 10240^2 1352 /
+// 1387; 7936^2 866 / 842, 8192^2 x 512 641 / 619, x 1300 1417 / 1413).
+template <typename T>
+static bool registers_better(long t128, long t64, long t32, int k, bool ta, bool tb, long ldc)
+{
+  if (sizeof(T) == 8) return k < 32 || (k < 128 && t64 < 512 && t32 > 1024);
+  const bool rows = !ta && tb, strided = ldc * 4 % 4096 == 0;
+  if (k < 64) return k % 32 != 0 && t64 >= 256 && t128 < 160;
+  return t128 >= 3072 && (rows || strided) && k >= 576 && k < (rows && strided ? 1536 : 1152);
+}
+
 template <typename T>
 int gemm_tile_of(int m, int n, int k, double* us)
 {
@@ -679,7 +700,8 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, c
   };
   int bm = g_force_tile;
   // 32-bit offsets inside a tile
-  const bool dma = p.vecA && p.vecB && lda < (1L << 21) && ldb < (1L << 21);
+  const bool dma = p.vecA && p.vecB && lda < (1L << 21) && ldb < (1L << 21) &&
+                   (bm || tile || !registers_better<T>(tiles(128), tiles(64), tiles(32), kpart ? kpart : k, ta, tb, ldc));
   if (dma) {
     bool mixed = false;
     if (bm == 0) {
@@ -700,7 +722,7 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, c
     else launch_dma<T, 64, 2>(s, ta, tb, p, batch);
     return;
   }
-  // operands at odd offsets (row panels of an odd tile size): the tiles of
+  // also operands at odd offsets (row panels of an odd tile size): the tiles of
   // the register-staged kernel by the same reasons, FP64 55.8 against 47.1
   // TFLOP/s with 64 and 128 (more resident waves per CU), FP32 128 once they
   // fill the chip
