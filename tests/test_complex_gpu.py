@@ -415,3 +415,37 @@ def test_ztrsm_diagonal_of_any_phase(xk, uplo, ta, n):
         ref = np.linalg.solve(_op(T, ta), alpha * B0)
         err = _inf(X - ref) / ((_inf(_op(T, ta)) + _inf(ref)) * max(n, 5) * EPS)
         assert err <= 10.0, err
+
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("ta", OPS)
+@pytest.mark.parametrize("uplo", [121, 122])
+@pytest.mark.parametrize("n", [1, 20, 150])
+@pytest.mark.parametrize("end", [1, -1])
+def test_ztrsm_diagonal_at_the_end_of_the_range(xk, end, n, uplo, ta, dtype):
+    """One column scaled to the top of the range, where the parts of its diagonal
+    entry are finite and the modulus is not, or to the bottom, where its reciprocal is
+    still finite: A = M S, M near the identity, S the scales.  Bar: 20 n eps on the
+    unscaled solution."""
+    r = rng(n + uplo + ta)
+    eps, top, j = np.finfo(dtype).eps, 1023 if dtype == np.complex128 else 127, n // 2
+    M = np.where(_tri(n, uplo), r.uniform(-1, 1, (n, n)) + 1j * r.uniform(-1, 1, (n, n)), 0) / (4 * n)
+    M[np.diag_indices(n)] = np.resize([0.8 + 0.7j, -1.0, 0.9j, 1.0 - 0.6j, -0.7 - 0.7j], n)
+    e = np.zeros(n, int)
+    e[j] = top if end > 0 else 3 - top
+    M[j, j] = 1.9 - 1.8j
+    s = np.ldexp(1.0, e)
+    A = np.zeros((n, n), dtype, order="F")
+    A.real, A.imag = np.ldexp(M.real, e), np.ldexp(M.imag, e)
+    with np.errstate(over="ignore"):
+        assert np.all(np.isfinite(A)) and np.isinf(np.abs(A[j, j])) == (end > 0)
+    M = A.astype(np.clongdouble) / s.astype(np.longdouble)
+    y = (r.uniform(0.5, 1, (n, 3)) + 1j * r.uniform(0.5, 1, (n, 3))).astype(np.clongdouble)
+    y *= np.longdouble(2.0 ** (10 * end) if ta == 111 else 2.0 ** -4)
+    B = np.asfortranarray((M @ y if ta == 111 else s[:, None].astype(np.longdouble) * ((M.T if ta == 112 else M.conj().T) @ y)).astype(dtype))
+    X = B.copy(order="F")
+    xk.trsm(141, uplo, ta, 131, 1.0, A, X)
+    xk.invalidate()
+    Y = X.astype(np.clongdouble) * s[:, None].astype(np.longdouble) if ta == 111 else X.astype(np.clongdouble)
+    assert np.all(np.abs(Y - y) <= 20 * n * eps * np.abs(y).max()), np.abs(Y - y).max() / np.abs(y).max()

@@ -1008,19 +1008,19 @@ void dev_ctrsm(const Exec& x, int side, int uplo, int transA, int diag, int m, i
   const bool lower_eff = (uplo == Lower) != tr;
   const int na = side == Left ? m : n;
   if (side == Left && na <= CPLX_REAL_MAX) {
-    // A = T' D with a real diagonal in T': rho(T') is triangular and B, as it
-    // lies in memory, its right-hand sides: a real solve of twice the order.
-    // NoTrans: X = D^-1 T'^-1 alpha B; ConjTrans: X = T'^-H D alpha B; Trans:
-    // the conjugate of that with conj(alpha B)
+    // A = T' D^-1 with a real diagonal in T': rho(T') is triangular and B, as
+    // it lies in memory, its right-hand sides: a real solve of twice the order.
+    // NoTrans: X = D T'^-1 alpha B; ConjTrans: X = T'^-H conj(D) alpha B;
+    // Trans: the conjugate of that with conj(alpha B)
     const long ldr = (2L * na + 31) / 32 * 32;
     T* R = (T*)scratch(WS_ZR, sizeof(T) * (size_t)ldr * 2 * na);
     T* D = (T*)scratch(WS_ZW, 2 * sizeof(T) * (size_t)na);
     cplx_trsm_form<T>(x.s, uplo, diag == Unit, na, A, lda, R, ldr, D);
     const T calpha[2] = {alpha[0], -alpha[1]};
-    if (transA == ConjTrans) cplx_scale_rows<T>(x.s, m, n, 0, 0, alpha, D, B, ldb);
-    else if (transA == Trans) cplx_scale_rows<T>(x.s, m, n, 1, 0, calpha, D, B, ldb);
+    if (transA == ConjTrans) cplx_scale_rows<T>(x.s, m, n, 0, 1, alpha, D, B, ldb);
+    else if (transA == Trans) cplx_scale_rows<T>(x.s, m, n, 1, 1, calpha, D, B, ldb);
     dev_trsm<T>(x, Left, uplo, tr ? Trans : NoTrans, NonUnit, 2 * m, n, T(1), R, ldr, B, 2 * ldb, 512);
-    if (transA == NoTrans) cplx_scale_rows<T>(x.s, m, n, 0, 1, alpha, D, B, ldb);
+    if (transA == NoTrans) cplx_scale_rows<T>(x.s, m, n, 0, 0, alpha, D, B, ldb);
     else if (transA == Trans) cplx_scale_rows<T>(x.s, m, n, 1, 0, one, nullptr, B, ldb);
     return;
   }

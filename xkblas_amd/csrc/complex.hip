@@ -83,9 +83,12 @@ __global__ __launch_bounds__(256) void cplx_deal_kernel(int rows, int cols, int 
 }
 
 // Real triangular form of a complex triangular matrix T for its solves: T = T'
-// D with D diagonal of modulus one and a real positive diagonal in T', so that
-// rho(T') is triangular itself.  R (2n x 2n, uplo triangle) <- rho(T'), D its
-// n diagonal entries (1 when unit: the diagonal is not read).
+// D^-1 with D diagonal and a real positive diagonal in T', so that rho(T') is
+// triangular itself.  That diagonal is |T(j, j)| where T(j, j) is real, and else a
+// power of two near it that neither overflows, as the modulus may, nor has a
+// subnormal or infinite reciprocal; D(j) = 2^e / T(j, j) is of size one.  R (2n x
+// 2n, uplo triangle) <- rho(T'), D its n entries (1 when unit: the diagonal is not
+// read).
 template <typename T>
 __global__ __launch_bounds__(256) void cplx_trsm_form_kernel(int uplo, int unit, int n, int j0,
                                                              const Cplx<T>* __restrict__ A, long lda,
@@ -98,17 +101,26 @@ __global__ __launch_bounds__(256) void cplx_trsm_form_kernel(int uplo, int unit,
   T h = T(1);
   if (!unit) {
     const Cplx<T> t = A[j + (long)j * lda];
-    h = t.im == T(0) ? fabs(t.re) : hypot(t.re, t.im);
-    if (t.im == T(0)) d.re = t.re < T(0) ? T(-1) : T(1);
-    else d = Cplx<T>{t.re / h, t.im / h};
+    if (t.im == T(0)) {
+      h = fabs(t.re);
+      d.re = t.re < T(0) ? T(-1) : T(1);
+    } else {
+      constexpr int most = sizeof(T) == 8 ? 1022 : 126;
+      int e;
+      (void)frexp(fmax(fabs(t.re), fabs(t.im)), &e);
+      e = max(-most, min(most, e - 1));
+      const T re = ldexp(t.re, -e), im = ldexp(t.im, -e), q = re * re + im * im;
+      d = Cplx<T>{re / q, -im / q};
+      h = ldexp(T(1), e);
+    }
   }
   Cplx<T> z{h, T(0)};
   if (i == j) {
     D[j] = d;
   } else {
-    const Cplx<T> a = A[i + (long)j * lda];  // times conj(d)
+    const Cplx<T> a = A[i + (long)j * lda];  // times d
     z = d.im == T(0) ? Cplx<T>{a.re * d.re, a.im * d.re}
-                     : Cplx<T>{a.re * d.re + a.im * d.im, a.im * d.re - a.re * d.im};
+                     : Cplx<T>{a.re * d.re - a.im * d.im, a.im * d.re + a.re * d.im};
   }
   T* r = R + 2 * i + (long)(2 * j) * ldr;
   r[0] = z.re;

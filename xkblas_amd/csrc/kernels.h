@@ -116,7 +116,7 @@ template <typename T>
 void cplx_rho(hipStream_t s, int sigma, int rows, int cols, const T* A, long lda, T* Y, long ldy);
 template <typename T>
 void cplx_deal(hipStream_t s, int sign, int rows, int cols, const T* B, long ldb, T* Y, long ldy);
-// The triangle A = T' D (D of modulus one, T' with a real positive diagonal):
+// The triangle A = T' D^-1 (T' with a real positive diagonal, D of size one):
 // R (2n x 2n, uplo triangle) <- rho(T'), D its n entries; and B(i, j) <- alpha
 // B(i, j) D(i) with conj(B) / conj(D) as asked (D null: 1).
 template <typename T>
