@@ -63,3 +63,33 @@ def test_triangle_in_parts(xk, n, k, trans, uplo, dt):
     bar = (2 * k + 8) * np.finfo(real).eps * (1.25 * np.abs(X) @ np.abs(X).T)
     C[off] = ref[off]
     assert np.all(np.abs(C - ref) <= bar)
+
+
+CHILD = """
+import sys
+sys.path.insert(0, %r)
+import numpy as np, xkblas_amd as xk
+L = xk.lib()
+L.xkblas_init()
+r = np.random.default_rng(3)
+A, B = (np.asfortranarray(r.uniform(-1, 1, s)) for s in ((300, 1500), (1500, 200)))
+out = []
+for tile in (0, 32):  # a set tile: one part
+    L.xkblas_set_gemm_tile(tile)
+    C = np.zeros((300, 200), order="F")
+    xk.gemm(xk.NoTrans, xk.NoTrans, 1.0, A, B, 0.0, C)
+    out.append(C)
+print("same" if np.array_equal(*out) else "different")
+"""
+
+
+@pytest.mark.parametrize("value,want", [("0", "same"), ("1", "different")])
+def test_no_parts_when_switched_off(xk, value, want):
+    """XKBLAS_SPLITK=0: the sums of one part, bit for bit."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    p = subprocess.run([sys.executable, "-c", CHILD % root], env=dict(os.environ, XKBLAS_SPLITK=value), timeout=60,
+                       capture_output=True, text=True)
+    assert p.returncode == 0 and p.stdout.strip() == want, p.stdout + p.stderr

@@ -32,6 +32,14 @@ namespace xk {
 
 enum { WS_SPLITK = 31 };
 
+// Whether any product may be split along its inner dimension (XKBLAS_SPLITK=0:
+// none).
+static bool splitk_enabled()
+{
+  static const int v = getenv("XKBLAS_SPLITK") ? atoi(getenv("XKBLAS_SPLITK")) : 1;
+  return v != 0;
+}
+
 // Parts of the inner dimension of a product with few tiles: the parts are
 // multiplied side by side (one launch, each into its own partial result) and
 // summed by a second pass over the result.  They fill the CUs that the tiles
@@ -50,7 +58,7 @@ enum { WS_SPLITK = 31 };
 int gemm_k_parts(int m, int n, int k, int tri)
 {
   const long a = (m + 63) / 64, b = (n + 63) / 64, t64 = tri == TRI_FULL ? a * b : a * (a + 1) / 2;
-  if (k < 512 || t64 >= 768 || gemm_get_tile() != 0) return 1;  // a set tile: one product as it is
+  if (k < 512 || t64 >= 768 || !splitk_enabled() || gemm_get_tile() != 0) return 1;  // a set tile: one product as it is
   const long most = std::max(8L, std::min(32L, 512 / t64));
   return (int)std::max(1L, std::min(most, (long)k / (t64 <= 48 ? 192 : 600)));
 }
@@ -232,14 +240,8 @@ enum { WS_TRSM = 4, WS_TRSMW = 5 };
 // products and late updates of a TRSM sweep with few right-hand sides) are
 // latency-bound: each tile walks its k slices one after the other.  Split
 // the inner dimension into 2, 4 or 8 chunks computed by one batched launch
-// into partial products, summed by a reduction (XKBLAS_SPLITK=0 turns it
-// off).  Returns false when the shape does not qualify.
-static bool splitk_enabled()
-{
-  static const int v = getenv("XKBLAS_SPLITK") ? atoi(getenv("XKBLAS_SPLITK")) : 1;
-  return v != 0;
-}
-
+// into partial products, summed by a reduction.  Returns false when the shape
+// does not qualify.
 template <typename T>
 static bool gemm_splitk(hipStream_t s, int ta, int tb, int m, int n, int k, T alpha, const T* A, long lda,
                         const T* B, long ldb, T beta, T* C, long ldc)
