@@ -183,14 +183,6 @@ static void inverse_levels(hipStream_t s, int uplo, int diag, int n, const T* A,
   }
 }
 
-template <typename T>
-void dev_trtri(const Exec& x, hipStream_t s, int uplo, int diag, int n, const T* A, long lda, T* Tinv, long ldinv,
-               int wslot)
-{
-  fill_zero<T>(s, n, n, Tinv, ldinv);
-  inverse_levels<T>(s, uplo, diag, n, A, lda, 0, Tinv, ldinv, 0, 1, wslot, true);
-}
-
 // Cholesky of the first nc columns of the trapezoid of nr rows at A (Lower;
 // Upper: the first nc rows of nr columns), right-looking in blocks of LEAF:
 // leaf (factor and inverse in one launch, the inverse of block j at Tinv + j
@@ -912,8 +904,8 @@ void dev_ctrmm(const Exec& x, int side, int uplo, int transA, int diag, int m, i
   else cgemm_impl<T>(x, NoTrans, transA, m, n, n, alpha, W, ldw, F, ldf, zero, B, ldb, 0, 0);
 }
 
-// Complex triangular inverse (Tinv n x n, other triangle zeroed): the
-// recursion of dev_trtri with complex products; leaves of 64.
+// Complex triangular inverse (Tinv n x n, other triangle zeroed): halves
+// joined by complex products, leaves of 64.
 enum { WS_ZW = 23, WS_ZR = 24, WS_ZPAN = 25, WS_ZINV = 26, WS_ZRI = 29, WS_ZDW = 30 };
 
 template <typename T>
@@ -1436,7 +1428,6 @@ int dev_posv_ir(const Exec& x, const Exec& xl, const Exec& xf, int uplo, int n, 
   template void dev_syrk<T>(const Exec&, int, int, int, int, T, const T*, long, T, T*, long);                     \
   template void dev_trsm<T>(const Exec&, int, int, int, int, int, int, T, const T*, long, T*, long, int);        \
   template void dev_potrf<T>(const Exec&, int, int, T*, long, int, int*, const PotrfHooks<T>*);                  \
-  template void dev_trtri<T>(const Exec&, hipStream_t, int, int, int, const T*, long, T*, long, int);        \
   template void dev_gemmt<T>(const Exec&, int, int, int, int, int, T, const T*, long, const T*, long, T, T*,     \
                              long);                                                                             \
   template void dev_syr2k<T>(const Exec&, int, int, int, int, T, const T*, long, const T*, long, T, T*, long);  \

@@ -159,9 +159,4 @@ void dev_ctrmm(const Exec& x, int side, int uplo, int transA, int diag, int m, i
 int dev_posv_ir(const Exec& x, const Exec& xl, const Exec& xf, int uplo, int n, int nrhs, const double* A, long lda,
                 const double* B, long ldb, double* X, long ldx, int nb, int itermax, int* iter);
 
-// Inverse of the triangular n x n block A into Tinv (other triangle zeroed).
-template <typename T>
-void dev_trtri(const Exec& x, hipStream_t s, int uplo, int diag, int n, const T* A, long lda, T* Tinv, long ldinv,
-               int wslot);
-
 }  // namespace xk

@@ -1,6 +1,6 @@
 // factor.hip — latency-bound diagonal-block kernels for gfx950:
 // Cholesky + inverse of blocks of order <= 128, triangular inverse, and small
-// helpers (2-D copy, triangle zeroing, int fill).
+// helpers (2-D copy, sums of partial products, int fill).
 //
 // The rows/columns of a leaf's last 16 x 16 tile beyond n are the identity.
 // The Cholesky leaf writes the factor and its inverse in one launch.
@@ -751,25 +751,6 @@ void copy2d(hipStream_t s, int m, int n, const T* X, long ldx, T* Y, long ldy)
   XK_HIP(hipGetLastError());
 }
 
-template <typename T>
-__global__ void zero_tri_kernel(int uplo, int n, T* A, long lda)
-{
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = blockIdx.y;
-  if (i < n && j < n) {
-    if ((uplo == Lower && i < j) || (uplo == Upper && i > j)) A[i + (long)j * lda] = T(0);
-  }
-}
-
-template <typename T>
-void zero_triangle(hipStream_t s, int uplo, int n, T* A, long lda)
-{
-  if (n <= 0) return;
-  XK_CHECK(n <= 65535, "zero_triangle: order too large");
-  hipLaunchKernelGGL((zero_tri_kernel<T>), dim3((n + 255) / 256, n), dim3(256), 0, s, uplo, n, A, lda);
-  XK_HIP(hipGetLastError());
-}
-
 // C <- beta C + sum_p W_p (W_p: m x n, leading dimension m, p-th at p m n);
 // beta == 0 never reads C.
 template <typename T>
@@ -814,7 +795,6 @@ void fill_int(hipStream_t s, int* p, int n, int v)
   template void potrf_leaf<T>(hipStream_t, int, int, T*, long, long, T*, long, long, int, int*, int, int);         \
   template void trtri_leaf<T>(hipStream_t, int, int, int, const T*, long, long, T*, long, long, int);         \
   template void copy2d<T>(hipStream_t, int, int, const T*, long, T*, long);                                    \
-  template void zero_triangle<T>(hipStream_t, int, int, T*, long);                                            \
   template void splitk_reduce<T>(hipStream_t, int, int, int, const T*, T, T*, long, int);
 XK_INST(double)
 XK_INST(float)

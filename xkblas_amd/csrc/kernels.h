@@ -62,11 +62,6 @@ void trsm_panel(hipStream_t s, int uplo, int m, int n, T* P, long lda, const T* 
 template <typename T>
 void copy2d(hipStream_t s, int m, int n, const T* X, long ldx, T* Y, long ldy);
 
-// Zero the strictly upper (uplo == Lower) or strictly lower part of an n x n
-// block.
-template <typename T>
-void zero_triangle(hipStream_t s, int uplo, int n, T* A, long lda);
-
 // C <- beta C + sum over `parts` of the m x n partial products W (leading
 // dimension m, one every m n elements); beta == 0 never reads C.
 template <typename T>
