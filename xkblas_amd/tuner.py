@@ -3,7 +3,8 @@
 The library exposes a timing service (``xkblas_tune_time``: one call of a
 given shape and configuration on device-resident operands, HIP-event kernel
 time) and the knobs the model chooses between: the GEMM macro tile, the block
-order NB of TRSM/POTRF, the split count and the BF16 residue-GEMM variant.
+order NB of TRSM and of POTRF with split products, the split count and the BF16
+residue-GEMM variant.
 This module
 
 * collects timings of GEMM / SYRK / TRSM / POTRF calls with shapes drawn
@@ -50,8 +51,16 @@ def split_counts(mode, k):
     return [nm.value]
 
 
+def own_blocks(op, dtype, mode):
+    """POTRF in the MFMA modes: the library chooses its block columns itself
+    and takes no NB."""
+    return op == "potrf" and not (mode in SPLIT_MODES and dtype == 0)
+
+
 def candidates(op, dtype, mode, m, n, k):
     """Configurations the model chooses between for one call."""
+    if own_blocks(op, dtype, mode):
+        return [{"tile": 0, "nb": 0, "split": 0, "kernel": 0}]
     if op in ("gemm", "syrk"):
         if mode in SPLIT_MODES and dtype == 0:
             kernels = (0, 1) if mode == 2 else (0,)
@@ -60,6 +69,9 @@ def candidates(op, dtype, mode, m, n, k):
         return [{"tile": t, "nb": 0, "split": 0, "kernel": 0} for t in tiles]
     dim = m
     nbs = [b for b in (64, 128, 256, 512, 1024, 2048, 4096) if b <= max(64, dim) and (b < 4096 or dim >= 16384)]
+    rule = heuristic(op, dtype, mode, m, n, k)["nb"]  # for small orders the whole triangle
+    if rule not in nbs:
+        nbs.append(rule)
     return [{"tile": 0, "nb": b, "split": 0, "kernel": 0} for b in nbs]
 
 
@@ -71,7 +83,7 @@ def heuristic(op, dtype, mode, m, n, k):
     L.xkblas_set_param(0, 0)
     nb = int(L.xkblas_auto_tilesize(None, KERN[op], m, n if op != "potrf" else m, k))
     L.xkblas_set_param(old, 0)
-    if op in ("gemm", "syrk"):
+    if op in ("gemm", "syrk") or own_blocks(op, dtype, mode):
         return {"tile": 0, "nb": 0, "split": 0, "kernel": 0}
     return {"tile": 0, "nb": min(nb, max(64, m)), "split": 0, "kernel": 0}
 
