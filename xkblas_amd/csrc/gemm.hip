@@ -663,14 +663,15 @@ static bool registers_better(long t128, long t64, long t32, int k, bool ta, bool
 }
 
 template <typename T>
-int gemm_tile_of(int m, int n, int k, double* us)
+int gemm_tile_of(bool ta, bool tb, int m, int n, int k, long ldc, double* us)
 {
   auto tiles = [&](int t) { return (long)((m + t - 1) / t) * ((n + t - 1) / t); };
   bool mixed;
+  if (registers_better<T>(tiles(128), tiles(64), tiles(32), k, ta, tb, ldc)) return 0;
   return dma_tile<T>(tiles(128), tiles(64), k, true, mixed, us);
 }
-template int gemm_tile_of<double>(int, int, int, double*);
-template int gemm_tile_of<float>(int, int, int, double*);
+template int gemm_tile_of<double>(bool, bool, int, int, int, long, double*);
+template int gemm_tile_of<float>(bool, bool, int, int, int, long, double*);
 
 template <typename T>
 void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, const T* A, long lda,

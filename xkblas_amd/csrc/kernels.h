@@ -22,9 +22,9 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha,
           int tile = 0);
 
 // The tile gemm() takes for a product with aligned operands, and about how
-// long the product runs (unless with 32 x 32 tiles).
+// long the product runs (unless with 32 x 32 tiles); 0: through registers.
 template <typename T>
-int gemm_tile_of(int m, int n, int k, double* us);
+int gemm_tile_of(bool ta, bool tb, int m, int n, int k, long ldc, double* us);
 // Time of a full round over the chip of tiles of 128 x 128 (512 of them) or 64
 // x 64 (1280).
 template <typename T>

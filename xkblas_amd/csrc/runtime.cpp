@@ -1291,7 +1291,7 @@ bool pipeline_enabled()
 // 101.1; smaller products in one launch.  (By rounds up to 6 % more, 4096^3 left on
 // the device took 1.91 ms instead of 1.71, 2430 x 2059 x 1300 0.48 instead of 0.38.)
 template <typename T>
-std::vector<int> result_panels(const Exec& x, int M, int N, int K, bool split, int& tile)
+std::vector<int> result_panels(const Exec& x, bool ta, bool tb, int M, int N, int K, long ldc, bool split, int& tile)
 {
   std::vector<int> ends;
   tile = 0;
@@ -1306,8 +1306,8 @@ std::vector<int> result_panels(const Exec& x, int M, int N, int K, bool split, i
     us = 2.0 * M * N * K * planes / (planes > 13 ? 2.7e9 : 1.15e9);
   } else {
     if (gemm_get_tile() != 0 || gemm_k_parts(M, N, K, TRI_FULL) > 1) return ends;
-    bm = gemm_tile_of<T>(M, N, K, &us);
-    if (bm == 32) return ends;
+    bm = gemm_tile_of<T>(ta, tb, M, N, K, ldc, &us);
+    if (bm < 64) return ends;
     places = bm == 128 ? 512 : 1280;
   }
   const int tn = (N + bm - 1) / bm;
@@ -1348,7 +1348,7 @@ std::vector<int> result_panels(const Exec& x, int M, int N, int K, bool split, i
         }
       }
       double rest = us - over[i];
-      if (!planes && gemm_tile_of<T>(M, N - at[i] * bm, K, &rest) == 32) continue;
+      if (!planes && gemm_tile_of<T>(ta, tb, M, N - at[i] * bm, K, ldc, &rest) < 64) continue;
       const double prod = over[i] + rest + p * boundary, end = std::max(back[p][i], prod) + copy * (tn - at[i]);
       if (end < best && prod <= (1 + may) * us) {
         best = end;
@@ -1410,7 +1410,7 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
     resident = r.all_valid(rA, 0, 0, Am, An) && r.all_valid(rB, 0, 0, Bm, Bn) &&
                (!readC || r.all_valid(rC, 0, 0, M, N));
     if (resident) {
-      ends = result_panels<T>(x, M, N, K, split, x.tile);
+      ends = result_panels<T>(x, transA != NoTrans, transB != NoTrans, M, N, K, rC->ldd, split, x.tile);
     } else if (M > nb && (!r.all_valid(rA, 0, 0, Am, An) || (readC && !r.all_valid(rC, 0, 0, M, N)))) {
       for (int e = nb; e < M; e += nb) ends.push_back(e);
       ends.push_back(M);
