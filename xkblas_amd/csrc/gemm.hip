@@ -612,13 +612,11 @@ static void launch_mixed(hipStream_t s, bool ta, bool tb, GemmParams<T>& p, int 
 // 64.4 / 64.9.  (With registers between memory and LDS, tiles as now: 8192^3
 // 58.5, 4096^3 51.6, 1024^3 31.4, 512^3 12.8; FP32 133, 111, 47.7, 11.0.)
 template <typename T>
-double gemm_round_us(int tile, int k)
+static double round_us(int tile, int k)
 {
   return tile == 128 ? 512 * 128 * 128 * (k + 150.0) / (sizeof(T) == 8 ? 35.25e6 : 68e6)
                      : 1280 * 64 * 64 * (k + 57.0) / (sizeof(T) == 8 ? 33e6 : 60e6);
 }
-template double gemm_round_us<double>(int, int);
-template double gemm_round_us<float>(int, int);
 
 template <typename T>
 static int dma_tile(long t128, long t64, int k, bool may_mix, bool& mixed, double* us = nullptr)
@@ -635,11 +633,23 @@ static int dma_tile(long t128, long t64, int k, bool may_mix, bool& mixed, doubl
     mixed = may_mix && quarters < plain;
     last = mixed ? quarters : plain;
   }
-  const double c128 = (w128 + last) * gemm_round_us<T>(128, k);
-  const double c64 = (w64 + (f64 == 0 ? 0 : 0.5 + 0.5 * f64)) * gemm_round_us<T>(64, k);
+  const double c128 = (w128 + last) * round_us<T>(128, k);
+  const double c64 = (w64 + (f64 == 0 ? 0 : 0.5 + 0.5 * f64)) * round_us<T>(64, k);
   if (us) *us = std::min(c128, c64);
   return c128 < c64 ? 128 : 64;
 }
+
+template <typename T>
+double gemm_tiles_us(int tile, long tiles, int k)
+{
+  const double r = tiles / (tile == 128 ? 512.0 : 1280.0), w = std::floor(r), f = r - w;
+  double last = f == 0 ? 0 : 0.5 + 0.5 * f;
+  if (tile == 128 && f > 0)
+    last = w == 0 ? std::min(1.0, 0.62 + 0.95 * std::max(0.0, f - 0.5)) : std::min({1.12, 0.6 + 0.95 * f, 0.1 + 1.2 * f});
+  return (w + last) * round_us<T>(tile, k);
+}
+template double gemm_tiles_us<double>(int, long, int);
+template double gemm_tiles_us<float>(int, long, int);
 
 // Whether the register-staged kernel is the faster one for aligned operands (us,
 // it / direct to LDS).

@@ -25,10 +25,10 @@ void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha,
 // long the product runs (unless with 32 x 32 tiles); 0: through registers.
 template <typename T>
 int gemm_tile_of(bool ta, bool tb, int m, int n, int k, long ldc, double* us);
-// Time of a full round over the chip of tiles of 128 x 128 (512 of them) or 64
-// x 64 (1280).
+// About how long `tiles` tiles of 128 x 128 (512 to a round over the chip) or 64
+// x 64 (1280) of inner dimension k run in a launch of their own.
 template <typename T>
-double gemm_round_us(int tile, int k);
+double gemm_tiles_us(int tile, long tiles, int k);
 
 // Forces the macro-tile shape of gemm(): 0 = automatic, 32, 64
 // or 128.

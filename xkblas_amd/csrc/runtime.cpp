@@ -1273,23 +1273,25 @@ bool pipeline_enabled()
 // columns at half of it).
 // Nothing says yet whether the result will be copied, so the panels may cost a
 // caller who leaves it on the device little, and are taken where the copied
-// result is there a tenth earlier: all but the last panel end where whole rounds
-// of the product's tiles over the chip do, at most 1.5 % of their places empty.
+// result is there a tenth earlier.  All but the last end where whole rounds of the
+// product's tiles over the chip do; among those ends the ones with the earliest
+// last copy.
 // MFMA modes: rounds of 512 tiles of 128 or 1280 of 64 (`tile`; the last panel
 // takes its own).  A boundary, where the chip drains, costs 12 us (FP32: 30) with two
-// workgroups on a CU (128) and a tenth of a round more with five (64); 5 % in all,
-// FP32 2 %.
-// One launch / panels, left on the device and copied back: FP64 4096^3 1.96 / 1.98
-// and 4.41 / 3.40 ms, 5003 x 3001 x 9011 4.15 / 4.32 and 6.37 / 5.02, 8192 x 8192 x
-// 2000 3.85 / 3.89 and 13.4 / 10.0; FP32 4096 x 4100 x 8192 2.18 / 2.23 and 3.45 /
-// 2.87.  (On two streams, in panels of 300 tiles, 2.6 ms left on the device for
-// 4096^3 and 1.9 instead of 1.4 for 3300 x 3300 x 4000.)
+// workgroups on a CU (128) and a tenth of a round more with five (64); the product
+// in panels, by its tiles' rounds, may take 8 % (FP32: 6 %) more than one launch,
+// and measures up to 7 %.  One launch / panels, left on the device and copied back:
+// FP64 4096^3 1.95 / 1.97 and 4.39 / 3.41 ms, 5003 x 3001 x 9011 4.14 / 4.31 and 6.40 /
+// 5.03, 6000^3 6.30 / 6.75 and 11.6 / 7.95, 8192 x 8192 x 2000 3.83 / 3.96 and 13.4 / 9.9;
+// FP32 4096 x 4100 x 8192 2.18 / 2.22 and 3.44 / 2.87.  (On two streams, in panels of
+// 300 tiles whatever the rounds, 2.6 ms left on the device for 4096^3 and 1.9 instead
+// of 1.4 for 3300 x 3300 x 4000.)
 // Split modes: rounds of 256 tiles of 256 over all planes.  A boundary costs up to
 // a round where the rounds end exactly (8192^3 BF16 0.1 ms) and two elsewhere
-// (4843 x 7959 x 7432 in two panels 6.46 -> 6.86 ms); 1 % in all.
-// BF16, as above: 16384^3 85.3 / 85.6 and 123.9 / 92.5; FP8 97.5 / 97.9 and 137.5 /
-// 101.1; smaller products in one launch.  (By rounds up to 6 % more, 4096^3 left on
-// the device took 1.91 ms instead of 1.71, 2430 x 2059 x 1300 0.48 instead of 0.38.)
+// (4843 x 7959 x 7432 in two panels 6.46 -> 6.86 ms); 1 % in all.  BF16, as above:
+// 16384^3 85.3 / 85.6 and 123.9 / 92.5; FP8 97.5 / 97.9 and 137.5 / 101.1; smaller
+// products in one launch.  (By rounds up to 6 % more, 4096^3 left on the device took
+// 1.91 ms instead of 1.71, 2430 x 2059 x 1300 0.48 instead of 0.38.)
 template <typename T>
 std::vector<int> result_panels(const Exec& x, bool ta, bool tb, int M, int N, int K, long ldc, bool split, int& tile)
 {
@@ -1297,69 +1299,77 @@ std::vector<int> result_panels(const Exec& x, bool ta, bool tb, int M, int N, in
   tile = 0;
   if ((double)M * N * sizeof(T) < 17e6) return ends;  // 0.3 ms
   double us = 0;  // of the product in one launch
-  int bm = 256, places = 256, planes = 0;
+  int planes = 0;
   if (split) {
     // fewer than 96 rounds of any count of moduli: the count takes 5 us of host time
     const bool fp8 = x.mode == XKBLAS_SPLIT_FP8_MATH;
     if ((long)((M + 255) / 256) * ((N + 255) / 256) * (fp8 ? 38 : 13) < 96 * 256) return ends;
     planes = split_plane_count(K, x.nsplit, fp8);
     us = 2.0 * M * N * K * planes / (planes > 13 ? 2.7e9 : 1.15e9);
-  } else {
-    if (gemm_get_tile() != 0 || gemm_k_parts(M, N, K, TRI_FULL) > 1) return ends;
-    bm = gemm_tile_of<T>(ta, tb, M, N, K, ldc, &us);
-    if (bm < 64) return ends;
-    places = bm == 128 ? 512 : 1280;
+  } else if (gemm_get_tile() != 0 || gemm_k_parts(M, N, K, TRI_FULL) > 1 ||
+             gemm_tile_of<T>(ta, tb, M, N, K, ldc, &us) < 64) {
+    return ends;
   }
-  const int tn = (N + bm - 1) / bm;
-  const long column = (long)((M + bm - 1) / bm) * std::max(planes, 1);  // places of a column of tiles
-  const long rounds = column * tn / places, step = std::max(1L, rounds / 16);
-  std::vector<int> at{0};  // ends, in columns of tiles
-  double boundary = (sizeof(T) == 8 ? 12 : 30) + (bm == 64 ? 0.1 * gemm_round_us<T>(64, K) : 0);
-  for (int exact = planes != 0; exact >= 0 && at.size() == 1; --exact) {
-    if (planes) boundary = us / std::max(1L, rounds) * (exact ? 1.0 : 2.0);
-    for (long q = step; q <= rounds && at.size() < 20; ++q) {
-      const long c = q * places / column;
-      if (c <= at.back() || c >= tn || (exact ? c * column != q * places : c * column * 1.015 < (double)q * places)) continue;
-      at.push_back((int)c);
-      q += step - 1;
+  const double may = planes ? 0.0105 : sizeof(T) == 8 ? 0.08 : 0.06;
+  double best = 0.9 * (us + (double)M * N * sizeof(T) / 57e3);
+  auto search = [&](int bm, int places) {
+    const int tn = (N + bm - 1) / bm;
+    const long column = (long)((M + bm - 1) / bm) * std::max(planes, 1);  // places of a column of tiles
+    const long rounds = column * tn / places, step = std::max(1L, rounds / 16);
+    std::vector<int> at{0};  // ends, in columns of tiles
+    double boundary = (sizeof(T) == 8 ? 12 : 30) + (bm == 64 ? 0.1 * gemm_tiles_us<T>(64, 1280, K) : 0);
+    for (int exact = planes != 0; exact >= 0 && at.size() == 1; --exact) {
+      if (planes) boundary = us / std::max(1L, rounds) * (exact ? 1.0 : 2.0);
+      for (long q = step; q <= rounds && at.size() < 20; ++q) {
+        const long c = q * places / column;
+        if (c <= at.back() || c >= tn || (exact && c * column < q * places)) continue;
+        at.push_back((int)c);
+        q += step - 1;
+      }
     }
-  }
-  const double may = planes ? 0.0105 : sizeof(T) == 8 ? 0.05 : 0.02;
-  const int most = std::min(4, 1 + (int)(may * us / boundary)), cnt = (int)at.size();
-  if (most < 2 || cnt < 2) return ends;
-  // when the product is over up to an end
-  std::vector<double> over(cnt);
-  for (int i = 0; i < cnt; ++i)
-    over[i] = planes ? us * at[i] / tn : (at[i] * column + places - 1) / places * gemm_round_us<T>(bm, K);
-  const double copy = (double)M * bm * sizeof(T) / 57e3;
-  // back[p][i]: when p panels up to at[i] are copied
-  std::vector<std::vector<double>> back(most, std::vector<double>(cnt, 1e300));
-  std::vector<std::vector<int>> from(most, std::vector<int>(cnt, 0));
-  back[0][0] = 0;
-  double best = 0.9 * (us + copy * tn);
-  int panels = 0, last = 0;
-  for (int p = 1; p < most; ++p)
-    for (int i = 1; i < cnt; ++i) {
-      for (int h = 0; h < i; ++h) {
-        const double end = std::max(back[p - 1][h], over[i] + (p - 1) * boundary) + copy * (at[i] - at[h]);
-        if (end < back[p][i]) {
-          back[p][i] = end;
-          from[p][i] = h;
+    const int most = std::min(8, 1 + (int)(may * us / boundary)), cnt = (int)at.size();
+    if (most < 2 || cnt < 2) return;
+    // p panels up to at[i]: the product over, the copies over, the end before
+    struct Panels {
+      double over = 1e300, back = 1e300;
+      int from = 0;
+    };
+    std::vector<std::vector<Panels>> best_of(most, std::vector<Panels>(cnt));
+    best_of[0][0].over = best_of[0][0].back = 0;
+    const double copy = (double)M * bm * sizeof(T) / 57e3;
+    auto panel_us = [&](int h, int i) {
+      return planes ? us * (at[i] - at[h]) / tn : gemm_tiles_us<T>(bm, (at[i] - at[h]) * column, K);
+    };
+    int panels = 0, last = 0;
+    for (int p = 1; p < most; ++p)
+      for (int i = 1; i < cnt; ++i) {
+        Panels& to = best_of[p][i];
+        for (int h = 0; h < i; ++h) {
+          const Panels& f = best_of[p - 1][h];
+          const double over = f.over + panel_us(h, i) + (p > 1 ? boundary : 0);
+          const double end = std::max(f.back, over) + copy * (at[i] - at[h]);
+          if (end < to.back) to = Panels{over, end, h};
+        }
+        double rest = us * (tn - at[i]) / tn;
+        if (!planes && gemm_tile_of<T>(ta, tb, M, N - at[i] * bm, K, ldc, &rest) < 64) continue;
+        const double prod = to.over + boundary + rest, end = std::max(to.back, prod) + copy * (tn - at[i]);
+        if (end < best && prod <= (1 + may) * us) {
+          best = end;
+          panels = p;
+          last = i;
         }
       }
-      double rest = us - over[i];
-      if (!planes && gemm_tile_of<T>(ta, tb, M, N - at[i] * bm, K, ldc, &rest) < 64) continue;
-      const double prod = over[i] + rest + p * boundary, end = std::max(back[p][i], prod) + copy * (tn - at[i]);
-      if (end < best && prod <= (1 + may) * us) {
-        best = end;
-        panels = p;
-        last = i;
-      }
-    }
-  if (panels == 0) return ends;
-  for (int p = panels, i = last; p >= 1; i = from[p--][i]) ends.insert(ends.begin(), at[i] * bm);
-  ends.push_back(N);
-  if (!planes) tile = bm;
+    if (panels == 0) return;
+    ends.assign(1, N);
+    for (int p = panels, i = last; p >= 1; i = best_of[p--][i].from) ends.insert(ends.begin(), at[i] * bm);
+    if (!planes) tile = bm;
+  };
+  if (planes) {
+    search(256, 256);
+  } else {
+    search(128, 512);
+    search(64, 1280);
+  }
   return ends;
 }
 
