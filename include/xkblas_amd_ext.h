@@ -40,8 +40,10 @@ void xkblas_set_lookahead(int on);
  * panels of C (one tile row each): panel p waits only for B and its own rows
  * of op(A) and C, so the host-to-device copies of panel p+1 overlap the
  * product of panel p, and xkblas_memory_coherent_async copies each panel's
- * rows back as soon as they are final.  Same result bits as one launch.
- * Default on; 0 turns it off (environment XKBLAS_PIPELINE). */
+ * rows back as soon as they are final.  With resident operands a large product
+ * runs in a few column panels instead, so that all but the last are copied back
+ * while the next is computed.  Same result bits as one launch.
+ * Default on; 0 turns both off (environment XKBLAS_PIPELINE). */
 void xkblas_set_pipeline(int on);
 
 /* Tile-cache introspection and capacity (bytes of HBM; the reference's
@@ -140,11 +142,13 @@ int  xkblas_split_side_bits(int k, int nsplit);  /* split-BF16 bits per side t *
  * row of k equal-magnitude entries keeps of its largest entry (its rounding
  * error is below 2^-t of it); rows with spread magnitudes keep more. */
 int  xkblas_split_info(int mode, int k, int nsplit, int* nmod, int* nplane);
-/* DPOTRF/SPOTRF trailing updates: 1 = paired (default; -1 selects it too):
+/* Cholesky trailing updates: 1 = paired (default; -1 selects it too):
  * every other step applies two panels as one rank-2NB update of the trailing
  * triangle, half at once and half at the next step, while the next block
  * column is still updated at once for the lookahead; 0 = one rank-NB update
- * per panel.  Environment XKBLAS_POTRF_PAIR sets the initial value. */
+ * per panel.  Applies to the blocked form: DPOTRF with split products and the
+ * factor of xkblas_dposv_ir; the MFMA modes' block columns have no pairs.
+ * Environment XKBLAS_POTRF_PAIR sets the initial value. */
 void xkblas_set_potrf_pairing(int mode);
 
 /* Mixed-precision solve of A X = B, A symmetric positive definite (the uplo

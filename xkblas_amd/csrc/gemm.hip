@@ -645,7 +645,8 @@ double gemm_tiles_us(int tile, long tiles, int k)
   const double r = tiles / (tile == 128 ? 512.0 : 1280.0), w = std::floor(r), f = r - w;
   double last = f == 0 ? 0 : 0.5 + 0.5 * f;
   if (tile == 128 && f > 0)
-    last = w == 0 ? std::min(1.0, 0.62 + 0.95 * std::max(0.0, f - 0.5)) : std::min({1.12, 0.6 + 0.95 * f, 0.1 + 1.2 * f});
+    last = w == 0 ? std::min(1.0, 0.62 + 0.95 * std::max(0.0, f - 0.5))
+                  : std::min({1.12, 0.6 + 0.95 * f, 0.1 + 1.2 * f});
   return (w + last) * round_us<T>(tile, k);
 }
 template double gemm_tiles_us<double>(int, long, int);
@@ -685,8 +686,8 @@ template int gemm_tile_of<float>(bool, bool, int, int, int, long, double*);
 
 template <typename T>
 void gemm(hipStream_t s, int transA, int transB, int m, int n, int k, T alpha, const T* A, long lda,
-          const T* B, long ldb, T beta, T* C, long ldc, int tri, int batch, long sA, long sB, long sC, int kmode, int kpart,
-          int tile)
+          const T* B, long ldb, T beta, T* C, long ldc, int tri, int batch, long sA, long sB, long sC, int kmode,
+          int kpart, int tile)
 {
   if (m <= 0 || n <= 0 || batch <= 0) return;
   if (tri != TRI_FULL)

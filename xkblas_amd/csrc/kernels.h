@@ -12,7 +12,8 @@ namespace xk {
 // the diagonal.
 // `batch` > 1 runs independent problems at element strides sA, sB, sC.
 // beta == 0 never reads C.  FP64 uses v_mfma_f64_16x16x4f64, FP32 uses
-// v_mfma_f32_16x16x4f32; tiles are staged through LDS, double-buffered.
+// v_mfma_f32_16x16x4f32; operands go through LDS, straight to it where both
+// are 16-byte aligned and that is faster.
 // `kmode` (KRANGE_*) limits each tile's inner range to where a triangular
 // op(A) (its rows) or op(B) (its columns) is not zero.
 template <typename T>
