@@ -8,6 +8,8 @@ for bit, in FP64 MFMA and in the split modes (row scalings span the whole
 inner dimension; B's residue planes are computed once), for ragged shapes,
 every transpose pair and beta = 0 (C not read) or not.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -143,3 +145,49 @@ def test_copies_back_of_short_and_long_calls(xk):
         assert np.array_equal(E, long_ + 2 * short)
         assert np.array_equal(C, long_)
     xk.invalidate()
+
+
+@pytest.mark.parametrize("follows", ["gemm", "syr2k"])
+def test_copy_back_of_a_short_calls_result_runs_under_the_next_call(xk, follows, tmp_path):
+    """A result waits for its own last write: its copy back (0.3 ms) ends while a
+    long call (2 ms and more) that was enqueued after it still runs, also where a
+    short call stands between."""
+    import csv
+    L = xk.lib()
+    n, m = 1500, 4200
+    r = rng(9)
+    a = np.asfortranarray(r.integers(-2, 3, (n, 20)).astype(np.float64))
+    A = np.asfortranarray(r.integers(-2, 3, (m, m)).astype(np.float64))
+    s = np.asfortranarray(r.integers(-2, 3, (40, 20)).astype(np.float64))
+    p = L.xkblas_malloc(n * n * 8)
+    buf = (ctypes.c_double * (n * n)).from_address(p)
+    C = np.frombuffer(buf).reshape((n, n), order="F")
+    D, E = np.zeros((m, m), order="F"), np.zeros((40, 40), order="F")
+
+    def calls():
+        xk.gemm(N_, T_, 1.0, a, a, 0.0, C, sync=False)
+        xk.gemm(N_, T_, 1.0, s, s, 0.0, E, sync=False)
+        if follows == "gemm":
+            xk.gemm(N_, N_, 1.0, A, A, 0.0, D, sync=False)
+        else:
+            xk.syr2k(122, N_, 1.0, A, A, 0.0, D, sync=False)
+
+    try:
+        calls()
+        L.xkblas_sync()  # the operands are resident
+        C[:] = 0
+        assert L.xkblas_trace_start(str(tmp_path).encode()) == 0
+        calls()
+        L.xkblas_memory_coherent_async(0, 0, n, n, C.ctypes.data, n, 8)
+        L.xkblas_sync()
+        assert L.xkblas_trace_stop() == 0
+        assert np.array_equal(C, a @ a.T)
+        with open(tmp_path / "kern.csv") as f:
+            kern = list(csv.DictReader(f))
+        with open(tmp_path / "cpy.csv") as f:
+            back = [c for c in csv.DictReader(f) if c["Dir"] == "2"]
+        assert sum(int(c["Size"]) for c in back) == n * n * 8
+        assert max(float(c["End"]) for c in back) < float(kern[-1]["End"])
+    finally:
+        xk.invalidate()
+        L.xkblas_free(p, n * n * 8)

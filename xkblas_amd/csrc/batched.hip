@@ -663,8 +663,7 @@ int xkblas_batch_run(void* plan)
   if (!pl) return -1;
   std::lock_guard<std::mutex> lock(api_mutex());
   Runtime& r = rt();
-  r.before_compute();
-  r.prof_begin("batch", pl->flops);
+  r.begin_compute("batch", pl->flops, nullptr);
   if (pl->exec) XK_HIP(hipGraphLaunch(pl->exec, r.s_comp));
   else enqueue_run(pl, r.s_comp);
   r.prof_end();
@@ -703,6 +702,7 @@ int xkblas_batch_run_noalloc(const xkblas_batch_problem_t* problems, int count)
   BatchProblem* d_probs = reinterpret_cast<BatchProblem*>(base + NOALLOC_PROBS_OFF);
   BatchItem* d_items = reinterpret_cast<BatchItem*>(base + NOALLOC_ITEMS_OFF);
   int* d_counter = reinterpret_cast<int*>(base);
+  r.stamp_written("batch", flops, nullptr);
   r.before_compute();
   if (count)
     XK_HIP(hipMemcpyAsync(d_probs, g_noalloc_probs, sizeof(BatchProblem) * count, hipMemcpyHostToDevice, r.s_comp));

@@ -234,21 +234,39 @@ void Runtime::drop(Replica* r)
 void Runtime::release(Replica* r)
 {
   unstamped.erase(std::remove(unstamped.begin(), unstamped.end(), r), unstamped.end());
-  if (r->written) XK_HIP(hipEventDestroy(r->written));
   delete r;
 }
 
-// An event behind the mirrors written by the last call, if it was a long one,
-// before other work follows on the compute stream: their copies back wait for it
-// alone.  The event takes 2 us of the stream: short calls that follow each other
-// would feel it (FP64 512 x 512 x 64 11.5 us a call, with an event each 13.7; from
-// 1e10 flops, 160 us, it is 1 %), and their results wait for the whole stream.
+// An event behind the mirrors written so far, before a call of class `cls` that
+// writes `out` follows on the compute stream: their copies back then wait for it
+// alone.  The event takes 2 to 4 us of the stream, which short calls that follow
+// each other would feel (FP64 512 x 512 x 64 11.5 us a call, with an event each 13.7):
+// it is recorded where a result waits that the host does not have and the coming
+// call is 30 us or more long, as long as the smallest copy with its waits, or the
+// result is a long call's (1e10 flops, 160 us: 1 %).  SYMM, TRMM, SYR2K and both
+// results copied back, with / without: FP64 order 188, 1002 columns 134 / 173 us,
+// 3009 x 789 2263 / 2608, complex 469 x 777 320 / 429, FP32 304 x 967 122 / 152.
 constexpr double STAMP_FLOPS = 1e10;
-void Runtime::stamp_written()
+void Runtime::stamp_written(const char* cls, double flops, const Replica* out)
 {
+  // about how long the call is: products at half of their best rate, and what
+  // several dependent launches take at any size
+  const size_t len = strlen(cls);
+  bool several = false;
+  for (const char* c : {"syr2k", "her2k", "trsm", "potrf", "posv", "batch"})
+    several |= strncmp(cls, c, strlen(c)) == 0;
+  const bool f32 = len > 3 && (strcmp(cls + len - 3, "f32") == 0 || strcmp(cls + len - 3, "c64") == 0);
+  const double us = flops / (f32 ? 80e6 : 40e6) + (several ? 30 : 8);
+  bool stamp = false;
+  for (const Replica* r : unstamped)
+    stamp |= r != out && r->panels.empty() && (us >= 30 || r->long_write) && !mirror_clean(r);
+  if (!stamp) return;
+  hipEvent_t ev;
+  XK_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+  std::shared_ptr<std::remove_pointer_t<hipEvent_t>> written(ev, [](hipEvent_t e) { XK_HIP(hipEventDestroy(e)); });
+  XK_HIP(hipEventRecord(ev, s_comp));
   for (Replica* r : unstamped) {
-    if (!r->written) XK_HIP(hipEventCreateWithFlags(&r->written, hipEventDisableTiming));
-    XK_HIP(hipEventRecord(r->written, s_comp));
+    r->written = written;
     r->stamped = true;
   }
   unstamped.clear();
@@ -394,8 +412,11 @@ void Runtime::mark_written(Replica* r, int r0, int c0, int m, int n, int uplo)
 {
   if (m <= 0 || n <= 0) return;
   clear_panels(r);
-  if (call_flops >= STAMP_FLOPS && std::find(unstamped.begin(), unstamped.end(), r) == unstamped.end())
+  if (std::find(unstamped.begin(), unstamped.end(), r) == unstamped.end()) {
+    if (unstamped.size() == 16) unstamped.erase(unstamped.begin());
     unstamped.push_back(r);
+  }
+  r->long_write = call_flops >= STAMP_FLOPS;
   r->stamped = false;
   const int ti0 = r0 / r->nb, ti1 = (r0 + m - 1) / r->nb;
   const int tj0 = c0 / r->nb, tj1 = (c0 + n - 1) / r->nb;
@@ -433,7 +454,7 @@ void Runtime::writeback(Replica* r, int r0, int c0, int m, int n, int uplo)
   }
   if (done < end) {
     if (r->stamped) {
-      XK_HIP(hipStreamWaitEvent(s_d2h, r->written, 0));
+      XK_HIP(hipStreamWaitEvent(s_d2h, r->written.get(), 0));
     } else {
       XK_HIP(hipEventRecord(ev_comp, s_comp));
       XK_HIP(hipStreamWaitEvent(s_d2h, ev_comp, 0));
@@ -645,7 +666,6 @@ void Runtime::copy_d2h(char* dst, size_t dpitch, const char* src, size_t spitch,
 // Order the compute stream after the pending copies.
 void Runtime::before_compute()
 {
-  if (!unstamped.empty()) stamp_written();
   if (pending_h2d) {
     XK_HIP(hipEventRecord(ev_h2d, s_h2d));
     XK_HIP(hipStreamWaitEvent(s_comp, ev_h2d, 0));
@@ -726,6 +746,14 @@ static uint64_t now_ns()
   struct timespec ts;
   clock_gettime(CLOCK_MONOTONIC, &ts);
   return (uint64_t)ts.tv_sec * 1000000000ull + (uint64_t)ts.tv_nsec;
+}
+
+// A call's work on the compute stream begins; it writes `out`.
+void Runtime::begin_compute(const char* cls, double flops, const Replica* out)
+{
+  stamp_written(cls, flops, out);
+  before_compute();
+  prof_begin(cls, flops);
 }
 
 void Runtime::prof_begin(const char* cls, double flops)
@@ -1429,8 +1457,7 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
   if (!ends.empty() && resident) {
     if (split) split_cache_register((const double*)rA->dev, rA->ldd, M, K, rowsA);
     std::vector<Replica::PanelEvent> pev;
-    r.before_compute();
-    r.prof_begin(sizeof(T) == 8 ? "gemm_f64" : "gemm_f32", flops);
+    r.begin_compute(sizeof(T) == 8 ? "gemm_f64" : "gemm_f32", flops, rC);
     x.parts = 1;  // the whole product's
     int j0 = 0;
     for (int end : ends) {
@@ -1452,6 +1479,7 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
     return 0;
   }
   if (!ends.empty()) {
+    r.stamp_written(sizeof(T) == 8 ? "gemm_f64" : "gemm_f32", flops, rC);
     r.fetch(rB, 0, 0, Bm, Bn);
     if (split) split_cache_register((const double*)rB->dev, rB->ldd, N, K, transB != NoTrans);
     std::vector<Replica::PanelEvent> pev;
@@ -1482,8 +1510,7 @@ int gemm_async(const char* fn, int transA, int transB, int M, int N, int K, cons
   if (rA) r.fetch(rA, 0, 0, Am, An);
   if (rB) r.fetch(rB, 0, 0, Bm, Bn);
   if (readC) r.fetch(rC, 0, 0, M, N);
-  r.before_compute();
-  r.prof_begin(sizeof(T) == 8 ? "gemm_f64" : "gemm_f32", flops);
+  r.begin_compute(sizeof(T) == 8 ? "gemm_f64" : "gemm_f32", flops, rC);
   dev_gemm<T>(x, transA, transB, M, N, use_ab ? K : 0, use_ab ? *alpha : T(0), rA ? (const T*)rA->dev : (const T*)rC->dev,
               rA ? rA->ldd : rC->ldd, rB ? (const T*)rB->dev : (const T*)rC->dev, rB ? rB->ldd : rC->ldd, *beta,
               (T*)rC->dev, rC->ldd);
@@ -1516,9 +1543,8 @@ int syrk_async(const char* fn, int uplo, int trans, int N, int K, const T* alpha
   Replica* rC = r.replica(C, N, N, LDC, sizeof(T), nb, keep);
   if (rA) r.fetch(rA, 0, 0, Am, An);
   r.fetch(rC, 0, 0, N, N);  // the other triangle must stay intact on the device
-  r.before_compute();
   Exec x = r.exec();
-  r.prof_begin(sizeof(T) == 8 ? "syrk_f64" : "syrk_f32", (double)K * N * (N + 1.0));
+  r.begin_compute(sizeof(T) == 8 ? "syrk_f64" : "syrk_f32", (double)K * N * (N + 1.0), rC);
   dev_syrk<T>(x, uplo, trans, N, use_a ? K : 0, use_a ? *alpha : T(0), rA ? (const T*)rA->dev : (const T*)rC->dev,
               rA ? rA->ldd : rC->ldd, *beta, (T*)rC->dev, rC->ldd);
   r.prof_end();
@@ -1551,10 +1577,9 @@ int trsm_async(const char* fn, int side, int uplo, int transA, int diag, int N, 
   Replica* rB = r.replica(B, N, NRHS, LDB, sizeof(T), nb, keep);
   r.fetch(rA, 0, 0, NA, NA);
   r.fetch(rB, 0, 0, N, NRHS);
-  r.before_compute();
   Exec x = r.exec();
   const double flops = side == Left ? (double)N * N * NRHS : (double)N * NRHS * NRHS;
-  r.prof_begin(sizeof(T) == 8 ? "trsm_f64" : "trsm_f32", flops);
+  r.begin_compute(sizeof(T) == 8 ? "trsm_f64" : "trsm_f32", flops, rB);
   // inner diagonal block order: the tile size, capped for the inverse GEMMs
   const int dnb = std::min(nb, 512);
   dev_trsm<T>(x, side, uplo, transA, diag, N, NRHS, *alpha, (const T*)rA->dev, rA->ldd, (T*)rB->dev, rB->ldd, dnb);
@@ -1579,11 +1604,11 @@ int potrf_async(const char* fn, int uplo, int N, T* A, int LDA)
   Replica* rA = r.replica(A, N, N, LDA, sizeof(T), nb, keep);
   if (rA->info_slot < 0) rA->info_slot = r.take_info_slot();
   r.fetch(rA, 0, 0, N, N);
-  r.before_compute();
   Exec x = r.exec();
   int* dinfo = r.d_info + rA->info_slot;
+  r.begin_compute(sizeof(T) == 8 ? "potrf_f64" : "potrf_f32",
+                  (double)N * N * N / 3.0 + (double)N * N / 2.0 + N / 6.0, rA);
   fill_int(x.s, dinfo, 1, INT_MAX);
-  r.prof_begin(sizeof(T) == 8 ? "potrf_f64" : "potrf_f32", (double)N * N * N / 3.0 + (double)N * N / 2.0 + N / 6.0);
   const int order = r.nb || !split_enabled<T>(x) ? nb : split_potrf_order(N, nb, false);
   dev_potrf<T>(x, uplo, N, (T*)rA->dev, rA->ldd, order, dinfo);
   r.prof_end();
@@ -1622,10 +1647,10 @@ int gemmt_async(const char* fn, int uplo, int transA, int transB, int N, int K, 
   if (rA) r.fetch(rA, 0, 0, Am, An);
   if (rB) r.fetch(rB, 0, 0, Bm, Bn);
   r.fetch(rC, 0, 0, N, N);  // the other triangle stays intact on the device
-  r.before_compute();
   Exec x = r.exec();
   const bool tri = uplo == Upper || uplo == Lower;
-  r.prof_begin(sizeof(T) == 8 ? "gemmt_f64" : "gemmt_f32", tri ? (double)K * N * (N + 1.0) : 2.0 * N * N * (double)K);
+  r.begin_compute(sizeof(T) == 8 ? "gemmt_f64" : "gemmt_f32",
+                  tri ? (double)K * N * (N + 1.0) : 2.0 * N * N * (double)K, rC);
   dev_gemmt<T>(x, uplo, transA, transB, N, use_ab ? K : 0, use_ab ? *alpha : T(0),
                rA ? (const T*)rA->dev : (const T*)rC->dev, rA ? rA->ldd : rC->ldd,
                rB ? (const T*)rB->dev : (const T*)rC->dev, rB ? rB->ldd : rC->ldd, *beta, (T*)rC->dev, rC->ldd);
@@ -1661,9 +1686,8 @@ int syr2k_async(const char* fn, int uplo, int trans, int N, int K, const T* alph
   if (rA) r.fetch(rA, 0, 0, Am, An);
   if (rB) r.fetch(rB, 0, 0, Am, An);
   r.fetch(rC, 0, 0, N, N);
-  r.before_compute();
   Exec x = r.exec();
-  r.prof_begin(sizeof(T) == 8 ? "syr2k_f64" : "syr2k_f32", 2.0 * K * N * (N + 1.0));
+  r.begin_compute(sizeof(T) == 8 ? "syr2k_f64" : "syr2k_f32", 2.0 * K * N * (N + 1.0), rC);
   dev_syr2k<T>(x, uplo, trans, N, use_ab ? K : 0, use_ab ? *alpha : T(0), rA ? (const T*)rA->dev : (const T*)rC->dev,
                rA ? rA->ldd : rC->ldd, rB ? (const T*)rB->dev : (const T*)rC->dev, rB ? rB->ldd : rC->ldd, *beta,
                (T*)rC->dev, rC->ldd);
@@ -1699,9 +1723,8 @@ int symm_async(const char* fn, int side, int uplo, int M, int N, const T* alpha,
   if (rA) r.fetch(rA, 0, 0, Am, Am);
   if (rB) r.fetch(rB, 0, 0, M, N);
   if (*beta != T(0)) r.fetch(rC, 0, 0, M, N);
-  r.before_compute();
   Exec x = r.exec();
-  r.prof_begin(sizeof(T) == 8 ? "symm_f64" : "symm_f32", 2.0 * M * N * (double)Am);
+  r.begin_compute(sizeof(T) == 8 ? "symm_f64" : "symm_f32", 2.0 * M * N * (double)Am, rC);
   dev_symm<T>(x, side, uplo, M, N, use_ab ? *alpha : T(0), rA ? (const T*)rA->dev : (const T*)rC->dev,
               rA ? rA->ldd : rC->ldd, rB ? (const T*)rB->dev : (const T*)rC->dev, rB ? rB->ldd : rC->ldd, *beta,
               (T*)rC->dev, rC->ldd);
@@ -1735,10 +1758,9 @@ int trmm_async(const char* fn, int side, int uplo, int transA, int diag, int N, 
   Replica* rB = r.replica(B, N, NRHS, LDB, sizeof(T), nb, keep);
   r.fetch(rA, 0, 0, NA, NA);
   r.fetch(rB, 0, 0, N, NRHS);
-  r.before_compute();
   Exec x = r.exec();
   const double flops = side == Left ? (double)N * N * NRHS : (double)N * NRHS * NRHS;
-  r.prof_begin(sizeof(T) == 8 ? "trmm_f64" : "trmm_f32", flops);
+  r.begin_compute(sizeof(T) == 8 ? "trmm_f64" : "trmm_f32", flops, rB);
   dev_trmm<T>(x, side, uplo, transA, diag, N, NRHS, *alpha, (const T*)rA->dev, rA->ldd, (T*)rB->dev, rB->ldd);
   r.prof_end();
   r.mark_written(rB, 0, 0, N, NRHS, 0);
@@ -1777,9 +1799,8 @@ int cgemm_async(const char* fn, int transA, int transB, int M, int N, int K, con
   if (rA) r.fetch(rA, 0, 0, Am, An);
   if (rB) r.fetch(rB, 0, 0, Bm, Bn);
   if (beta[0] != T(0) || beta[1] != T(0)) r.fetch(rC, 0, 0, M, N);
-  r.before_compute();
   Exec x = r.exec();
-  r.prof_begin(sizeof(T) == 8 ? "gemm_c128" : "gemm_c64", 8.0 * M * N * (double)K);
+  r.begin_compute(sizeof(T) == 8 ? "gemm_c128" : "gemm_c64", 8.0 * M * N * (double)K, rC);
   const T zero[2] = {T(0), T(0)};
   dev_cgemm<T>(x, transA, transB, M, N, use_ab ? K : 0, use_ab ? alpha : zero, rA ? (const T*)rA->dev : nullptr,
                rA ? rA->ldd : 1, rB ? (const T*)rB->dev : nullptr, rB ? rB->ldd : 1, beta, (T*)rC->dev, rC->ldd);
@@ -1813,9 +1834,8 @@ int cherk_async(const char* fn, int uplo, int trans, int N, int K, const T* alph
   Replica* rC = r.replica(C, N, N, LDC, elt, nb, keep);
   if (rA) r.fetch(rA, 0, 0, Am, An);
   r.fetch(rC, 0, 0, N, N);  // the other triangle stays intact on the device
-  r.before_compute();
   Exec x = r.exec();
-  r.prof_begin(sizeof(T) == 8 ? "herk_c128" : "herk_c64", 4.0 * K * N * (N + 1.0));
+  r.begin_compute(sizeof(T) == 8 ? "herk_c128" : "herk_c64", 4.0 * K * N * (N + 1.0), rC);
   dev_cherk<T>(x, uplo, trans, N, use_a ? K : 0, use_a ? *alpha : T(0), rA ? (const T*)rA->dev : nullptr,
                rA ? rA->ldd : 1, *beta, (T*)rC->dev, rC->ldd);
   r.prof_end();
@@ -1851,10 +1871,9 @@ int chemm_async(const char* fn, int herm, int side, int uplo, int M, int N, cons
   if (rA) r.fetch(rA, 0, 0, Am, Am);
   if (rB) r.fetch(rB, 0, 0, M, N);
   if (beta[0] != T(0) || beta[1] != T(0)) r.fetch(rC, 0, 0, M, N);
-  r.before_compute();
   Exec x = r.exec();
-  r.prof_begin(herm ? (sizeof(T) == 8 ? "hemm_c128" : "hemm_c64") : (sizeof(T) == 8 ? "symm_c128" : "symm_c64"),
-               8.0 * M * N * (double)Am);
+  r.begin_compute(herm ? (sizeof(T) == 8 ? "hemm_c128" : "hemm_c64") : (sizeof(T) == 8 ? "symm_c128" : "symm_c64"),
+                  8.0 * M * N * (double)Am, rC);
   dev_chemm<T>(x, herm, side, uplo, M, N, alpha, rA ? (const T*)rA->dev : nullptr, rA ? rA->ldd : 1,
                rB ? (const T*)rB->dev : nullptr, rB ? rB->ldd : 1, beta, (T*)rC->dev, rC->ldd);
   r.prof_end();
@@ -1894,9 +1913,8 @@ int csyr2k_async(const char* fn, int herm, int two, int uplo, int trans, int N, 
   if (rA) r.fetch(rA, 0, 0, Am, An);
   if (rB) r.fetch(rB, 0, 0, Am, An);
   r.fetch(rC, 0, 0, N, N);
-  r.before_compute();
   Exec x = r.exec();
-  r.prof_begin(two ? (herm ? "her2k_c" : "syr2k_c") : "syrk_c", (two ? 8.0 : 4.0) * K * N * (N + 1.0));
+  r.begin_compute(two ? (herm ? "her2k_c" : "syr2k_c") : "syrk_c", (two ? 8.0 : 4.0) * K * N * (N + 1.0), rC);
   const T zero[2] = {T(0), T(0)};
   const T* dA = rA ? (const T*)rA->dev : nullptr;
   const T* dB = two ? (rB ? (const T*)rB->dev : nullptr) : dA;
@@ -1946,9 +1964,8 @@ int cgemmt_async(const char* fn, int uplo, int transA, int transB, int N, int K,
   if (rA) r.fetch(rA, 0, 0, Am, An);
   if (rB) r.fetch(rB, 0, 0, Bm, Bn);
   r.fetch(rC, 0, 0, N, N);
-  r.before_compute();
   Exec x = r.exec();
-  r.prof_begin("gemmt_c", 8.0 * N * N * (double)K);
+  r.begin_compute("gemmt_c", 8.0 * N * N * (double)K, rC);
   const T zero[2] = {T(0), T(0)};
   dev_cgemmt<T>(x, uplo, transA, transB, N, use_ab ? K : 0, use_ab ? alpha : zero, rA ? (const T*)rA->dev : nullptr,
                 rA ? rA->ldd : 1, rB ? (const T*)rB->dev : nullptr, rB ? rB->ldd : 1, beta, (T*)rC->dev, rC->ldd);
@@ -1983,9 +2000,8 @@ int ctrmm_async(const char* fn, int side, int uplo, int transA, int diag, int N,
   Replica* rB = r.replica(B, N, NRHS, LDB, elt, nb, keep);
   r.fetch(rA, 0, 0, NA, NA);
   r.fetch(rB, 0, 0, N, NRHS);
-  r.before_compute();
   Exec x = r.exec();
-  r.prof_begin("trmm_c", 4.0 * (side == Left ? (double)N * N * NRHS : (double)N * NRHS * NRHS));
+  r.begin_compute("trmm_c", 4.0 * (side == Left ? (double)N * N * NRHS : (double)N * NRHS * NRHS), rB);
   dev_ctrmm<T>(x, side, uplo, transA, diag, N, NRHS, alpha, (const T*)rA->dev, rA->ldd, (T*)rB->dev, rB->ldd);
   r.prof_end();
   r.mark_written(rB, 0, 0, N, NRHS, 0);
@@ -2018,9 +2034,8 @@ int ctrsm_async(const char* fn, int side, int uplo, int transA, int diag, int N,
   Replica* rB = r.replica(B, N, NRHS, LDB, elt, nb, keep);
   r.fetch(rA, 0, 0, NA, NA);
   r.fetch(rB, 0, 0, N, NRHS);
-  r.before_compute();
   Exec x = r.exec();
-  r.prof_begin("trsm_c", 4.0 * (side == Left ? (double)N * N * NRHS : (double)N * NRHS * NRHS));
+  r.begin_compute("trsm_c", 4.0 * (side == Left ? (double)N * N * NRHS : (double)N * NRHS * NRHS), rB);
   dev_ctrsm<T>(x, side, uplo, transA, diag, N, NRHS, alpha, (const T*)rA->dev, rA->ldd, (T*)rB->dev, rB->ldd,
                std::min(nb, 256));
   r.prof_end();
@@ -2044,11 +2059,10 @@ int cpotrf_async(const char* fn, int uplo, int N, T* A, int LDA)
   Replica* rA = r.replica(A, N, N, LDA, 2 * sizeof(T), nb, keep);
   if (rA->info_slot < 0) rA->info_slot = r.take_info_slot();
   r.fetch(rA, 0, 0, N, N);
-  r.before_compute();
   Exec x = r.exec();
   int* dinfo = r.d_info + rA->info_slot;
+  r.begin_compute("potrf_c", 4.0 * ((double)N * N * N / 3.0 + (double)N * N / 2.0), rA);
   fill_int(x.s, dinfo, 1, INT_MAX);
-  r.prof_begin("potrf_c", 4.0 * ((double)N * N * N / 3.0 + (double)N * N / 2.0));
   dev_cpotrf<T>(x, uplo, N, (T*)rA->dev, rA->ldd, std::min(nb, 512), dinfo);
   r.prof_end();
   XK_HIP(hipMemcpyAsync(r.h_info + rA->info_slot, dinfo, sizeof(int), hipMemcpyDeviceToHost, x.s));
@@ -2275,14 +2289,13 @@ int xkblas_dposv_ir(int uplo, int N, int NRHS, const double* A, int LDA, const d
   Replica* rX = r.replica(X, N, NRHS, LDX, sizeof(double), nb, keep);
   r.fetch(rA, 0, 0, N, N);
   r.fetch(rB, 0, 0, N, NRHS);
-  r.before_compute();
   Exec xf = r.exec();              // the accurate factor: the current mode
   Exec x = xf;                     // residuals, updates and solves: FP64
   x.mode = XKBLAS_DEFAULT_MATH;
   Exec xl = xf;                    // the reduced factor: split-BF16, fewer moduli
   xl.mode = XKBLAS_SPLIT_BF16_MATH;
   xl.nsplit = g_ir_moduli;
-  r.prof_begin("posv_ir_f64", (double)N * N * N / 3.0 + 2.0 * N * N * (double)NRHS);
+  r.begin_compute("posv_ir_f64", (double)N * N * N / 3.0 + 2.0 * N * N * (double)NRHS, rX);
   const int order = r.nb ? nb : split_potrf_order(N, nb, true);
   const int info = dev_posv_ir(x, xl, xf, uplo, N, NRHS, (const double*)rA->dev, rA->ldd, (const double*)rB->dev,
                                rB->ldd, (double*)rX->dev, rX->ldd, order, g_ir_itermax, iter);

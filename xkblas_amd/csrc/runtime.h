@@ -3,6 +3,7 @@
 #include "blas3.h"
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -43,9 +44,10 @@ struct Replica {
   bool panel_cols = false;
   // The last write of the mirror is complete with `written` on the compute
   // stream once `stamped`; before that, with whatever the stream holds now.
-  // The event is recorded only when another call follows a long one's write.
-  hipEvent_t written = nullptr;
+  // One event serves every mirror that it stands behind.
+  std::shared_ptr<std::remove_pointer_t<hipEvent_t>> written;
   bool stamped = false;
+  bool long_write = false;  // the last write was a long call's
 };
 
 struct ProfEntry {
@@ -84,7 +86,7 @@ struct Runtime {
   hipEvent_t ev_comp = nullptr, ev_h2d = nullptr, ev_d2h = nullptr;
   hipEvent_t ev_pot0 = nullptr, ev_pot1 = nullptr;  // POTRF's lookahead ordering
   bool pending_h2d = false, pending_d2h = false;
-  std::vector<Replica*> unstamped;  // mirrors written by the last call on the compute stream, if it was a long one
+  std::vector<Replica*> unstamped;  // mirrors with no event behind their last write yet, latest last
   double call_flops = 0;            // of the running call
 
   std::unordered_map<const void*, Replica*> map;
@@ -156,7 +158,7 @@ struct Runtime {
   void mark_written(Replica* r, int r0, int c0, int m, int n, int uplo);
   void writeback(Replica* r, int r0, int c0, int m, int n, int uplo);
   bool copy_back(Replica* r, int row_lo, int row_hi, int col_lo, int col_hi, int uplo);
-  void stamp_written();
+  void stamp_written(const char* cls, double flops, const Replica* out);
   void release(Replica* r);
   bool all_valid(const Replica* r, int r0, int c0, int m, int n) const;
   void clear_panels(Replica* r);
@@ -167,6 +169,7 @@ struct Runtime {
   void free_retired();
   int take_info_slot();
   void before_compute();
+  void begin_compute(const char* cls, double flops, const Replica* out);
   bool host_pinned(const void* p, size_t bytes) const;
   void copy_h2d(char* dst, size_t dpitch, const char* src, size_t spitch, size_t width, size_t height);
   void copy_d2h(char* dst, size_t dpitch, const char* src, size_t spitch, size_t width, size_t height);
